@@ -119,6 +119,49 @@ inline bool few_fits(uint32_t N, uint32_t K, uint32_t M, int num_cus) {
     return 2 * tiles >= (uint64_t)num_cus;
 }
 
+// Launches below kW16MinTokens tokens whose 256 x 256 tiles leave CUs idle in
+// their last round: the whole rounds of tiles run as they are (`full` of
+// them) and every tile of the last round is cut along K into `splits`
+// workgroups, whose partial tiles a second launch adds up. The times are
+// estimates in us on MI355X (256 CUs), fitted to launches of 300-2000 tokens
+// x 3072-21504 features: a K stage of a tile takes 2.0 us on the 8-wave
+// kernel that also runs the splits (1.93 and 1.7 for Q8_0 and Q4_K where
+// tiles follow each other in the persistent kernels), a workgroup 8 us around
+// its stages, and the partial tiles are written and read at ~5 TB/s; the
+// 64 x 64 tiled kernel reaches 230 (Q8_0) and 300 TFLOP/s (Q4_K). Measured,
+// whole launch before -> after: 1101 x 3840 x 3840 Q8_0 (75 tiles x 3) 129 ->
+// 60 us, x 10240 348 -> 117; 520 x 9216 x 3072 Q4_K (108 x 2) 99 -> 60; 1536 x
+// 11520 x 3840 Q8_0 (256 whole tiles + 14 x 15) 236 -> 160; 2000 x 9216 x
+// 3072 Q4_K (256 + 32 x 8) 165 -> 139. Where the estimates are within 3%
+// the launch stays whole (2000 x 12288 x 3072 Q4_K, 128 tiles in its last
+// round: 168 whole, 177 split).
+constexpr size_t kPartTile = 256u * 256u * sizeof(float);  // one partial tile
+constexpr uint32_t kSplitMax = 16;
+// Fewer K stages than this run whole: a workgroup's fixed 8 us are then as
+// long as all of a tile's stages.
+constexpr uint32_t kSplitTileMinStages = 16;
+struct SplitPlan {
+    uint32_t full, splits;  // splits 1: no split
+};
+inline SplitPlan plan_split(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, int num_cus, bool persistent) {
+    const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
+    const uint32_t S = K / kStageK;
+    const uint64_t full = tiles / num_cus * num_cus, rem = tiles - full;
+    SplitPlan p{(uint32_t)full, 1};
+    const double whole = persistent
+                             ? (double)((tiles + num_cus - 1) / num_cus) * S * (wtype == kQ8_0 ? 1.93 : 1.7) + 6.0
+                             : 2e-6 * M * N * K / (wtype == kQ8_0 ? 230.0 : 300.0) + 8.0;
+    double best = 0.97 * whole;
+    for (uint32_t s = 2; rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
+        if (nonempty_splits(S, s) != s) continue;
+        const double rounds = (double)((rem * s + num_cus - 1) / num_cus);
+        const double us = (double)(full / num_cus) * (S * 2.0 + 8.0) + rounds * ((S + s - 1) / s * 2.0 + 8.0) + 3.0 +
+                          (double)rem * kPartTile * (s + 1) / 5e6;
+        if (us < best) best = us, p.splits = s;
+    }
+    return p;
+}
+
 // How one GEMM runs.
 //  * few: the few-token kernel (f32 / 16-bit activations read in place, no
 //    workspace);
@@ -129,6 +172,8 @@ inline bool few_fits(uint32_t N, uint32_t K, uint32_t M, int num_cus) {
 //    activations rounded to operand_type() into the workspace first; from
 //    kW16MinTokens tokens two-pass (the 16-bit weight image after them in
 //    the workspace);
+//  * split: below kW16MinTokens tokens, where plan_split finds that cutting
+//    the last round's tiles along K pays: [x16 | partial tiles];
 //  * otherwise the tiled kernel, split-K partials in the workspace.
 // With a workspace limit (the no-allocation entry point's fixed array) the
 // plan keeps within it: the two-pass path only when its image fits, as many
@@ -140,6 +185,7 @@ struct GemmPlan {
     uint32_t xt;                  // activation type the kernel reads
     TilePlan tiles;               // the tiled kernel's tile and splits (not persistent)
     uint32_t splits;              // the skinny kernel's K splits
+    uint32_t split, split_full;   // split > 1: 256 x 256 tiles, those past split_full cut along K into `split`
     size_t x16_off, img_off, ws;  // workspace: [x16 | image] (persistent), [packed x | partials]
                                   // (skinny), split-K partials (tiled)
 };
@@ -151,6 +197,7 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
     p.xt = xtype;
     p.tiles = TilePlan{64, 1};
     p.splits = 1;
+    p.split = 1;
     const uint64_t rb = row_bytes_of(wtype, K);
     const bool offsets31 = (uint64_t)M * K * 2u < (1ull << 31) && (uint64_t)N * rb < (1ull << 31);
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -174,6 +221,21 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
             p.xt = operand_type(wtype, xtype);
             p.splits = nonempty_splits(S, want);
             p.ws = x16 + (p.splits > 1 ? p.splits * part : 0u);
+            return p;
+        }
+    }
+    if (K % kStageK == 0 && N % 4 == 0 && offsets31 && M < kW16MinTokens) {
+        const SplitPlan sp = plan_split(wtype, N, K, M, num_cus, p.persistent);
+        const size_t x16 = xtype == kF32 ? align256((size_t)M * K * 2u) : 0u;
+        const size_t ws = x16 + (size_t)(tiles - sp.full) * sp.splits * kPartTile;
+        if (sp.splits > 1 && ws <= ws_limit) {
+            p.persistent = false;
+            p.split = sp.splits;
+            p.split_full = sp.full;
+            p.convert_x = xtype == kF32;
+            p.xt = operand_type(wtype, xtype);
+            p.img_off = x16;  // the partial tiles
+            p.ws = ws;
             return p;
         }
     }

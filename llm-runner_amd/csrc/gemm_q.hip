@@ -833,8 +833,16 @@ struct Frags8 {
     f16x8 x[4], w[2];
 };
 
-template <uint32_t WT, uint32_t XT, uint32_t EPI = kEpiStore, bool GROUPED = false>
+// SPLITK: one workgroup per item instead of a persistent walk. The first
+// split_full items are whole tiles, stored to Y; the other tiles are cut along
+// K: item split_full + j is split z = j / rem of tile split_full + j % rem (rem
+// = the tiles past split_full), stages [z split_stages, min(S, (z + 1)
+// split_stages)) with no padded ones, into the 256 x 256 partial tile j of
+// `part` (splitk_tiles_kernel adds them). For launches whose last round of
+// tiles leaves CUs idle; the rule and its figures are at plan::plan_split.
+template <uint32_t WT, uint32_t XT, uint32_t EPI = kEpiStore, bool GROUPED = false, bool SPLITK = false>
 __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args) {
+    static_assert(!SPLITK || (EPI == kEpiStore && !GROUPED), "partial tiles are plain stores of one problem");
     // every argument the kernel uses as a scalar local (see gemm_q_persist)
     const uint32_t N = args.N, K = args.K, tiles_m = args.tiles_m, tiles_n = args.tiles_n;
     const uint32_t ldy = args.ldy, ldy2 = args.ldy2, split = args.split, y2_bf16 = args.y2_bf16;
@@ -869,9 +877,27 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
     const uint32_t wh = wave >> 2;  // the weight-row half this wave dequantizes
 
     const uint32_t G = gridDim.x, total = tiles_m * tiles_n;
-    const uint32_t n_tiles = (total - blockIdx.x + G - 1) / G;  // >= 1: grid <= total
-    const uint32_t S = K / kBK;
-    const uint32_t SP = (S + 5u) / 6u * 6u;
+    const uint32_t n_tiles = SPLITK ? 1u : (total - blockIdx.x + G - 1) / G;  // >= 1: grid <= total
+    // SPLITK: this workgroup's item (an XCD's workgroups on consecutive tiles),
+    // its tile and its stages [S0, S)
+    uint32_t part_tile = 0u, item_tile = 0u, S0 = 0u, S = K / (uint32_t)kBK;
+    bool whole = true;
+    if constexpr (SPLITK) {
+        const uint32_t full = args.split_full, b = blockIdx.x;
+        whole = b < full;
+        if (whole) {
+            const uint32_t c = args.split_cus, r = b / c * c;
+            item_tile = r + xcd_linear(b - r, min(c, full - r));
+        } else {
+            const uint32_t rem = total - full;
+            part_tile = xcd_linear(b - full, G - full);
+            const uint32_t z = part_tile / rem;
+            item_tile = full + part_tile - z * rem;
+            S0 = z * args.split_stages;
+            S = min(S, S0 + args.split_stages);
+        }
+    }
+    const uint32_t SP = SPLITK ? 0xffffffffu : (S + 5u) / 6u * 6u;  // SPLITK: no next tile to advance to
     const uint32_t rb = (WT == kGgmlQ8_0) ? (K / 32u) * 34u : (K / 256u) * 144u;
     const uint32_t xrow = K * 2u;
 
@@ -903,7 +929,10 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
     };
     auto tile_origin = [&](uint32_t k, uint32_t& p, uint32_t& m0, uint32_t& n0) {
         uint32_t tm, tn;
-        map_tile_persist(blockIdx.x + k * G, G, tiles_m, tiles_n, tm, tn);
+        if constexpr (SPLITK)
+            tile_of_linear(item_tile, tiles_m, tiles_n, tm, tn);
+        else
+            map_tile_persist(blockIdx.x + k * G, G, tiles_m, tiles_n, tm, tn);
         p = GROUPED && tm >= Tp0 ? 1u : 0u;
         m0 = (tm - (p ? Tp0 : 0u)) * 256u;
         n0 = tn * 256u;
@@ -911,14 +940,14 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
     auto x_tile = [&](Cursor& c, uint32_t k) {
         uint32_t p, m0, n0;
         tile_origin(k, p, m0, n0);
-        c.s = 0;
+        c.s = S0;
         c.base = (const uint8_t*)pick(p, Xp0, Xp1) + (uint64_t)m0 * xrow;
         c.size = k < n_tiles ? (pick(p, Mp0, Mp1) - m0) * xrow : 0u;
     };
     auto w_tile = [&](Cursor& c, uint32_t k) {
         uint32_t p, m0, n0;
         tile_origin(k, p, m0, n0);
-        c.s = 0;
+        c.s = S0;
         c.base = pick(p, Wp0, Wp1) + (uint64_t)(pick(p, Rp0, Rp1) + n0) * rb;
         c.size = k < n_tiles ? (N - n0) * rb : 0u;
     };
@@ -1026,6 +1055,23 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
                 }
             });
         } else {
+            if constexpr (SPLITK) {
+                if (!whole) {  // the partial tile's rows below M (features past N included)
+                    float* const P = args.part + (uint64_t)part_tile * 65536u;
+#pragma unroll
+                    for (int a = 0; a < 2; a++)
+#pragma unroll
+                        for (int b = 0; b < 4; b++) {
+                            if (m0 + wm * 128u + b * 32u + l32 >= M) continue;
+                            float* const row = P + (wm * 128u + b * 32u + l32) * 256u + wn * 64u + a * 32u + 4u * kh;
+#pragma unroll
+                            for (int g = 0; g < 4; g++)
+                                *(f32x4*)(row + 8u * g) = f32x4{acc[a][b][4 * g], acc[a][b][4 * g + 1],
+                                                                acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]};
+                        }
+                    return;
+                }
+            }
             each([&](uint32_t m, uint32_t n, uint32_t, f32x4 v) __attribute__((always_inline)) {
                 *(f32x4*)(Y + (uint64_t)m * ldy + n) = v;
             });
@@ -1036,8 +1082,10 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
     // weights are dequantized and its activations have landed
     x_tile(cx, 0);
     w_tile(cw, 0);
-    x_tile(nx, 1);
-    w_tile(nw, 1);
+    if constexpr (!SPLITK) {
+        x_tile(nx, 1);
+        w_tile(nw, 1);
+    }
     issue_w_all(R0);
     issue_w_all(R1);
     issue_x_all(X0);
@@ -1045,7 +1093,7 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
     issue_x_all(X1);
     LLMR_WAIT_VMCNT(2 * W_LOADS + 2 * X_DMAS);
     {
-        const auto sc0 = R0.scale(0, wh);
+        const auto sc0 = R0.scale(S0, wh);
         R0.template store<0>(W0, sc0, wbase, wh);
         R0.template store<1>(W0, sc0, wbase, wh);
         R0.template store<2>(W0, sc0, wbase, wh);
@@ -1100,13 +1148,30 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         for (int i = 0; i < 4; i++) F1.x[i] = f16x8{};
 #pragma unroll
         for (int i = 0; i < 2; i++) F1.w[i] = f16x8{};
-        for (uint32_t s0 = 0; s0 < SP; s0 += 6) {
-            LLMR_PERSIST8_STAGE(X0, W0, X2, W1, R1, R0, s0 + 1)
-            LLMR_PERSIST8_STAGE(X1, W1, X0, W0, R2, R1, s0 + 2)
-            LLMR_PERSIST8_STAGE(X2, W0, X1, W1, R0, R2, s0 + 3)
-            LLMR_PERSIST8_STAGE(X0, W1, X2, W0, R1, R0, s0 + 4)
-            LLMR_PERSIST8_STAGE(X1, W0, X0, W1, R2, R1, s0 + 5)
-            LLMR_PERSIST8_STAGE(X2, W1, X1, W0, R0, R2, s0 + 6 == SP ? 0u : s0 + 6)
+        if constexpr (SPLITK) {
+            for (uint32_t s0 = S0;; s0 += 6) {
+                LLMR_PERSIST8_STAGE(X0, W0, X2, W1, R1, R0, s0 + 1)
+                if (s0 + 1 >= S) break;
+                LLMR_PERSIST8_STAGE(X1, W1, X0, W0, R2, R1, s0 + 2)
+                if (s0 + 2 >= S) break;
+                LLMR_PERSIST8_STAGE(X2, W0, X1, W1, R0, R2, s0 + 3)
+                if (s0 + 3 >= S) break;
+                LLMR_PERSIST8_STAGE(X0, W1, X2, W0, R1, R0, s0 + 4)
+                if (s0 + 4 >= S) break;
+                LLMR_PERSIST8_STAGE(X1, W0, X0, W1, R2, R1, s0 + 5)
+                if (s0 + 5 >= S) break;
+                LLMR_PERSIST8_STAGE(X2, W1, X1, W0, R0, R2, s0 + 6)
+                if (s0 + 6 >= S) break;
+            }
+        } else {
+            for (uint32_t s0 = 0; s0 < SP; s0 += 6) {
+                LLMR_PERSIST8_STAGE(X0, W0, X2, W1, R1, R0, s0 + 1)
+                LLMR_PERSIST8_STAGE(X1, W1, X0, W0, R2, R1, s0 + 2)
+                LLMR_PERSIST8_STAGE(X2, W0, X1, W1, R0, R2, s0 + 3)
+                LLMR_PERSIST8_STAGE(X0, W1, X2, W0, R1, R0, s0 + 4)
+                LLMR_PERSIST8_STAGE(X1, W0, X0, W1, R2, R1, s0 + 5)
+                LLMR_PERSIST8_STAGE(X2, W1, X1, W0, R0, R2, s0 + 6 == SP ? 0u : s0 + 6)
+            }
         }
         mfma_step(F1);
         store_tile(k);
@@ -1174,6 +1239,32 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const float* __restr
     f32x4 a = ((const f32x4*)P)[i];
     for (uint32_t q = 1; q < splits; q++) a += ((const f32x4*)(P + q * stride))[i];
     ((f32x4*)Y)[i] = a;
+}
+
+// The tiles past `full` of a split launch: tile full + t of Y = the sum over z of
+// its partial tiles P[z rem + t] (256 x 256 floats each), in split order. One
+// workgroup per 16 rows of a tile.
+__global__ void __launch_bounds__(256) splitk_tiles_kernel(const float* __restrict__ P, float* __restrict__ Y,
+                                                           uint32_t M, uint32_t N, uint32_t tiles_m, uint32_t tiles_n,
+                                                           uint32_t full, uint32_t rem, uint32_t splits) {
+    const uint32_t t = blockIdx.x >> 4, r0 = (blockIdx.x & 15u) * 16u + (threadIdx.x >> 6);
+    const uint32_t c = 4u * (threadIdx.x & 63u);
+    uint32_t tm, tn;
+    tile_of_linear(full + t, tiles_m, tiles_n, tm, tn);
+    const uint32_t n = tn * 256u + c, m0 = tm * 256u + (blockIdx.x & 15u) * 16u;
+    if (m0 >= M) return;
+    const float* const p = P + (uint64_t)t * 65536u + r0 * 256u + c;
+    f32x4 a[4];  // (rows past M in the last 16 hold leftovers that are not stored)
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) a[i] = *(const f32x4*)(p + i * 1024u);
+    for (uint32_t z = 1; z < splits; z++)
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) a[i] += *(const f32x4*)(p + (uint64_t)z * rem * 65536u + i * 1024u);
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        const uint32_t m = tm * 256u + r0 + 4u * i;
+        if (m < M && n < N) *(f32x4*)(Y + (uint64_t)m * N + n) = a[i];  // N % 4 == 0
+    }
 }
 
 }  // namespace
@@ -1416,6 +1507,52 @@ hipError_t launch_batch_matmul_swiglu(const void* wg, const void* wu, uint32_t w
     return hipGetLastError();
 }
 
+namespace {
+
+// The 256 x 256 tiles of one GEMM: the first pl.split_full whole, the rest cut
+// into pl.split K ranges (one workgroup each), then the sum of the partials.
+hipError_t launch_split(const void* w, uint32_t wtype, const void* x, uint32_t xtype, float* y, uint32_t N, uint32_t K,
+                        uint32_t M, uint32_t row_offset, const GemmPlan& pl, int num_cus, void* ws, hipStream_t st) {
+    const uint32_t tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256, total = tiles_m * tiles_n;
+    if (!plan::splits_nonempty(K / (uint32_t)kBK, pl.split) || N % 4 || K % kBK || pl.split_full >= total)
+        return hipErrorInvalidValue;
+    const void* x16 = x;
+    if (pl.convert_x) {
+        x16 = (uint8_t*)ws + pl.x16_off;
+        const hipError_t e = convert_activations(x, xtype, (void*)x16, pl.xt, (size_t)M * K, st);
+        if (e != hipSuccess) return e;
+    }
+    PersistArgs a{};
+    a.p[0] = PersistProblem{(const uint8_t*)w, x16, y, nullptr, nullptr, M, row_offset, tiles_m};
+    a.N = N;
+    a.K = K;
+    a.tiles_m = tiles_m;
+    a.tiles_n = tiles_n;
+    a.epi = kEpiStore;
+    a.ldy = N;
+    a.part = (float*)((uint8_t*)ws + pl.img_off);
+    a.split_full = pl.split_full;
+    a.split_cus = (uint32_t)num_cus;
+    a.split_stages = (K / (uint32_t)kBK + pl.split - 1u) / pl.split;
+    const uint32_t rem = total - pl.split_full;
+    const dim3 grid(pl.split_full + rem * pl.split), block(512);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, block, 0, st, a); };
+    if (wtype == kGgmlQ8_0) {
+        if (pl.xt == kGgmlF16) go(gemm_q_persist8<kGgmlQ8_0, kGgmlF16, kEpiStore, false, true>);
+        else go(gemm_q_persist8<kGgmlQ8_0, kGgmlBF16, kEpiStore, false, true>);
+    } else {
+        if (pl.xt == kGgmlF16) go(gemm_q_persist8<kGgmlQ4K, kGgmlF16, kEpiStore, false, true>);
+        else go(gemm_q_persist8<kGgmlQ4K, kGgmlBF16, kEpiStore, false, true>);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(splitk_tiles_kernel, dim3(rem * 16u), dim3(256), 0, st, a.part, y, M, N, tiles_m, tiles_n,
+                       pl.split_full, rem, pl.split);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uint32_t xtype,
                                float* y, uint32_t out_dim, uint32_t in_dim, uint32_t seq_len,
                                uint32_t row_offset, int num_cus, void* ws, hipStream_t st, size_t ws_limit) {
@@ -1426,6 +1563,7 @@ hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uin
     const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit);
     if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, st);
     if (pl.skinny) return launch_gemm_skinny(w, wtype, x, xtype, y, N, K, M, row_offset, pl.splits, ws, st);
+    if (pl.split > 1) return launch_split(w, wtype, x, xtype, y, N, K, M, row_offset, pl, num_cus, ws, st);
     if (!pl.persistent) {
         if (wtype == kGgmlQ8_0)
             return dispatch_w<kGgmlQ8_0>(w, xtype, x, y, N, K, M, row_offset, pl.tiles, (float*)ws, st);

@@ -57,6 +57,9 @@ struct PersistArgs {
     const uint8_t* W2;  // SwiGLU: the up weight (p[0].W is the gate)
     uint32_t N, K, tiles_m, tiles_n;  // tiles_m of both problems
     uint32_t epi, ldy, ldy2, split, y2_bf16;
+    // SPLITK launches: the tiles run whole, the CUs, K stages per split of the other tiles, their partial tiles
+    uint32_t split_full, split_cus, split_stages;
+    float* part;
     HeadsEpi heads;
     NextImages next;
 };
@@ -124,6 +127,13 @@ __device__ __forceinline__ void map_tile_persist(uint32_t T, uint32_t G, uint32_
         L = (T - b) + (b % kXcd) * (G / kXcd) + b / kXcd;
     }
     tile_of_linear(L, tiles_m, tiles_n, tm, tn);
+}
+
+// Workgroup b of a grid of G -> its position when the XCDs (b % 8) take
+// contiguous runs of G / 8 (+1 for the first G % 8) positions.
+__device__ __forceinline__ uint32_t xcd_linear(uint32_t b, uint32_t G) {
+    const uint32_t x = b % 8u;
+    return x * (G / 8u) + min(x, G % 8u) + b / 8u;
 }
 
 // The two-pass kernel's order (grid G = the CUs, G % 8 == 0): full rounds as

@@ -244,6 +244,48 @@ def test_persistent_every_tile(dev, wtype, M, N, K, xtype, row_offset):
     assert torch.equal(y, y2)
 
 
+# Launches below 2048 tokens whose last round of tiles is cut along K.
+SPLIT_TILE_CASES = [
+    # (wtype, M, N, K, xtype, row_offset)
+    (8, 1101, 3840, 3840, 0, 0),     # 75 tiles x 3 splits of 20 stages, f32 activations as fp16
+    (12, 1101, 3072, 3072, 0, 8),    # 60 tiles x 4, f32 activations as bf16, row_offset
+    (8, 257, 1028, 2048, 30, 0),     # one row and four features past a tile
+    (12, 513, 2052, 5120, 1, 4),     # splits of unequal stage counts
+    (8, 1536, 11520, 1088, 30, 0),   # 256 whole tiles, 14 cut into splits of 17 stages in all
+    (12, 2047, 9216, 3072, 30, 0),   # 256 whole tiles, 32 x 8
+]
+
+
+@pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", SPLIT_TILE_CASES)
+def test_split_tiles(dev, wtype, M, N, K, xtype, row_offset):
+    """Every 256 x 256 tile of a launch with tiles cut along K against an f32
+    product of the dequantized weight and the unrounded activations: within
+    the GEMM bar (a split left out or added twice is off by 1 / sqrt(16) or
+    more), the same bits again, and nothing written past the output."""
+    import torch
+    from llmr_amd import ops
+    w = _weights(dev, wtype, N + row_offset, K, 170 + wtype)
+    g = torch.Generator(device="cpu").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g)
+    x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
+    buf = torch.full(((M + 1) * N,), 7.0, device=dev)
+    y = buf[:M * N].view(M, N)
+    ops.batch_matmul(w, wtype, x, N, row_offset=row_offset, out=y)
+    ref = x.float() @ ops.dequant(w, wtype, N, K, row_offset).t()
+    torch.cuda.synchronize()
+    assert bool((buf[M * N:] == 7.0).all())
+    tm, tn = (M + 255) // 256, (N + 255) // 256
+    pad = (0, tn * 256 - N, 0, tm * 256 - M)
+    d2 = torch.nn.functional.pad((y - ref).double() ** 2, pad).view(tm, 256, tn, 256).sum((1, 3))
+    r2 = torch.nn.functional.pad(ref.double() ** 2, pad).view(tm, 256, tn, 256).sum((1, 3))
+    err = (d2 / r2).sqrt()
+    print(f"split tiles wtype={wtype} M={M} N={N} K={K}: worst tile rel_l2={float(err.max()):.3e}")
+    assert float(err.max()) <= TOL
+    y2 = ops.batch_matmul(w, wtype, x, N, row_offset=row_offset)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2)
+
+
 @pytest.mark.parametrize("name", ["flux_linear1", "flux_linear2", "zimage_qkv"])
 def test_full_size_sampled_rows(orc, dev, name):
     """Full-size launches; the oracle checks a sample of tokens (every column)."""
