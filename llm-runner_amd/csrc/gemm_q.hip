@@ -1392,9 +1392,16 @@ bool swiglu_fused(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M) {
 
 }  // namespace
 
+namespace {
+// Whether a GEMV kernel takes the launch (gemv_q.hip).
+bool runs_gemv(uint32_t wtype, uint32_t K, uint32_t M) {
+    return wtype == kGgmlQ4K ? M <= kGemvMaxTokens : gemv_q8_fits(K, M);
+}
+}  // namespace
+
 size_t batch_matmul_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M,
                                     int num_cus, size_t ws_limit) {
-    if (M == 0 || N == 0 || (wtype == kGgmlQ4K && M <= kGemvMaxTokens)) return 0;
+    if (M == 0 || N == 0 || runs_gemv(wtype, K, M)) return 0;
     return plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit).ws;
 }
 
@@ -1404,7 +1411,7 @@ namespace {
 GemmPlan lora_plan(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, uint32_t rank, int num_cus) {
     GemmPlan p{};
     if (rank == 0 || rank > kLoraImageMaxRank || M == 0 || N == 0) return p;
-    if (wtype == kGgmlQ4K && M <= kGemvMaxTokens) return p;
+    if (runs_gemv(wtype, K, M)) return p;
     p = plan_gemm(wtype, xtype, N, K, M, num_cus, kNoWorkspaceLimit);
     if (!p.two_pass) p = GemmPlan{};
     return p;
@@ -1558,8 +1565,9 @@ hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uin
                                uint32_t row_offset, int num_cus, void* ws, hipStream_t st, size_t ws_limit) {
     if (seq_len == 0 || out_dim == 0) return hipSuccess;
     const uint32_t N = out_dim, K = in_dim, M = seq_len;
-    if (wtype == kGgmlQ4K && M <= kGemvMaxTokens)
-        return launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, st);
+    if (runs_gemv(wtype, K, M))
+        return wtype == kGgmlQ4K ? launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, st)
+                                 : launch_gemv_q8(w, xtype, x, y, N, K, M, row_offset, st);
     const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit);
     if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, st);
     if (pl.skinny) return launch_gemm_skinny(w, wtype, x, xtype, y, N, K, M, row_offset, pl.splits, ws, st);

@@ -1,23 +1,19 @@
-// gemv_q.hip - Q4_K dequant-GEMM for a handful of tokens (M <= 4): the
+// gemv_q.hip - dequant-GEMM for a handful of tokens (M <= 4): the
 // modulation and timestep projections of a DiT step (M = 1) stream a whole
 // weight matrix for a few dot products, so they are bound by HBM reads of the
-// packed weight, not by the matrix cores. Here every weight byte is read
-// once, coalesced, dequantized in registers in f32 and used for all M tokens.
+// packed weight. Here every weight byte is read once and used for all M tokens.
 //
-// A wave covers 16 weight rows: lane t (of 16) walks superblocks t, t+16,
-// ..., and each lane serves 4 of the rows with one register copy of the
-// activations it needs (a 64-element slice per token at a time); the 16
-// partial sums of a row are reduced with lane shuffles. When the
-// activations fit in 48 KiB of LDS the variant below is used (activations
-// staged in LDS, 64-element units spread over all 16 lanes). Arithmetic is
-// f32 throughout, as the reference's batch_matmul_q4k (llm.slang:2264-2365)
-// with activations in f32: the register variant forms each weight as
-// (d*sc)*q - dmin*mn with one rounding (the FMA below; both products are
-// exact), as the reference does; the LDS variant sums the same products as
-// d*sc * sum q x - dmin*mn * sum x per 32-element sub-block (the activation
-// sums shared by a lane's rows), one FMA per weight instead of two VALU
-// operations (double-block modulation launch 379-416 -> 342-371 us).
+// gemv_i8_kernel (below) takes Q4_K and Q8_0 weights as long as the activations
+// fit its LDS; gemv_q4k_kernel is the Q4_K form for longer rows: a wave covers
+// 16 weight rows, lane t (of 16) walks superblocks t, t+16, ..., and each lane
+// serves 4 of the rows with one register copy of the activations it needs (a
+// 64-element slice per token at a time); the 16 partial sums of a row are
+// reduced with lane shuffles. Arithmetic is f32 throughout, as the reference's
+// batch_matmul_q4k (llm.slang:2264-2365) with activations in f32: each weight
+// is (d*sc)*q - dmin*mn with one rounding (the FMA; both products are exact).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "llmr_device.h"
 #include "llmr_internal.h"
@@ -141,23 +137,44 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
     }
 }
 
-// The same products with the activations staged in LDS (f32, once per
-// workgroup) and the work of a row split into 64-element units (quarter s
-// of superblock sb: its header and 32 quant bytes): lane t of 16 takes units
-// t, t+16, ..., so all lanes work whatever K / 256 is, and the next unit's
-// weight loads (header and quants of the lane's 4 rows) are issued before
-// the current unit is multiplied, keeping two units of loads in flight.
-constexpr uint32_t kGemvLdsBytes = 48u * 1024u;
-
-// 4 rows per lane (64 per workgroup): measured against 2 and 1, 4 is as fast
-// or faster at every Flux / Z-Image modulation shape.
-constexpr int kGemvRowsPerLane = 4;
-struct UnitW {
-    u32x4 hdr[4], qa[4], qb[4];  // the rows' header and 32 quant bytes of one unit
-};
+// ---------------------------------------------------------------------------
+// gemv_i8_kernel: the same products on the integer matrix cores.
+//
+// What bounds a projection of 1-4 tokens is the weight stream, if the vector
+// ALU keeps up: one FMA per weight on the nibble as a float took 3.6 VALU
+// instructions per weight and lane (18 us for the 31.9 MB of 18432 x 3072).
+// Here a 4x4x4 int8 MFMA (16 blocks of 4 x 4 outputs over 4 k each) multiplies
+// the quants as they are with the activations cut into four int8 digits:
+//  * a Q4_K nibble masked in place is an int8 (3 instructions for 8 weights), a
+//    Q8_0 quant is one already;
+//  * each activation, scaled by a power of two so that its 32-element
+//    sub-block's largest lies in [2^29, 2^30) and rounded to an integer (31
+//    bits under the largest), is the sum of four signed base-256 digits; sums of
+//    quant x digit over a sub-block are exact in int32, and the four of them
+//    make one f32 with a single rounding;
+//  * Q4_K: the sums start at -8 times the sub-block's digit sums, so they are of
+//    the quants less 8, and acc += (d sc) sum (q - 8) x - (dmin mn - 8 d sc) sum x
+//    cancels little of what the two f32 terms round.
+// That is at least as exact as f32 FMAs on f32 activations (18432 x 3072: 1.4e-7
+// relative to 64 bits, the FMA kernel 2.5e-7). An infinite or NaN activation has
+// no digits: such a workgroup multiplies in f32 (gemv_plain_row).
+// A wave owns 16 weight rows and walks them 4 units at a time: lane l = 16 rq +
+// 4 g + j has row 4 rq + j and unit g, so the four lanes of an MFMA block share
+// a unit. One token: the block's four rows of A are the token's digits; two to
+// four tokens: A's rows are the tokens, one MFMA per digit. The weight bytes are
+// loaded 16 bytes a lane along the rows (whole lines) a step ahead and change
+// lanes through the wave's own LDS region (a lane reads its 144 or 136 bytes at
+// conflict-free strides); no barrier in the loop. At one token and K = 3072 the
+// LDS holds three workgroups per CU. KS waves share 16 rows (each takes every
+// KS-th step), so that launches of few rows still put work on every CU.
+// Measured per call, before -> after (one token, FMA kernel; Q8_0, the few-token
+// GEMMs): 18432 x 3072 Q4_K 19.5 -> 9.7 us (3.3 TB/s), 38 of them grouped 328
+// -> 210 us (5.8 TB/s), 3072 x 15360 76 -> 12, two and four tokens of 18432 x
+// 3072 31 -> 16 and 56 -> 28 us; 11520 x 3840 Q8_0 54 -> 9.8 us (4.8 TB/s).
+// ---------------------------------------------------------------------------
 
 // Up to CAP projections of one shape [N, K] (each its own weight, input
-// and output rows, ldy apart): workgroup b serves rows 64 (b % bpj) .. of
+// and output rows, ldy apart): workgroup b serves rows (64 / KS) (b % bpj) .. of
 // job b / bpj. CAP = 1 for one projection, kGemvMaxJobs for a group.
 constexpr uint32_t kGemvMaxJobs = 64;
 template <uint32_t CAP>
@@ -168,145 +185,426 @@ struct GemvJobs {
     uint32_t m[CAP], row_offset[CAP];
 };
 
-template <uint32_t XT, int MM, uint32_t CAP, int RPL = kGemvRowsPerLane>
-__global__ void __launch_bounds__(256) gemv_q4k_lds_kernel(const GemvJobs<CAP> jobs, uint32_t N, uint32_t K,
-                                                            uint32_t ldy, uint32_t bpj) {
+// A lane's unit: a Q4_K super-block (256 k, 144 bytes) or four Q8_0 blocks
+// (128 k, 136 bytes; eight would keep the third workgroup off the CU). A step of
+// a wave is 16 rows x 4 units, loaded as 16-byte pieces along the rows.
+template <uint32_t WT>
+struct GemvW {
+    static constexpr uint32_t kK = WT == kGgmlQ4K ? 256u : 128u, kBytes = WT == kGgmlQ4K ? 144u : 136u;
+    static constexpr uint32_t kStep = 64u * kBytes, kRowPieces = 4u * kBytes / 16u;
+    static constexpr uint32_t kLoads = (16u * kRowPieces + 63u) / 64u;  // pieces per lane (Q8_0: half of the last)
+};
+
+// LDS of the activations per unit, T token slots (1, 2 or 4). Digits: 16 k at a
+// time, [digit][token][16 bytes]. Then per sub-block: Q4_K, the sums' start
+// [digit][token] (one token: [digit]); (1 / scale, activation sum) per token.
+// Units are padded so the four a wave reads together lie 64 bytes apart in the
+// banks.
+template <uint32_t WT, int T>
+struct GemvX {
+    static constexpr uint32_t kSub = GemvW<WT>::kK / 32u;
+    static constexpr uint32_t kDigits = GemvW<WT>::kK / 16u * (64u * T);
+    static constexpr uint32_t kStart = WT == kGgmlQ4K ? (T == 1 ? 16u : 64u) : 0u;
+    static constexpr uint32_t kSubBytes = kStart + (T == 4 ? 32u : 16u);
+    static constexpr uint32_t kUsed = kDigits + kSub * kSubBytes, kUnit = kUsed + (320u - kUsed % 256u) % 256u;
+};
+constexpr uint32_t kGemvLdsLimit = 160u * 1024u;
+template <uint32_t WT, int T>
+constexpr uint32_t gemv_lds_bytes(uint32_t K) {
+    const uint32_t nu4 = (K / GemvW<WT>::kK + 3u) / 4u * 4u;
+    return nu4 * GemvX<WT, T>::kUnit + 4u * GemvW<WT>::kStep + 16u;
+}
+
+// One dequantized weight: element k of the row at w.
+template <uint32_t WT>
+__device__ __forceinline__ float gemv_weight(const uint8_t* w, uint32_t k) {
+    if constexpr (WT == kGgmlQ8_0) {
+        const uint8_t* b = w + (uint64_t)(k / 32u) * 34u;
+        return f16_bits_to_f32((uint32_t)b[0] | ((uint32_t)b[1] << 8)) * (float)(int8_t)b[2u + k % 32u];
+    } else {
+        const uint8_t* b = w + (uint64_t)(k / 256u) * 144u;
+        const uint32_t e = k % 256u, i = e >> 5, qb = b[16u + 32u * (e >> 6) + (e & 31u)];
+        const u32x4 h = *(const u32x4_a4*)b;
+        uint32_t sc, mn;
+        q4k_scale_min(i, h.y, h.z, h.w, sc, mn);
+        const float d = f16_bits_to_f32(h.x & 0xffffu) * (float)sc, m = f16_bits_to_f32(h.x >> 16) * (float)mn;
+        return __builtin_fmaf((float)(i & 1u ? qb >> 4 : qb & 15u), d, -m);
+    }
+}
+template <uint32_t XT>
+__device__ __forceinline__ float gemv_x(const void* X, uint64_t e) {
+    if constexpr (XT == kGgmlF32) return ((const float*)X)[e];
+    const uint16_t v = ((const uint16_t*)X)[e];
+    if constexpr (XT == kGgmlBF16) return __uint_as_float((uint32_t)v << 16);
+    return (float)__builtin_bit_cast(_Float16, v);
+}
+// A row times token m in f32, by one wave.
+template <uint32_t WT, uint32_t XT>
+__device__ __forceinline__ float gemv_plain_row(const uint8_t* w, const void* X, uint32_t m, uint32_t K, uint32_t lane) {
+    float a = 0.0f;
+    for (uint32_t k = lane; k < K; k += 64u)
+        a = __builtin_fmaf(gemv_weight<WT>(w, k), gemv_x<XT>(X, (uint64_t)m * K + k), a);
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+    return a;
+}
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+
+template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
+__global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const GemvJobs<CAP> jobs, uint32_t N, uint32_t K,
+                                                          uint32_t ldy, uint32_t bpj) {
+    static_assert(T == 1 || T == 2 || T == 4, "one token, two, or up to four");
+    typedef GemvW<WT> GW;
+    typedef GemvX<WT, T> GX;
     const uint32_t job = CAP == 1u ? 0u : blockIdx.x / bpj;
     const uint32_t blk = CAP == 1u ? blockIdx.x : blockIdx.x - job * bpj;
-    const uint8_t* __restrict__ W = jobs.w[job];
     const void* __restrict__ X = jobs.x[job];
     float* __restrict__ Y = jobs.y[job];
-    const uint32_t M = jobs.m[job], row_offset = jobs.row_offset[job];
-    extern __shared__ f32x4 xs[];  // [M][K / 4]
-    const uint32_t K4 = K / 4u;
-#pragma unroll
-    for (int m = 0; m < MM; ++m)
-        if (m < (int)M)
-            for (uint32_t i = threadIdx.x; i < K4; i += 256u) xs[m * K4 + i] = load_x4<XT>(X, (uint64_t)m * K + 4u * i);
-    __syncthreads();
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t t = lane & 15u, r = lane >> 4;
-    const uint32_t n0 = blk * (16u * RPL) + wave * (4u * RPL) + r;  // rows n0 + 4i, i < RPL
-    const uint32_t U = (K / 256u) * 4u;
-    const uint64_t rb = (uint64_t)(K / 256u) * 144u;
-    // rows past N read row N - 1 (in bounds, branch-free) and are not stored
-    auto load_unit = [&](uint32_t u) __attribute__((always_inline)) {
-        const uint32_t sb = u >> 2, j = u & 3u;
-        UnitW w;
-#pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            const uint32_t n = min(n0 + 4u * i, N - 1u);
-            const uint8_t* b = W + (uint64_t)(row_offset + n) * rb + (uint64_t)sb * 144u;
-            w.hdr[i] = *(const u32x4_a4*)b;
-            w.qa[i] = *(const u32x4_a4*)(b + 16u + 32u * j);
-            w.qb[i] = *(const u32x4_a4*)(b + 32u + 32u * j);
+    const uint32_t M = jobs.m[job];
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    const uint32_t nu = K / GW::kK, steps = (nu + 3u) / 4u, nu4 = 4u * steps;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t* const wsb = smem + nu4 * GX::kUnit;
+    uint8_t* const ws = wsb + wave * GW::kStep;           // the wave's weight bytes of a step
+    uint32_t* const odd = (uint32_t*)(wsb + 4u * GW::kStep);  // an activation is infinite or NaN
+    if (tid == 0) *odd = 0u;
+
+    // activations: thread -> 8 k of one token, four neighbours a sub-block; the
+    // first pieces (all of them up to K = 4096) are requested before the weights
+    // (loads return in order: behind the weights they would wait for them)
+    const uint32_t pieces = nu4 * (GW::kK / 8u), total = pieces * (uint32_t)T;
+    struct X8 {
+        f32x4 a, b;
+    };
+    auto load_x = [&](uint32_t i) __attribute__((always_inline)) {
+        X8 v{};
+        const uint32_t m = T == 1 ? 0u : i / pieces, k = 8u * (T == 1 ? i : i - m * pieces);
+        if (i < total && m < M && k < K) {
+            v.a = load_x4<XT>(X, (uint64_t)m * K + k);
+            v.b = load_x4<XT>(X, (uint64_t)m * K + k + 4u);
         }
+        return v;
+    };
+    constexpr uint32_t kAhead = T == 1 ? 2u : T == 2 ? 4u : 8u;
+    X8 xa[kAhead];
+#pragma unroll
+    for (uint32_t q = 0; q < kAhead; q++) xa[q] = load_x(tid + 256u * q);
+
+    // the wave's 16 rows as a buffer: rows past N read as zero
+    const uint32_t n0 = blk * (64u / KS) + wave / KS * 16u, rb = nu * GW::kBytes;
+    const uint8_t* const W = jobs.w[job] + (uint64_t)jobs.row_offset[job] * rb;
+    const uint32_t wbytes = n0 < N ? min(16u, N - n0) * rb : 0u;
+    uint32_t voff[GW::kLoads];  // piece c = 64 i + lane of a step: row c / kRowPieces, 16 (c % kRowPieces) bytes in
+#pragma unroll
+    for (uint32_t i = 0; i < GW::kLoads; i++) {
+        const uint32_t c = 64u * i + lane, r = c / GW::kRowPieces;
+        voff[i] = r < 16u ? r * rb + 16u * (c - r * GW::kRowPieces) : 0x80000000u;
+    }
+    struct Set {
+        u32x4 v[GW::kLoads];
+    };
+    // (the last step may read into the next row: those units are masked below)
+    auto load_w = [&](uint32_t s) __attribute__((always_inline)) {
+        Set w;
+        const rsrc_t r = make_rsrc(W + (uint64_t)n0 * rb, s < steps ? wbytes : 0u);
+#pragma unroll
+        for (uint32_t i = 0; i < GW::kLoads; i++)
+            w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i], 4u * GW::kBytes * s, 0));
         return w;
     };
-    float acc[4][MM];
+    const uint32_t s0 = wave % KS;
+    Set set = load_w(s0);
+    __syncthreads();  // odd is cleared
+
+    bool bad = false;
+    auto stage_x = [&](uint32_t i, const X8& v) __attribute__((always_inline)) {
+        const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
+        float mx = 0.0f, sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
 #pragma unroll
-    for (int i = 0; i < RPL; i++)
+        for (int e = 0; e < 8; e++) {
+            bad = bad || !(__builtin_fabsf(x[e]) < INFINITY);
+            mx = fmaxf(mx, __builtin_fabsf(x[e]));
+        }
 #pragma unroll
-        for (int m = 0; m < MM; m++) acc[i][m] = 0.0f;
-    // (U >= 4 > t is not guaranteed for K = 256: lanes t >= U have no unit)
-    UnitW cur = load_unit(min(t, U - 1u));
-    for (uint32_t u = t; u < U; u += 16u) {
-        const UnitW nxt = load_unit(min(u + 16u, U - 1u));
-        const uint32_t sb = u >> 2, j = u & 3u;
+        for (int o = 1; o < 4; o <<= 1) {
+            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+            sum += __shfl_xor(sum, o, 64);
+        }
+        // scale 2^e with 2^e mx in [2^29, 2^30), e kept where 2^e and 2^-e are normal
+        const int e = min(126, max(-126, 156 - (int)((__float_as_uint(mx) >> 23) & 0xffu)));
+        const float up = __uint_as_float((uint32_t)(127 + e) << 23), down = __uint_as_float((uint32_t)(127 - e) << 23);
+        uint32_t dg[2][4];  // [four k][digit, lowest first]: a byte per k
+        int start[4] = {0, 0, 0, 0};
 #pragma unroll
-        for (int m = 0; m < MM; ++m) {
-            if (m >= (int)M) continue;
-            // activations of elements 64j .. 64j+63 of superblock sb
-            const f32x4* xr = xs + m * K4 + sb * 64u + 16u * j;
-            f32x4 xl[8], xh[8];
+        for (int h = 0; h < 2; h++) {
+            uint32_t v4[4];
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                xl[c] = xr[c];
-                xh[c] = xr[c + 8];
+            for (int q = 0; q < 4; q++) {
+                // |v| < 2^30 + 1: adding 0x808080 and flipping those bits turns the
+                // three low bytes into signed digits (the carries go up)
+                const int i32 = (int)rintf(x[4 * h + q] * up);
+                v4[q] = ((uint32_t)i32 + 0x00808080u) ^ 0x00808080u;
             }
-            // the sub-blocks' activation sums, shared by the lane's rows
-            float sxl = 0.0f, sxh = 0.0f;
+            // 4 x 4 byte transpose
+            const uint32_t a0 = __builtin_amdgcn_perm(v4[1], v4[0], 0x05010400u);  // b0 b0' b1 b1'
+            const uint32_t a1 = __builtin_amdgcn_perm(v4[1], v4[0], 0x07030602u);  // b2 b2' b3 b3'
+            const uint32_t c0 = __builtin_amdgcn_perm(v4[3], v4[2], 0x05010400u);
+            const uint32_t c1 = __builtin_amdgcn_perm(v4[3], v4[2], 0x07030602u);
+            dg[h][0] = __builtin_amdgcn_perm(c0, a0, 0x05040100u);
+            dg[h][1] = __builtin_amdgcn_perm(c0, a0, 0x07060302u);
+            dg[h][2] = __builtin_amdgcn_perm(c1, a1, 0x05040100u);
+            dg[h][3] = __builtin_amdgcn_perm(c1, a1, 0x07060302u);
+            if constexpr (WT == kGgmlQ4K)
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                sxl += (xl[c].x + xl[c].y) + (xl[c].z + xl[c].w);
-                sxh += (xh[c].x + xh[c].y) + (xh[c].z + xh[c].w);
+                for (int p = 0; p < 4; p++) start[p] = __builtin_amdgcn_sdot4((int)dg[h][p], 0x01010101, start[p], false);
+        }
+        if constexpr (WT == kGgmlQ4K)
+#pragma unroll
+            for (int p = 0; p < 4; p++) {
+                start[p] += __shfl_xor(start[p], 1, 64);
+                start[p] += __shfl_xor(start[p], 2, 64);
+                start[p] *= -8;
             }
+        if (i >= total) return;
+        const uint32_t m = T == 1 ? 0u : i / pieces, c = T == 1 ? i : i - m * pieces;  // chunk of 8 k
+        const uint32_t u = c / (GW::kK / 8u), cu = c % (GW::kK / 8u);
+        uint8_t* const dst = smem + u * GX::kUnit + cu / 2u * (64u * T) + m * 16u + 8u * (cu & 1u);
 #pragma unroll
-            for (int i = 0; i < RPL; ++i) {
-                const float d = f16_bits_to_f32(cur.hdr[i].x & 0xffffu), dmin = f16_bits_to_f32(cur.hdr[i].x >> 16);
-                uint32_t sc0, mn0, sc1, mn1;
-                q4k_scale_min(2u * j, cur.hdr[i].y, cur.hdr[i].z, cur.hdr[i].w, sc0, mn0);
-                q4k_scale_min(2u * j + 1u, cur.hdr[i].y, cur.hdr[i].z, cur.hdr[i].w, sc1, mn1);
-                const float d0 = d * (float)sc0, m0 = dmin * (float)mn0;
-                const float d1 = d * (float)sc1, m1 = dmin * (float)mn1;
-                // sum (d0 q - m0) x = d0 sum q x - m0 sum x per 32-element
-                // sub-block: one FMA per weight on the nibble as a float
-                float ql = 0.0f, qh = 0.0f;
+        for (int p = 0; p < 4; p++) *(u32x2*)(dst + p * (16u * T)) = u32x2{dg[0][p], dg[1][p]};
+        if (cu % 4u == 0u) {
+            uint8_t* const sb = smem + u * GX::kUnit + GX::kDigits + cu / 4u * GX::kSubBytes;
+            if constexpr (WT == kGgmlQ4K) {
+                if constexpr (T == 1) {
+                    *(i32x4*)sb = i32x4{start[0], start[1], start[2], start[3]};
+                } else {
 #pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    const uint32_t word = c < 4 ? cur.qa[i][c] : cur.qb[i][c - 4];
-                    // nibbles in the bytes of lo / hi; hidden from the compiler's
-                    // known bits so each byte converts with one v_cvt_f32_ubyteN
-                    // (seen as a 4-bit field it extracts with v_bfe_u32 first)
-                    uint32_t lo = word & 0x0f0f0f0fu, hi = (word >> 4) & 0x0f0f0f0fu;
-                    asm("" : "+v"(lo), "+v"(hi));
-                    const f32x4 a = xl[c], h = xh[c];
-                    ql = __builtin_fmaf((float)(lo & 0xffu), a.x, ql);
-                    ql = __builtin_fmaf((float)((lo >> 8) & 0xffu), a.y, ql);
-                    ql = __builtin_fmaf((float)((lo >> 16) & 0xffu), a.z, ql);
-                    ql = __builtin_fmaf((float)(lo >> 24), a.w, ql);
-                    qh = __builtin_fmaf((float)(hi & 0xffu), h.x, qh);
-                    qh = __builtin_fmaf((float)((hi >> 8) & 0xffu), h.y, qh);
-                    qh = __builtin_fmaf((float)((hi >> 16) & 0xffu), h.z, qh);
-                    qh = __builtin_fmaf((float)(hi >> 24), h.w, qh);
+                    for (int p = 0; p < 4; p++) *(int*)(sb + 16u * p + 4u * m) = start[p];  // (rows past T: unused)
                 }
-                acc[i][m] += (d0 * ql - m0 * sxl) + (d1 * qh - m1 * sxh);
             }
+            *(f32x2*)(sb + GX::kStart + 8u * m) = f32x2{down, sum};
         }
-        cur = nxt;
+    };
+#pragma unroll
+    for (uint32_t q = 0; q < kAhead; q++)
+        if (256u * q < total) stage_x(tid + 256u * q, xa[q]);
+    for (uint32_t i = 256u * kAhead + tid; i < (total + 255u) / 256u * 256u; i += 256u) stage_x(i, load_x(i));
+    if (bad) *odd = 1u;
+    __syncthreads();
+    if (*odd != 0u) {  // a whole workgroup's branch: nothing below waits for it
+        for (uint32_t r = wave; r < 64u / KS; r += 4u)
+            for (uint32_t m = 0; m < M; m++) {
+                const uint32_t n = blk * (64u / KS) + r;
+                if (n >= N) continue;
+                const float a = gemv_plain_row<WT, XT>(W + (uint64_t)n * rb, X, m, K, lane);
+                if (lane == 0) Y[(uint64_t)m * ldy + n] = a;
+            }
+        return;
     }
+
+    const uint32_t j = lane & 3u, g = (lane >> 2) & 3u, rq = lane >> 4;
+    const uint8_t* const wl = ws + ((4u * rq + j) * 4u + g) * GW::kBytes;
+    float acc[T];
 #pragma unroll
-    for (int i = 0; i < RPL; i++)
+    for (int m = 0; m < T; m++) acc[m] = 0.0f;
+    constexpr int P = T == 1 ? 1 : 4;  // accumulator tiles: [digits] of one token, or [tokens] per digit
+
+    // D += A B for 16 k of two sub-blocks at once (independent accumulators, so
+    // the MFMAs follow each other): w the lane's quants (16 bytes), xb the
+    // unit's digits of these 16 k; this lane's row of A is digit j (one token)
+    // or token j
+    auto mul16 = [&](i32x4 (&d)[P], const uint8_t* xb, u32x4 w, i32x4 (&d2)[P], const uint8_t* xb2, u32x4 w2)
+        __attribute__((always_inline)) {
+        u32x4 a[P], a2[P];
 #pragma unroll
-        for (int m = 0; m < MM; m++) {
-#pragma unroll
-            for (int o = 8; o > 0; o >>= 1) acc[i][m] += __shfl_xor(acc[i][m], o, 64);
+        for (int p = 0; p < P; p++) {
+            const uint32_t at = 16u * T * p + (T == 1 ? 16u * j : 16u * (j % T));
+            a[p] = *(const u32x4*)(xb + at);
+            a2[p] = *(const u32x4*)(xb2 + at);
         }
-    if (t == 0) {
 #pragma unroll
-        for (int i = 0; i < RPL; i++) {
-            const uint32_t n = n0 + 4u * i;
-            if (n < N) {
+        for (int q = 0; q < 4; q++) {
 #pragma unroll
-                for (int m = 0; m < MM; m++)
-                    if (m < (int)M) Y[(uint64_t)m * ldy + n] = acc[i][m];
+            for (int p = 0; p < P; p++) d[p] = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a[p][q], (int)w[q], d[p], 0, 0, 0);
+#pragma unroll
+            for (int p = 0; p < P; p++)
+                d2[p] = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a2[p][q], (int)w2[q], d2[p], 0, 0, 0);
+        }
+    };
+    auto begin = [&](i32x4 (&d)[P], const uint8_t* sb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < P; p++) {
+            if constexpr (WT == kGgmlQ4K)
+                d[p] = *(const i32x4*)(sb + 16u * p);
+            else
+                d[p] = i32x4{0, 0, 0, 0};
+        }
+    };
+    // acc += ds (sum q x) - dm (sum x) of one sub-block
+    auto add = [&](const i32x4 (&d)[P], const uint8_t* sb, float ds, float dm) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < T; m++) {
+            const f32x2 s = *(const f32x2*)(sb + GX::kStart + 8u * m);
+            const int d0 = T == 1 ? d[0].x : d[0][m], d1 = T == 1 ? d[0].y : d[1 % P][m];
+            const int d2 = T == 1 ? d[0].z : d[2 % P][m], d3 = T == 1 ? d[0].w : d[3 % P][m];
+            // both pairs are below 2^24
+            const float t = __builtin_fmaf((float)(d3 * 256 + d2), 65536.0f, (float)(d1 * 256 + d0));
+            acc[m] = __builtin_fmaf(ds * t, s.x, acc[m]);
+            if constexpr (WT == kGgmlQ4K) acc[m] = __builtin_fmaf(-dm, s.y, acc[m]);
+        }
+    };
+
+    for (uint32_t s = s0; s < steps; s += KS) {
+        // the step's bytes into the wave's region (its reads of the step before
+        // are done: a wave's LDS accesses run in order), the next step's loads out
+#pragma unroll
+        for (uint32_t i = 0; i < GW::kLoads; i++)
+            if (64u * i + 63u < 16u * GW::kRowPieces || 64u * i + lane < 16u * GW::kRowPieces)
+                *(u32x4*)(ws + 1024u * i + 16u * lane) = set.v[i];
+        set = load_w(s + KS);
+        const uint32_t u = 4u * s + g;
+        const bool live = u < nu;  // (a unit past the row adds 0)
+        const uint8_t* const xb = smem + u * GX::kUnit;
+        const uint8_t* const sb = xb + GX::kDigits;
+        if constexpr (WT == kGgmlQ4K) {
+            const u32x4 h = *(const u32x4*)wl;
+            const uint32_t s0w = h.y, s1w = h.z, s2w = h.w;
+            const float dd = live ? f16_bits_to_f32(h.x & 0xffffu) : 0.0f;
+            const float dmin = live ? f16_bits_to_f32(h.x >> 16) : 0.0f;
+            // get_scale_min_k4 of the eight sub-blocks, four bytes at a time
+            const uint32_t sc4[2] = {s0w & 0x3f3f3f3fu, (s2w & 0x0f0f0f0fu) | ((s0w >> 2) & 0x30303030u)};
+            const uint32_t mn4[2] = {s1w & 0x3f3f3f3fu, ((s2w >> 4) & 0x0f0f0f0fu) | ((s1w >> 2) & 0x30303030u)};
+#pragma unroll
+            for (int q = 0; q < 4; q++) {  // sub-blocks 2q (low nibbles) and 2q + 1 (high)
+                __builtin_amdgcn_sched_barrier(0);  // one quarter's operands at a time
+                const u32x4 qa = *(const u32x4*)(wl + 16u + 32u * q), qb = *(const u32x4*)(wl + 32u + 32u * q);
+                const u32x4 m4 = {0x0f0f0f0fu, 0x0f0f0f0fu, 0x0f0f0f0fu, 0x0f0f0f0fu};
+                i32x4 lo[P], hi[P];
+                begin(lo, sb + (2u * q) * GX::kSubBytes);
+                begin(hi, sb + (2u * q + 1u) * GX::kSubBytes);
+                mul16(lo, xb + (4u * q) * (64u * T), qa & m4, hi, xb + (4u * q + 2u) * (64u * T), (qa >> 4) & m4);
+                mul16(lo, xb + (4u * q + 1u) * (64u * T), qb & m4, hi, xb + (4u * q + 3u) * (64u * T), (qb >> 4) & m4);
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const uint32_t b = 2u * q + e;
+                    const float ds = dd * (float)((sc4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
+                    const float dm = dmin * (float)((mn4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
+                    add(e ? hi : lo, sb + b * GX::kSubBytes, ds, __builtin_fmaf(-8.0f, ds, dm));
+                }
+            }
+        } else {
+            // four blocks of 34 bytes: block b's scale at byte 34 b, its quants two bytes on
+            uint32_t wd[34];
+#pragma unroll
+            for (int i = 0; i < 17; i++) {
+                const u32x2 v = *(const u32x2*)(wl + 8u * i);
+                wd[2 * i] = v.x;
+                wd[2 * i + 1] = v.y;
+            }
+#pragma unroll
+            for (int b = 0; b < 4; b += 2) {  // block b's quants lie two bytes past a dword, block b + 1's on one
+                __builtin_amdgcn_sched_barrier(0);
+                const int dw = 17 * (b / 2);
+                uint32_t q[8], q2[8];  // quant bytes 4 i .. 4 i + 3 of each block
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    q[i] = __builtin_amdgcn_alignbyte(wd[dw + i + 1], wd[dw + i], 2);
+                    q2[i] = wd[dw + 9 + i];
+                }
+                i32x4 t[P], t2[P];
+                begin(t, sb);
+                begin(t2, sb);
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    mul16(t, xb + (2u * b + h) * (64u * T), u32x4{q[4 * h], q[4 * h + 1], q[4 * h + 2], q[4 * h + 3]},
+                          t2, xb + (2u * b + 2u + h) * (64u * T),
+                          u32x4{q2[4 * h], q2[4 * h + 1], q2[4 * h + 2], q2[4 * h + 3]});
+                add(t, sb + b * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw] & 0xffffu) : 0.0f, 0.0f);
+                add(t2, sb + (b + 1) * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw + 8] >> 16) : 0.0f, 0.0f);
             }
         }
+    }
+
+    // the four unit lanes of a row, then the KS waves, in wave order
+    const uint32_t r = 4u * rq + j;
+#pragma unroll
+    for (int m = 0; m < T; m++) {
+        acc[m] += __shfl_xor(acc[m], 4, 64);
+        acc[m] += __shfl_xor(acc[m], 8, 64);
+    }
+    if constexpr (KS > 1) {
+        float* const red = (float*)wsb;  // [wave][token][row], over the waves' weight regions
+        __syncthreads();
+        if (g == 0)
+#pragma unroll
+            for (int m = 0; m < T; m++) red[(wave * T + m) * 16u + r] = acc[m];
+        __syncthreads();
+        for (uint32_t i = tid; i < 64u / KS * T; i += 256u) {
+            const uint32_t row = i % (64u / KS), m = i / (64u / KS), w0 = row / 16u * KS, n = blk * (64u / KS) + row;
+            float v = red[(w0 * T + m) * 16u + row % 16u];
+#pragma unroll
+            for (uint32_t w = 1; w < KS; w++) v += red[((w0 + w) * T + m) * 16u + row % 16u];
+            if (n < N && m < M) Y[(uint64_t)m * ldy + n] = v;
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < T; m++)
+            if (g == 0 && n0 + r < N && (uint32_t)m < M) Y[(uint64_t)m * ldy + n0 + r] = acc[m];
     }
 }
 
-template <uint32_t XT, uint32_t CAP>
-void launch_lds(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy, uint32_t max_m,
-                hipStream_t st) {
-    const uint32_t bpj = (N + 16u * kGemvRowsPerLane - 1u) / (16u * kGemvRowsPerLane);
-    const dim3 grid(bpj * n_jobs), block(256);
-    const uint32_t lds = max_m * K * 4u;
-    if (max_m <= 1)
-        hipLaunchKernelGGL((gemv_q4k_lds_kernel<XT, 1, CAP>), grid, block, lds, st, jobs, N, K, ldy, bpj);
-    else if (max_m <= 2)
-        hipLaunchKernelGGL((gemv_q4k_lds_kernel<XT, 2, CAP>), grid, block, lds, st, jobs, N, K, ldy, bpj);
-    else
-        hipLaunchKernelGGL((gemv_q4k_lds_kernel<XT, 4, CAP>), grid, block, lds, st, jobs, N, K, ldy, bpj);
+// Whether gemv_i8_kernel takes M tokens x K: whole super-blocks (Q8_0 rows in
+// whole 16-byte pieces) and the digits in LDS.
+template <uint32_t WT>
+bool gemv_fits(uint32_t K, uint32_t M) {
+    if (M == 0 || M > kGemvMaxTokens || K % 256u || K == 0 || K > (1u << 20)) return false;
+    return (M == 1 ? gemv_lds_bytes<WT, 1>(K) : M == 2 ? gemv_lds_bytes<WT, 2>(K) : gemv_lds_bytes<WT, 4>(K)) <=
+           kGemvLdsLimit;
+}
+
+template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
+hipError_t launch_gemv_k(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
+                         hipStream_t st) {
+    auto kern = gemv_i8_kernel<WT, XT, T, CAP, KS>;
+    static const hipError_t attr =
+        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvLdsLimit);
+    if (attr != hipSuccess) return attr;
+    const uint32_t rows = 64u / KS, bpj = (N + rows - 1u) / rows;
+    hipLaunchKernelGGL(kern, dim3(bpj * n_jobs), dim3(256), (gemv_lds_bytes<WT, T>(K)), st, jobs, N, K, ldy, bpj);
+    return hipGetLastError();
+}
+
+// Fewer than 128 workgroups of 64 rows leave half the CUs without one: the
+// four waves then share 16 rows (one token, 3072 x 15360 Q4_K: 24 -> 12 us; four
+// tokens, 3072 x 3072: 13.6 -> 9.4). From 128 on it costs more, as every
+// workgroup cuts the activations into digits (four tokens, 9216 x 3072: 13.7
+// against 25 us; one token, 18432 x 3072: 9.7 against 11.1).
+template <uint32_t WT, uint32_t XT, int T, uint32_t CAP>
+hipError_t launch_gemv_t(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
+                         hipStream_t st) {
+    if ((N + 63u) / 64u * n_jobs < 128u) return launch_gemv_k<WT, XT, T, CAP, 4>(jobs, n_jobs, N, K, ldy, st);
+    return launch_gemv_k<WT, XT, T, CAP, 1>(jobs, n_jobs, N, K, ldy, st);
+}
+
+template <uint32_t WT, uint32_t CAP>
+hipError_t launch_gemv(uint32_t xtype, const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
+                       uint32_t max_m, hipStream_t st) {
+    auto by_x = [&](auto xt) {
+        constexpr uint32_t XT = decltype(xt)::value;
+        return max_m <= 1   ? launch_gemv_t<WT, XT, 1, CAP>(jobs, n_jobs, N, K, ldy, st)
+               : max_m <= 2 ? launch_gemv_t<WT, XT, 2, CAP>(jobs, n_jobs, N, K, ldy, st)
+                            : launch_gemv_t<WT, XT, 4, CAP>(jobs, n_jobs, N, K, ldy, st);
+    };
+    switch (xtype) {
+        case kGgmlF32: return by_x(std::integral_constant<uint32_t, kGgmlF32>{});
+        case kGgmlF16: return by_x(std::integral_constant<uint32_t, kGgmlF16>{});
+        default: return by_x(std::integral_constant<uint32_t, kGgmlBF16>{});
+    }
 }
 
 template <uint32_t XT>
 hipError_t launch_t(const void* w, const void* x, float* y, uint32_t N, uint32_t K, uint32_t M, uint32_t row_offset,
                     hipStream_t st) {
-    if ((uint64_t)M * K * 4u <= kGemvLdsBytes) {
-        const GemvJobs<1> one{{(const uint8_t*)w}, {x}, {y}, {M}, {row_offset}};
-        launch_lds<XT>(one, 1u, N, K, N, M, st);
-        return hipGetLastError();
-    }
     const dim3 grid((N + 63u) / 64u), block(256);
     const uint8_t* W = (const uint8_t*)w;
     if (M <= 1) hipLaunchKernelGGL((gemv_q4k_kernel<XT, 1>), grid, block, 0, st, W, x, y, N, K, M, row_offset);
@@ -324,7 +622,6 @@ hipError_t launch_gemv_q4k_multi(uint32_t xtype, const GemmJob* jobs, uint32_t n
     GemvJobs<kGemvMaxJobs> t{};
     uint32_t max_m = 0;
     for (uint32_t q = 0; q < n_jobs; q++) {
-        if (jobs[q].M > kGemvMaxTokens || (uint64_t)jobs[q].M * K * 4u > kGemvLdsBytes) return hipErrorNotSupported;
         t.w[q] = (const uint8_t*)jobs[q].w;
         t.x[q] = jobs[q].x;
         t.y[q] = jobs[q].y;
@@ -333,23 +630,33 @@ hipError_t launch_gemv_q4k_multi(uint32_t xtype, const GemmJob* jobs, uint32_t n
         max_m = max(max_m, jobs[q].M);
     }
     if (max_m == 0) return hipSuccess;
-    switch (xtype) {
-        case kGgmlF32: launch_lds<kGgmlF32>(t, n_jobs, N, K, ldy, max_m, st); break;
-        case kGgmlF16: launch_lds<kGgmlF16>(t, n_jobs, N, K, ldy, max_m, st); break;
-        default: launch_lds<kGgmlBF16>(t, n_jobs, N, K, ldy, max_m, st); break;
-    }
-    return hipGetLastError();
+    if (!gemv_fits<kGgmlQ4K>(K, max_m)) return hipErrorNotSupported;
+    return launch_gemv<kGgmlQ4K>(xtype, t, n_jobs, N, K, ldy, max_m, st);
 }
 
 hipError_t launch_gemv_q4k(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K,
                            uint32_t M, uint32_t row_offset, hipStream_t st) {
     if (M == 0 || N == 0) return hipSuccess;
     if (M > kGemvMaxTokens) return hipErrorInvalidValue;
+    if (gemv_fits<kGgmlQ4K>(K, M)) {
+        const GemvJobs<1> one{{(const uint8_t*)w}, {x}, {y}, {M}, {row_offset}};
+        return launch_gemv<kGgmlQ4K>(xtype, one, 1u, N, K, N, M, st);
+    }
     switch (xtype) {
         case kGgmlF32: return launch_t<kGgmlF32>(w, x, y, N, K, M, row_offset, st);
         case kGgmlF16: return launch_t<kGgmlF16>(w, x, y, N, K, M, row_offset, st);
         default: return launch_t<kGgmlBF16>(w, x, y, N, K, M, row_offset, st);
     }
+}
+
+bool gemv_q8_fits(uint32_t K, uint32_t M) { return gemv_fits<kGgmlQ8_0>(K, M); }
+
+hipError_t launch_gemv_q8(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K, uint32_t M,
+                          uint32_t row_offset, hipStream_t st) {
+    if (M == 0 || N == 0) return hipSuccess;
+    if (!gemv_fits<kGgmlQ8_0>(K, M)) return hipErrorInvalidValue;
+    const GemvJobs<1> one{{(const uint8_t*)w}, {x}, {y}, {M}, {row_offset}};
+    return launch_gemv<kGgmlQ8_0>(xtype, one, 1u, N, K, N, M, st);
 }
 
 }  // namespace llmr

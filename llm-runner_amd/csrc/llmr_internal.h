@@ -100,6 +100,11 @@ using plan::kGemvMaxTokens;
 hipError_t launch_gemv_q4k(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K,
                            uint32_t M, uint32_t row_offset, hipStream_t st);
 
+// The same for Q8_0 weights, where gemv_q8_fits.
+bool gemv_q8_fits(uint32_t K, uint32_t M);
+hipError_t launch_gemv_q8(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K, uint32_t M,
+                          uint32_t row_offset, hipStream_t st);
+
 // SwiGLU of two Q8_0 GEMMs (batch_matmul_swiglu_q8). `ws` must hold
 // swiglu_workspace_bytes(...) bytes (may be 0).
 size_t swiglu_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t out_dim, uint32_t in_dim,

@@ -85,6 +85,66 @@ def test_small_m_q4k_f32_matches_reference_arithmetic(orc, dev, M, N, K, row_off
     assert err <= 1e-5
 
 
+@pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", [
+    (12, 1, 8256, 768, 0, 0),      # 129 workgroups of 64 rows; three super-blocks of a step's four
+    (12, 2, 8193, 256, 0, 3),      # one row past a workgroup, one super-block
+    (12, 3, 8200, 1280, 30, 0),    # five super-blocks: a second step of one
+    (12, 4, 77, 2304, 1, 16),      # few rows: the waves share them, nine super-blocks
+    (12, 1, 5, 4352, 0, 0),        # 17 super-blocks, five rows
+    (8, 1, 8240, 256, 0, 0),       # Q8_0: two units of a step's four
+    (8, 3, 8195, 1792, 1, 2),      # 14 units
+    (8, 2, 130, 768, 30, 0),
+    (8, 4, 33, 3840, 0, 5),
+])
+def test_gemv_against_64_bits(dev, wtype, M, N, K, xtype, row_offset):
+    """At most four tokens: int8 digits of the activations times the quants,
+    exact sums per 32-element sub-block, f32 over the sub-blocks: relative L2
+    against float64 of the same weights and activations below 1e-6 (at most
+    2 x 68 f32 additions per lane, 2^-24 each at random signs: 7e-7). One
+    activation of 1e6 and one of 1e-6 per token: the digits scale per
+    sub-block."""
+    import torch
+    from llmr_amd import ops
+    w = _weights(dev, wtype, N + row_offset, K, 270 + wtype)
+    g = torch.Generator(device="cpu").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g)
+    if xtype != 1:
+        x[:, K // 2] = 1e6
+    x[:, 3] = 1e-6
+    x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
+    buf = torch.full((M * N + 64,), 7.0, device=dev)
+    y = buf[:M * N].view(M, N)
+    ops.batch_matmul(w, wtype, x, N, row_offset=row_offset, out=y)
+    ref = x.double() @ ops.dequant(w, wtype, N, K, row_offset).double().t()
+    torch.cuda.synchronize()
+    assert bool((buf[M * N:] == 7.0).all())
+    for m in range(M):
+        err = float((y[m] - ref[m]).norm() / ref[m].norm())
+        print(f"gemv wtype={wtype} M={M} N={N} K={K} token {m}: rel_l2={err:.2e}")
+        assert err < 1e-6
+
+
+@pytest.mark.parametrize("wtype", [8, 12])
+def test_gemv_nonfinite_activations(dev, wtype):
+    """An infinite or NaN activation gives the products of the dequantized
+    weight (Inf of each weight's sign, NaN at a zero weight) for its token and
+    leaves the others as they are."""
+    import torch
+    from llmr_amd import ops
+    M, N, K = 3, 70, 512
+    w = _weights(dev, wtype, N, K, 280 + wtype)
+    x = torch.randn(M, K, generator=torch.Generator(device="cpu").manual_seed(9))
+    good = ops.batch_matmul(w, wtype, x.to(dev), N).cpu()
+    x[0, 100] = float("inf")
+    x[2, 400] = float("nan")
+    y = ops.batch_matmul(w, wtype, x.to(dev), N).cpu()
+    col = ops.dequant(w, wtype, N, K).cpu()[:, 100]
+    want = torch.where(col == 0, torch.tensor(float("nan")), torch.copysign(torch.tensor(float("inf")), col))
+    assert torch.equal(torch.nan_to_num(y[0], nan=7.0), torch.nan_to_num(want, nan=7.0))
+    assert bool(torch.isnan(y[2]).all())
+    assert rel_l2(y[1].numpy(), good[1].numpy()) < 1e-6
+
+
 @pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", CASES)
 def test_gemm_parity(orc, dev, wtype, M, N, K, xtype, row_offset):
     from llmr_amd import gguf, synth
