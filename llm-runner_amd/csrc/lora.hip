@@ -15,13 +15,10 @@
 // restatement: hop 1's sums as a 256-thread workgroup forms them (strided
 // partials, then the tree), hop 2's and the merge's in rank order.
 //
-// Work layout (MI355X): hop 1 gives each workgroup 4 tokens x 8 ranks per
-// pass (A is read once per 4 tokens instead of once per (token, rank) sum),
-// its k loop unrolled for loads in flight and a small LDS tree for several
-// workgroups per CU; hop 2 gives each workgroup 256 output features x 64
-// tokens, so B is read once per 64 tokens. Both are
-// bandwidth-bound: the dominant traffic is hop 2's read-modify-write of the
-// f32 output.
+// Work layout (MI355X): hop 1 gives each wave 4 tokens x 8 ranks (A is read
+// once per 4 tokens instead of once per (token, rank) sum) with the tree across
+// its lanes; hop 2 gives each workgroup 256 output features x 16 or 32 tokens.
+// Hop 2's read-modify-write of the f32 output is the dominant traffic.
 #include <hip/hip_runtime.h>
 
 #include "llmr_device.h"
@@ -102,6 +99,113 @@ __global__ void __launch_bounds__(256) lora_down_kernel(const float* __restrict_
             __syncthreads();  // red is rewritten by the next half
         }
     }
+}
+
+// The same sums, a wave per 4 tokens x 8 ranks with no LDS: lane l carries the
+// partial sums gi = 4 l .. 4 l + 3 (16-byte loads of A and x), and the tree
+// s = 128 .. 4 runs across lanes l + 32, 16, .., 1, s = 2 and 1 in the lane. Each
+// cross-lane level adds two sums at once (the lanes with the level's bit clear
+// keep one, the others the other), so 32 sums cost 128 exchanges instead of
+// 768. What bounds it is A from L2 (rank x in_dim floats per 4 tokens); through
+// LDS with a barrier per tree level it was 55 us for 1536 x 3072 x 32, this is
+// 16. Needs 16-byte aligned A and x, in_dim % 4 == 0.
+constexpr uint32_t kWaveTokens = 4, kWaveRanks = 8;
+__device__ __forceinline__ float tree_pair(float a, float b, uint32_t lane, uint32_t bit) {
+    // lanes with `bit` clear: a[l] + a[l ^ bit]; set: b[l] + b[l ^ bit]
+    const bool up = (lane & bit) != 0u;
+    return (up ? b : a) + __shfl_xor(up ? a : b, (int)bit, 64);
+}
+template <uint32_t XT>
+__global__ void __launch_bounds__(256, 2) lora_down_wave_kernel(const float* __restrict__ A, const void* __restrict__ X,
+                                                                 float* __restrict__ scratch, uint32_t rank,
+                                                                 uint32_t in_dim, uint32_t seq_len, uint32_t rank_groups) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t id = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t r0 = id % rank_groups * kWaveRanks, s0 = id / rank_groups * kWaveTokens;
+    if (s0 >= seq_len) return;
+    f32x4 acc[kWaveTokens][kWaveRanks];
+#pragma unroll
+    for (uint32_t t = 0; t < kWaveTokens; t++)
+#pragma unroll
+        for (uint32_t r = 0; r < kWaveRanks; r++) acc[t][r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // rows past seq_len or rank read the last row and are not stored
+    struct In {
+        f32x4 x[kWaveTokens], a[kWaveRanks];
+    };
+    auto load = [&](uint32_t k) __attribute__((always_inline)) {
+        In v;
+#pragma unroll
+        for (uint32_t t = 0; t < kWaveTokens; t++) {
+            const uint64_t e = (uint64_t)min(s0 + t, seq_len - 1u) * in_dim + k;
+            if constexpr (XT == kGgmlF32) {
+                v.x[t] = *(const f32x4*)((const float*)X + e);
+            } else {
+                const u32x2 w = *(const u32x2*)((const uint16_t*)X + e);
+                const uint32_t lo = w.x, hi = w.y;
+                if constexpr (XT == kGgmlBF16) {
+                    v.x[t] = f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u),
+                                   __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)};
+                } else {
+                    const f16x2 p = __builtin_bit_cast(f16x2, lo), q = __builtin_bit_cast(f16x2, hi);
+                    v.x[t] = f32x4{(float)p.x, (float)p.y, (float)q.x, (float)q.y};
+                }
+            }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < kWaveRanks; r++)
+            v.a[r] = *(const f32x4*)(A + (uint64_t)min(r0 + r, rank - 1u) * in_dim + k);
+        return v;
+    };
+    const uint32_t k0 = 4u * lane;
+    if (k0 < in_dim) {
+        In cur = load(k0);
+        for (uint32_t k = k0; k < in_dim; k += 256u) {
+            In nxt;
+            const bool more = k + 256u < in_dim;
+            if (more) nxt = load(k + 256u);
+#pragma unroll
+            for (uint32_t t = 0; t < kWaveTokens; t++)
+#pragma unroll
+                for (uint32_t r = 0; r < kWaveRanks; r++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++)
+                        acc[t][r][c] = __builtin_fmaf(cur.a[r][c], cur.x[t][c], acc[t][r][c]);
+            if (more) cur = nxt;
+        }
+    }
+    // sum q = 8 t + r; after the five pairing levels lane l holds sum 16 b5 +
+    // 8 b4 + 4 b3 + 2 b2 + b1 of its bits, after the sixth both lanes of a pair
+    f32x4 v16[16], v8[8], v4[4], v2[2], v1;
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[q / 8][q % 8][c]),
+                                                            __float_as_uint(acc[2 + q / 8][q % 8][c]), false, false);
+            v16[q][c] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        }
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v16[q][c]), __float_as_uint(v16[8 + q][c]),
+                                                            false, false);
+            v8[q][c] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) v4[q][c] = tree_pair(v8[q][c], v8[4 + q][c], lane, 8u);
+#pragma unroll
+        for (int q = 0; q < 2; q++) v2[q][c] = tree_pair(v4[q][c], v4[2 + q][c], lane, 4u);
+        v1[c] = tree_pair(v2[0][c], v2[1][c], lane, 2u);
+        v1[c] += __shfl_xor(v1[c], 1, 64);
+    }
+    const float sum = (v1.x + v1.z) + (v1.y + v1.w);
+    const uint32_t q = (lane >> 5 & 1u) * 16u + (lane >> 4 & 1u) * 8u + (lane >> 3 & 1u) * 4u + (lane >> 2 & 1u) * 2u +
+                       (lane >> 1 & 1u);
+    const uint32_t t = s0 + q / kWaveRanks, r = r0 + q % kWaveRanks;
+    if ((lane & 1u) == 0u && t < seq_len && r < rank) scratch[(uint64_t)t * rank + r] = sum;
 }
 
 // out[s * out_dim + row_offset + o] += scale * sum_r B[(wro + o) * rank + r] *
@@ -201,59 +305,71 @@ __global__ void __launch_bounds__(256) lora_up_kernel(const float* __restrict__ 
             if (h * 256u + gi < no && t < nt) ybase[(uint64_t)t * out_dim + h * 256u] = yv[h][t] + scale * acc[h][t];
 }
 
-// Hop 2 for ranks up to RK (8, 16 or 32; rank % 4 == 0): thread gi owns
-// output column o0 + gi, whose B row (rank floats) stays in registers for
-// the workgroup's kUpRegSpan tokens; the tokens' scratch rows go through LDS
-// in blocks of kUpRegTokens (broadcast reads), the block's output values are
-// read before its sums. Same arithmetic as lora_up_kernel: the sum over
-// ranks in rank order from 0, then y + scale * sum. Its LDS footprint is
-// 2 KiB (lora_up_kernel's 70 KiB held two workgroups per CU), so enough
-// workgroups share a CU to overlap their output reads and writes with the
-// FMAs of others.
-constexpr uint32_t kUpRegTokens = 16;
-constexpr uint32_t kUpRegSpan = 128;
-template <uint32_t RK>
+// Hop 2 for ranks 4, 8, .. 32 (R) and multiples of 32 (R = 32, chunks of it):
+// thread gi owns output column o0 + gi, whose B row stays in registers (a chunk
+// at a time) for the workgroup's T tokens; their scratch rows are the same for
+// the whole wave, so they come as scalar loads and are scalar operands of the
+// FMAs, and all the output values are requested before the first sum (rows past
+// seq_len read zero and are not stored: the buffer ends there). Same arithmetic
+// as lora_up_kernel: the sum over ranks in rank order from 0, then y + scale *
+// sum. What bounds it is the output's read and write. With the scratch rows
+// through LDS (a broadcast read per 4 FMAs is as slow as they are), 16 tokens at
+// a time and 128 a workgroup, 1536 x 9216 x 32 took 59 us (1.9 TB/s), 4608 x
+// 21504 x 32 240 us; this takes 32 and 190 (4.2 TB/s). B through LDS instead of
+// each lane reading its own row: 15 us slower. Both hops of 1536 x 9216 x 3072:
+// 110 -> 49 us at rank 32, 191 -> 78 at rank 64.
+template <uint32_t R, uint32_t T, bool CHUNKS>
 __global__ void __launch_bounds__(256) lora_up_reg_kernel(const float* __restrict__ B,
                                                            const float* __restrict__ scratch, float* __restrict__ out,
                                                            uint32_t rank, uint32_t out_dim, uint32_t seq_len,
                                                            float scale, uint32_t row_offset, uint32_t weight_row_offset,
                                                            uint32_t b_rows) {
-    __shared__ __attribute__((aligned(16))) float sc[kUpRegTokens][RK];
-    const uint32_t gi = threadIdx.x, o = blockIdx.x * 256u + gi;
-    const uint32_t s_begin = blockIdx.y * kUpRegSpan, s_end = min(seq_len, s_begin + kUpRegSpan);
-    const bool live = o < b_rows;
-    const uint32_t q = rank / 4u;  // 16-byte pieces of a rank row
-    float bv[RK];
+    typedef __attribute__((address_space(4))) const float cfloat;
+    const uint32_t o = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t s0 = blockIdx.y * T, nt = min(T, seq_len - s0);
+    const rsrc_t yr = make_rsrc(out + (uint64_t)s0 * out_dim, (uint64_t)nt * out_dim * 4u);
+    const uint32_t yo = o < b_rows ? (row_offset + o) * 4u : 0x80000000u;
+    float yv[T];
 #pragma unroll
-    for (uint32_t r = 0; r < RK; r += 4) {
-        const f32x4 v = live && r < rank ? *(const f32x4*)(B + (uint64_t)(weight_row_offset + o) * rank + r)
-                                         : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        bv[r] = v.x;
-        bv[r + 1] = v.y;
-        bv[r + 2] = v.z;
-        bv[r + 3] = v.w;
-    }
-    float* const ycol = out + row_offset + o;
-    for (uint32_t s0 = s_begin; s0 < s_end; s0 += kUpRegTokens) {
-        const uint32_t nt = min(kUpRegTokens, s_end - s0);
-        for (uint32_t i = gi; i < nt * q; i += 256u) {
-            const uint32_t t = i / q, r = 4u * (i % q);
-            *(f32x4*)&sc[t][r] = *(const f32x4*)(scratch + (uint64_t)(s0 + t) * rank + r);
+    for (uint32_t t = 0; t < T; t++)
+        yv[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yr, yo, t * out_dim * 4u, 0));
+    const uint32_t ld = CHUNKS ? rank : R;
+    const float* const brow = B + (uint64_t)(weight_row_offset + min(o, b_rows - 1u)) * ld;
+    float bv[R];
+    auto load_b = [&](uint32_t c) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t r = 0; r < R; r += 4) {
+            const f32x4 v = *(const f32x4*)(brow + c * R + r);
+            bv[r] = v.x;
+            bv[r + 1] = v.y;
+            bv[r + 2] = v.z;
+            bv[r + 3] = v.w;
         }
-        __syncthreads();
-        float yv[kUpRegTokens];
+    };
+    auto sum = [&](uint32_t t, uint32_t c, float a) __attribute__((always_inline)) {
+        cfloat* const sc = (cfloat*)(scratch + (uint64_t)min(s0 + t, seq_len - 1u) * ld + c * R);
 #pragma unroll
-        for (uint32_t t = 0; t < kUpRegTokens; t++)
-            yv[t] = live && t < nt ? ycol[(uint64_t)(s0 + t) * out_dim] : 0.0f;
+        for (uint32_t r = 0; r < R; r++) a = __builtin_fmaf(bv[r], sc[r], a);
+        return a;
+    };
+    auto store = [&](uint32_t t, float a) __attribute__((always_inline)) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(yv[t] + scale * a), yr, yo, t * out_dim * 4u, 0);
+    };
+    if constexpr (!CHUNKS) {
+        load_b(0);
 #pragma unroll
-        for (uint32_t t = 0; t < kUpRegTokens; t++) {
-            float a = 0.0f;
+        for (uint32_t t = 0; t < T; t++) store(t, sum(t, 0, 0.0f));
+    } else {
+        float a[T];
 #pragma unroll
-            for (uint32_t r = 0; r < RK; r++)
-                if (r < rank) a = __builtin_fmaf(bv[r], sc[t][r], a);
-            if (live && t < nt) ycol[(uint64_t)(s0 + t) * out_dim] = yv[t] + scale * a;
+        for (uint32_t t = 0; t < T; t++) a[t] = 0.0f;
+        for (uint32_t c = 0; c < rank / R; c++) {
+            load_b(c);
+#pragma unroll
+            for (uint32_t t = 0; t < T; t++) a[t] = sum(t, c, a[t]);
         }
-        __syncthreads();  // sc is refilled by the next block
+#pragma unroll
+        for (uint32_t t = 0; t < T; t++) store(t, a[t]);
     }
 }
 
@@ -303,31 +419,58 @@ hipError_t launch_lora_correction(const float* A, const float* B, uint32_t rank,
                                   uint32_t seq_len, uint32_t b_rows, uint32_t row_offset, uint32_t weight_row_offset,
                                   hipStream_t st) {
     if (rank == 0 || seq_len == 0) return hipSuccess;
-    const dim3 gd((seq_len + kDownTokens - 1) / kDownTokens);
+    const bool wide = in_dim % 4u == 0u && ((uintptr_t)A & 15u) == 0u && ((uintptr_t)x & 15u) == 0u;
+    auto down = [&](auto xt) {
+        constexpr uint32_t XT = decltype(xt)::value;
+        if (wide) {
+            const uint32_t rg = (rank + kWaveRanks - 1u) / kWaveRanks;
+            const uint64_t waves = (uint64_t)rg * ((seq_len + kWaveTokens - 1u) / kWaveTokens);
+            hipLaunchKernelGGL(lora_down_wave_kernel<XT>, dim3((uint32_t)((waves + 3u) / 4u)), dim3(256), 0, st, A, x,
+                               scratch, rank, in_dim, seq_len, rg);
+        } else {
+            hipLaunchKernelGGL(lora_down_kernel<XT>, dim3((seq_len + kDownTokens - 1) / kDownTokens), dim3(256), 0, st,
+                               A, x, scratch, rank, in_dim, seq_len);
+        }
+    };
     switch (xtype) {
-        case kGgmlF32:
-            hipLaunchKernelGGL(lora_down_kernel<kGgmlF32>, gd, dim3(256), 0, st, A, x, scratch, rank, in_dim, seq_len);
-            break;
-        case kGgmlF16:
-            hipLaunchKernelGGL(lora_down_kernel<kGgmlF16>, gd, dim3(256), 0, st, A, x, scratch, rank, in_dim, seq_len);
-            break;
-        default:
-            hipLaunchKernelGGL(lora_down_kernel<kGgmlBF16>, gd, dim3(256), 0, st, A, x, scratch, rank, in_dim,
-                               seq_len);
-            break;
+        case kGgmlF32: down(std::integral_constant<uint32_t, kGgmlF32>{}); break;
+        case kGgmlF16: down(std::integral_constant<uint32_t, kGgmlF16>{}); break;
+        default: down(std::integral_constant<uint32_t, kGgmlBF16>{}); break;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || b_rows == 0) return e;
-    if (rank <= 32u && rank % 4u == 0u) {
-        const dim3 gr((b_rows + 255u) / 256u, (seq_len + kUpRegSpan - 1) / kUpRegSpan);
-        auto go = [&](auto rk) {
-            hipLaunchKernelGGL(lora_up_reg_kernel<decltype(rk)::value>, gr, dim3(256), 0, st, B,
-                               (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
-                               weight_row_offset, b_rows);
+    // (32 rows of the output within a buffer's 31-bit offsets)
+    if (rank % 4u == 0u && (rank <= 32u || rank % 32u == 0u) && (uint64_t)out_dim * 32u * 4u < (1ull << 31)) {
+        // 32 tokens a workgroup (B read half as often) where that still gives
+        // every CU 16 workgroups: 4608 x 21504 x 32 both hops 235 against 257 us
+        // with 16, 1536 x 9216 x 32 52 against 49, 300 x 3072 x 16 23 against 17
+        const uint32_t cols = (b_rows + 255u) / 256u;
+        const bool wide_t = (uint64_t)cols * ((seq_len + 31u) / 32u) >= 4096u;
+        auto go = [&](auto r) {
+            constexpr uint32_t R = decltype(r)::value;
+            if (rank > R)
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, true>), dim3(cols, (seq_len + 15u) / 16u), dim3(256), 0,
+                                   st, B, (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
+                                   weight_row_offset, b_rows);
+            else if (wide_t)
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 32, false>), dim3(cols, (seq_len + 31u) / 32u), dim3(256), 0, st, B,
+                                   (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
+                                   weight_row_offset, b_rows);
+            else
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, false>), dim3(cols, (seq_len + 15u) / 16u), dim3(256), 0, st, B,
+                                   (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
+                                   weight_row_offset, b_rows);
         };
-        if (rank <= 8u) go(std::integral_constant<uint32_t, 8>{});
-        else if (rank <= 16u) go(std::integral_constant<uint32_t, 16>{});
-        else go(std::integral_constant<uint32_t, 32>{});
+        switch (rank) {
+            case 4: go(std::integral_constant<uint32_t, 4>{}); break;
+            case 8: go(std::integral_constant<uint32_t, 8>{}); break;
+            case 12: go(std::integral_constant<uint32_t, 12>{}); break;
+            case 16: go(std::integral_constant<uint32_t, 16>{}); break;
+            case 20: go(std::integral_constant<uint32_t, 20>{}); break;
+            case 24: go(std::integral_constant<uint32_t, 24>{}); break;
+            case 28: go(std::integral_constant<uint32_t, 28>{}); break;
+            default: go(std::integral_constant<uint32_t, 32>{}); break;
+        }
         return hipGetLastError();
     }
     const dim3 gu((b_rows + 511u) / 512u, (seq_len + kUpTokens - 1) / kUpTokens);

@@ -55,6 +55,35 @@ def test_lora_correction_bit_exact(orc, dev, seq, in_dim, rank, out_dim, b_rows,
     np.testing.assert_array_equal(y.cpu().numpy(), y_ref)
 
 
+@pytest.mark.parametrize("seq,in_dim,rank,out_dim,xtype,shift", [
+    (35, 1028, 12, 300, 30, 0),   # part-filled token and rank groups, one lane's last pass
+    (6, 254, 5, 64, 0, 0),        # in_dim % 4 != 0: the LDS form of hop 1
+    (9, 512, 8, 264, 1, 1),       # activations one element past 16 bytes: the same
+    (33, 256, 32, 257, 30, 0),    # one token and one column past a hop-2 workgroup
+    (18, 260, 96, 300, 0, 0),     # three chunks of 32 ranks
+    (1030, 64, 4, 33000, 30, 0),  # enough workgroups for 32 tokens each
+])
+def test_lora_correction_edges_bit_exact(orc, dev, seq, in_dim, rank, out_dim, xtype, shift):
+    """The correction at the edges of its token, rank and column groups and at
+    the alignments that take the narrow loads, bit for bit."""
+    import torch
+    from llmr_amd import ops
+    r = np.random.default_rng(seq * 100 + rank)
+    A, B, lora = _lora(dev, r, rank, in_dim, out_dim, 0.7)
+    x = r.standard_normal((seq, in_dim)).astype(np.float32)
+    flat = _act(np.concatenate([np.zeros(shift, np.float32), x.ravel()]), xtype, dev)
+    xt = flat[shift:].view(seq, in_dim)
+    y0 = r.standard_normal((seq, out_dim)).astype(np.float32)
+    y = torch.from_numpy(y0).to(dev)
+    scratch = torch.empty(seq * rank, device=dev)
+    ops.dispatch_lora_correction(ops.default_graph(), lora, scratch, ops.Tensor.from_torch(xt),
+                                 ops.Tensor.from_torch(y), in_dim, out_dim, seq)
+    torch.cuda.synchronize()
+    s_ref = orc.lora_down(A, xt.float().cpu().numpy())
+    np.testing.assert_array_equal(scratch.cpu().numpy().reshape(seq, rank), s_ref)
+    np.testing.assert_array_equal(y.cpu().numpy(), orc.lora_up(B, s_ref, y0, 0.7))
+
+
 def test_batch_matmul_with_lora_equals_base_plus_correction(orc, dev):
     """dispatch_batch_matmul with an adapter = the plain GEMM, then the
     correction on its output (dit.c3:1299-1300), at the Flux img_attn.qkv K
