@@ -1,7 +1,7 @@
-// gemm_few.hip - dequant-GEMM for few tokens (M <= 256) with enough output
-// features to give at least every other CU a 32 x 96 tile: batch_matmul_q8 /
+// gemm_few.hip - dequant-GEMM for few tokens (M <= 512): batch_matmul_q8 /
 // batch_matmul_q4k (llm.slang:1639-1767, :2277-2365), e.g. the single Q8_0
-// linear of 256 tokens x 3072 -> 3072 with f32 activations.
+// linear of 256 tokens x 3072 -> 3072 with f32 activations, or the text
+// projection of a prompt.
 //
 //   Y[m, n] = sum_k X[m, k] * W[row_offset + n, k]     (f32 out, row stride N)
 //
@@ -14,9 +14,12 @@
 // per CU at K = 3072). Splitting K across CUs would cut that by sqrt(splits)
 // but adds the partial sums' round trip through memory and a second launch.
 //
-// Workgroup = 8 waves (two per SIMD) over one 32-token x 96-feature tile;
-// wave w takes the K stages w, w + 8, w + 16, ... (64 k each) and keeps the
-// whole tile in three 32x32x16 MFMA accumulators; at the end the eight
+// Workgroup = 8 waves (two per SIMD) over one tile of 32 tokens x FF features,
+// 96 or 32 (plan::few_features holds the rule and the figures): 96 where a
+// launch has whole rounds of them, 32 where it has not, as three 32-feature
+// workgroups share a CU (50 KiB of LDS each) and hide each other's latency.
+// Wave w takes the K stages w, w + 8, w + 16, ... (64 k each) and keeps the
+// whole tile in FF / 32 32x32x16 MFMA accumulators; at the end the eight
 // partial tiles meet in LDS and are summed in wave order (deterministic).
 // (Twelve waves, with half again as many loads in flight per CU, measured
 // slower: the load path's throughput is the bound, not its latency.)
@@ -55,10 +58,9 @@ namespace llmr {
 
 namespace {
 
-constexpr uint32_t kFT = plan::kFewTokens, kFF = plan::kFewFeatures, kFB = kFF / 32u;  // 3 feature blocks
+constexpr uint32_t kFT = plan::kFewTokens;
 constexpr uint32_t kFewWaves = 8;  // two per SIMD
-constexpr uint32_t kRedLd = kFF + 4u;  // floats per LDS row of a partial tile (16-byte pad)
-static_assert(kFT == 32 && kFF % 32 == 0, "one 32-token block, whole 32-feature blocks");
+static_assert(kFT == 32, "one 32-token block");
 
 // A lane's packed weight bytes of one stage and feature block, as read back
 // from the wave's LDS region.
@@ -101,9 +103,9 @@ struct FewW<kGgmlQ4K> {
 // stage (no read crosses them); lane l of Q4_K weight load j holds row
 // 16 j + l / 4, piece l % 4 (0 the superblock header, 1-2 the quarter's
 // quants, 3 nothing).
-template <uint32_t WT, uint32_t XT>
+template <uint32_t WT, uint32_t XT, uint32_t FF>
 struct FewLoads {
-    static constexpr uint32_t kXi = XT == kGgmlF32 ? 8u : 4u, kWj = WT == kGgmlQ8_0 ? 8u : 6u;
+    static constexpr uint32_t kXi = XT == kGgmlF32 ? 8u : 4u, kWj = WT == kGgmlQ8_0 ? (FF + 11u) / 12u : FF / 16u;
     u32x4 x[kXi], w[kWj];
     __device__ __forceinline__ void load(rsrc_t xr, rsrc_t wr, uint32_t m_row, uint32_t K, uint64_t rb,
                                          uint32_t s, uint32_t lane) {
@@ -121,7 +123,8 @@ struct FewLoads {
             const uint32_t po = p < 4u ? 16u * p : 52u;
 #pragma unroll
             for (uint32_t j = 0; j < kWj; j++)
-                w[j] = bload16(wr, lane < 60u ? (uint32_t)((12u * j + q) * rb) + po : 0x80000000u, 68u * s);
+                w[j] = bload16(wr, lane < 60u && 12u * j + q < FF ? (uint32_t)((12u * j + q) * rb) + po : 0x80000000u,
+                               68u * s);
         } else {
             const uint32_t p = lane & 3u, sh = (s >> 2) * 144u;
             const uint32_t off = p == 0 ? sh : p < 3 ? sh + 16u + 32u * (s & 3u) + 16u * (p - 1u) : 0x80000000u;
@@ -155,12 +158,12 @@ struct FewLoads {
         constexpr uint32_t kRow = FewW<WT>::kRow;
         if constexpr (WT == kGgmlQ8_0) {
             const uint32_t q = lane / 5u, p = lane - 5u * q;
-            const bool piece = lane < 60u && p < 4u, last = lane < 60u && p == 4u;
 #pragma unroll
             for (uint32_t j = 0; j < kWj; j++) {
+                const bool live = lane < 60u && 12u * j + q < FF;
                 const uint32_t row = (12u * j + q) * kRow;
-                *(u32x4*)(ws + (piece ? row + 16u * p : kFF * kRow)) = w[j];
-                *(uint32_t*)(ws + (last ? row + 64u : kFF * kRow)) = w[j].w;
+                *(u32x4*)(ws + (live && p < 4u ? row + 16u * p : FF * kRow)) = w[j];
+                *(uint32_t*)(ws + (live && p == 4u ? row + 64u : FF * kRow)) = w[j].w;
             }
         } else {
 #pragma unroll
@@ -230,13 +233,15 @@ struct FewWop<kGgmlQ4K, OT> {
     }
 };
 
-template <uint32_t WT, uint32_t XT>
-__global__ void __launch_bounds__(kFewWaves * 64u, 1)
+template <uint32_t WT, uint32_t XT, uint32_t FF>
+__global__ void __launch_bounds__(kFewWaves * 64u, FF == 96u ? 1 : 4)
     gemm_q_few(const uint8_t* __restrict__ W, const void* __restrict__ X, float* __restrict__ Y, uint32_t N,
                uint32_t K, uint32_t M, uint32_t row_offset, uint32_t tiles_m, uint32_t tiles_n) {
     constexpr uint32_t OT = (XT == kGgmlBF16 || (XT == kGgmlF32 && WT == kGgmlQ4K)) ? kGgmlBF16 : kGgmlF16;
     // per wave: its stage's 16-bit activations (32 x 128 bytes) and packed
     // weight rows; after the loop, the waves' partial tiles
+    constexpr uint32_t kFF = FF, kFB = FF / 32u;
+    constexpr uint32_t kRedLd = kFF + 4u;  // floats per LDS row of a partial tile (16-byte pad)
     constexpr uint32_t kXs = kFT * 128u, kWs = kFF * FewW<WT>::kRow + 16u, kWave = kXs + kWs;  // + a pad dword
     constexpr uint32_t kRed = kFewWaves * kFT * kRedLd * 4u;
     __shared__ __attribute__((aligned(16))) uint8_t lds[kFewWaves * kWave > kRed ? kFewWaves * kWave : kRed];
@@ -275,7 +280,7 @@ __global__ void __launch_bounds__(kFewWaves * 64u, 1)
     // in vector registers, they made every buffer load a loop over the
     // lanes' values.
     const uint32_t n = S > wave ? (S - wave + kFewWaves - 1u) / kFewWaves : 0u;
-    FewLoads<WT, XT> ld;
+    FewLoads<WT, XT, FF> ld;
     auto load = [&](uint32_t i) {
         const bool live = i < n;
         const uint32_t s = __builtin_amdgcn_readfirstlane(live ? wave + kFewWaves * i : 0u);
@@ -341,22 +346,26 @@ __global__ void __launch_bounds__(kFewWaves * 64u, 1)
 }  // namespace
 
 hipError_t launch_gemm_few(const void* w, uint32_t wtype, const void* x, uint32_t xtype, float* y, uint32_t N,
-                           uint32_t K, uint32_t M, uint32_t row_offset, hipStream_t st) {
-    if (M == 0 || M > plan::kFewMaxTokens || K % kBK || K == 0) return hipErrorInvalidValue;
-    const uint32_t tiles_m = (M + kFT - 1) / kFT, tiles_n = (N + kFF - 1) / kFF;
+                           uint32_t K, uint32_t M, uint32_t row_offset, uint32_t features, hipStream_t st) {
+    if (M == 0 || M > plan::kFewMaxTokens || K % kBK || K == 0 || (features != 32u && features != 96u))
+        return hipErrorInvalidValue;
+    const uint32_t tiles_m = (M + kFT - 1) / kFT, tiles_n = (N + features - 1) / features;
     const dim3 grid(tiles_m * tiles_n), block(kFewWaves * 64u);
-    auto go = [&](auto kern) {
+    auto go = [&](auto wt, auto xt) {
+        constexpr uint32_t WT = decltype(wt)::value, XT = decltype(xt)::value;
+        auto kern = features == 96u ? gemm_q_few<WT, XT, 96> : gemm_q_few<WT, XT, 32>;
         hipLaunchKernelGGL(kern, grid, block, 0, st, (const uint8_t*)w, x, y, N, K, M, row_offset, tiles_m, tiles_n);
     };
-    if (wtype == kGgmlQ8_0) {
-        if (xtype == kGgmlF32) go(gemm_q_few<kGgmlQ8_0, kGgmlF32>);
-        else if (xtype == kGgmlF16) go(gemm_q_few<kGgmlQ8_0, kGgmlF16>);
-        else go(gemm_q_few<kGgmlQ8_0, kGgmlBF16>);
-    } else {
-        if (xtype == kGgmlF32) go(gemm_q_few<kGgmlQ4K, kGgmlF32>);
-        else if (xtype == kGgmlF16) go(gemm_q_few<kGgmlQ4K, kGgmlF16>);
-        else go(gemm_q_few<kGgmlQ4K, kGgmlBF16>);
-    }
+    using F32 = std::integral_constant<uint32_t, kGgmlF32>;
+    using F16 = std::integral_constant<uint32_t, kGgmlF16>;
+    using BF16 = std::integral_constant<uint32_t, kGgmlBF16>;
+    auto by_x = [&](auto wt) {
+        if (xtype == kGgmlF32) go(wt, F32{});
+        else if (xtype == kGgmlF16) go(wt, F16{});
+        else go(wt, BF16{});
+    };
+    if (wtype == kGgmlQ8_0) by_x(std::integral_constant<uint32_t, kGgmlQ8_0>{});
+    else by_x(std::integral_constant<uint32_t, kGgmlQ4K>{});
     return hipGetLastError();
 }
 

@@ -32,8 +32,9 @@ constexpr uint32_t kW16MinTokens = 2048;
 // workgroups per CU, with at least kSplitMinStages stages per split.
 constexpr uint32_t kSplitWgsPerCu = 2, kSplitMinStages = 4;
 // The few-token kernel (gemm_few.hip): a workgroup owns 32 tokens x
-// kFewFeatures features over the whole K.
-constexpr uint32_t kFewTokens = 32, kFewFeatures = 96, kFewMaxTokens = 256;
+// kFewFeatures or kFewNarrow features over the whole K.
+constexpr uint32_t kFewTokens = 32, kFewFeatures = 96, kFewNarrow = 32, kFewMaxTokens = 512;
+constexpr uint32_t kSkinnyMaxTokens = 256;
 
 inline uint64_t row_bytes_of(uint32_t wtype, uint32_t K) {
     return wtype == kQ8_0 ? (uint64_t)(K / 32) * 34 : (uint64_t)(K / 256) * 144;
@@ -107,16 +108,50 @@ inline TilePlan plan_tiles(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, i
     return t;
 }
 
-// Whether the few-token kernel takes M x N x K: at most kFewMaxTokens
-// tokens, whole stages, and at least half the CUs' worth of 32 x 96 tiles
-// (fewer: the skinny kernel, which splits K to fill the CUs).
-inline bool few_fits(uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+// Whether the few-token kernel can take M x N x K: at most kFewMaxTokens
+// tokens, whole stages, 32-bit buffer offsets.
+inline bool few_fits(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M) {
     if (M == 0 || M > kFewMaxTokens || K % kStageK || K == 0) return false;
-    // 32-bit buffer offsets of the f32 activation rows and of the weight
-    // rows past N that a last tile addresses
-    if ((uint64_t)(M + kFewTokens) * K * 4u >= (1ull << 31)) return false;
-    const uint64_t tiles = (uint64_t)((M + kFewTokens - 1) / kFewTokens) * ((N + kFewFeatures - 1) / kFewFeatures);
-    return 2 * tiles >= (uint64_t)num_cus;
+    // the f32 activation rows and the weight rows past N that a last tile addresses
+    return (uint64_t)(M + kFewTokens) * K * 4u < (1ull << 31) &&
+           (uint64_t)(N + kFewFeatures) * row_bytes_of(wtype, K) < (1ull << 32);
+}
+
+// The few-token kernel's tile width up to kSkinnyMaxTokens tokens (0: the
+// skinny kernel). 96-feature tiles read the fewest bytes per CU but hold it
+// alone (102 KiB of LDS), so their cost is whole rounds over the CUs;
+// 32-feature tiles share a CU three at a time and cost by their number (f32
+// activations, re-read by every tile, more so past K = 8192), plus a fixed part
+// of a round. In units of a 32-feature tile; measured on 256 CUs, 96 -> 32
+// features: 77 x 9216 x 3072 Q4_K bf16 27.2 -> 19.2 us, 200 x 3840 x 3840 31.0 -> 22.7,
+// 64 x 9216 x 3072 15.2 / 15.7, 200 x 3072 x 3072 15.2 / 15.4, Q8_0 f32 15.7 / 21.0.
+// Below half the CUs' worth of 96-feature tiles the skinny kernel (packed
+// activations, K splits, partial sums: three launches) is the better one only
+// for f32 activations with long rows (77 x 3072 x 12288 43 against 48 us); the
+// 32-feature tiles take 77 x 3072 x 4096 Q4_K bf16 in 12.8 us against 19.5, 32 x
+// 3840 x 3840 8.7 against 19.6, 5 x 9216 x 3072 10.5 against 43.
+inline uint32_t few_features(uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+    const uint64_t tm = (M + kFewTokens - 1) / kFewTokens, c = (uint64_t)num_cus;
+    const uint64_t wide = tm * ((N + kFewFeatures - 1) / kFewFeatures), narrow = tm * ((N + kFewNarrow - 1) / kFewNarrow);
+    const bool long_f32 = xtype == kF32 && K > 8192;
+    if (2 * wide < c) return long_f32 && N >= 512 && N % 4 == 0 ? 0u : kFewNarrow;
+    const double f = long_f32 ? 1.6 : xtype == kF32 ? 1.3 : 1.03;
+    return f * narrow + 0.7 * c < 3.0 * c * ((wide + c - 1) / c) ? kFewNarrow : kFewFeatures;
+}
+// Time in us of the 32-feature tiles past kSkinnyMaxTokens tokens (300 x 3072
+// x 3072 Q4_K bf16: 960 tiles), for the choice against plan_split and the tiled kernel.
+inline double few_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+    const double tiles = (double)((M + kFewTokens - 1) / kFewTokens) * ((N + kFewNarrow - 1) / kFewNarrow);
+    return 5.0 + (xtype == kF32 ? 7.0 : wtype == kQ8_0 ? 4.6 : 4.3) * K / 3072.0 * tiles / num_cus;
+}
+// Time in us of the tiled kernel: two of its workgroups per CU run at full
+// speed, its 64 x 64 tiles four at a time (three with f32 activations).
+inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+    const TilePlan t = plan_tiles(wtype, N, K, M, num_cus);
+    const double wgs = (double)((M + t.bm - 1) / t.bm) * ((N + t.bm - 1) / t.bm) * t.splits, c = (double)num_cus;
+    const double rounds = wgs <= 2 * c ? 1.0 : wgs <= (xtype == kF32 ? 3 : 4) * c ? 1.8 : std::max(3.1, 0.55 * wgs / c);
+    const double per_k = (t.bm == 64 ? 1.0 : t.bm == 128 ? 2.8 : 8.0) * (wtype == kQ8_0 ? 0.0105 : 0.0090);
+    return 6.0 + rounds * ((double)K / t.splits) * per_k;
 }
 
 // Launches below kW16MinTokens tokens whose 256 x 256 tiles leave CUs idle in
@@ -127,8 +162,7 @@ inline bool few_fits(uint32_t N, uint32_t K, uint32_t M, int num_cus) {
 // x 3072-21504 features: a K stage of a tile takes 2.0 us on the 8-wave
 // kernel that also runs the splits (1.93 and 1.7 for Q8_0 and Q4_K where
 // tiles follow each other in the persistent kernels), a workgroup 8 us around
-// its stages, and the partial tiles are written and read at ~5 TB/s; the
-// 64 x 64 tiled kernel reaches 230 (Q8_0) and 300 TFLOP/s (Q4_K). Measured,
+// its stages, and the partial tiles are written and read at ~5 TB/s. Measured,
 // whole launch before -> after: 1101 x 3840 x 3840 Q8_0 (75 tiles x 3) 129 ->
 // 60 us, x 10240 348 -> 117; 520 x 9216 x 3072 Q4_K (108 x 2) 99 -> 60; 1536 x
 // 11520 x 3840 Q8_0 (256 whole tiles + 14 x 15) 236 -> 160; 2000 x 9216 x
@@ -142,31 +176,34 @@ constexpr uint32_t kSplitMax = 16;
 constexpr uint32_t kSplitTileMinStages = 16;
 struct SplitPlan {
     uint32_t full, splits;  // splits 1: no split
+    double us;              // of the launch, split or whole
 };
-inline SplitPlan plan_split(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, int num_cus, bool persistent) {
+inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus, bool persistent) {
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
     const uint32_t S = K / kStageK;
     const uint64_t full = tiles / num_cus * num_cus, rem = tiles - full;
-    SplitPlan p{(uint32_t)full, 1};
+    SplitPlan p{(uint32_t)full, 1, 0.0};
     const double whole = persistent
                              ? (double)((tiles + num_cus - 1) / num_cus) * S * (wtype == kQ8_0 ? 1.93 : 1.7) + 6.0
-                             : 2e-6 * M * N * K / (wtype == kQ8_0 ? 230.0 : 300.0) + 8.0;
+                             : tiled_us(wtype, xtype, N, K, M, num_cus);
+    p.us = whole;
     double best = 0.97 * whole;
     for (uint32_t s = 2; rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
         if (nonempty_splits(S, s) != s) continue;
         const double rounds = (double)((rem * s + num_cus - 1) / num_cus);
         const double us = (double)(full / num_cus) * (S * 2.0 + 8.0) + rounds * ((S + s - 1) / s * 2.0 + 8.0) + 3.0 +
                           (double)rem * kPartTile * (s + 1) / 5e6;
-        if (us < best) best = us, p.splits = s;
+        if (us < best) best = p.us = us, p.splits = s;
     }
     return p;
 }
 
 // How one GEMM runs.
 //  * few: the few-token kernel (f32 / 16-bit activations read in place, no
-//    workspace);
-//  * skinny: the few-token kernel with K splits (M <= 256 with too few 32 x
-//    96 tiles): workspace = [f32 activations as 16 bits | split partials];
+//    workspace), to kSkinnyMaxTokens tokens as few_features says, past them
+//    where few_us is the least;
+//  * skinny: the few-token kernel with K splits (where few_features is 0):
+//    workspace = [f32 activations as 16 bits | split partials];
 //  * persistent: the 256 x 256 persistent kernels (at least half the CUs'
 //    worth of tiles, whole stages, N % 4 == 0, 31-bit buffer offsets), f32
 //    activations rounded to operand_type() into the workspace first; from
@@ -185,6 +222,7 @@ struct GemmPlan {
     uint32_t xt;                  // activation type the kernel reads
     TilePlan tiles;               // the tiled kernel's tile and splits (not persistent)
     uint32_t splits;              // the skinny kernel's K splits
+    uint32_t few_features;        // few: features of a tile
     uint32_t split, split_full;   // split > 1: 256 x 256 tiles, those past split_full cut along K into `split`
     size_t x16_off, img_off, ws;  // workspace: [x16 | image] (persistent), [packed x | partials]
                                   // (skinny), split-K partials (tiled)
@@ -202,11 +240,15 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
     const bool offsets31 = (uint64_t)M * K * 2u < (1ull << 31) && (uint64_t)N * rb < (1ull << 31);
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
     p.persistent = K % kStageK == 0 && N % 4 == 0 && 2 * tiles >= (uint64_t)num_cus && offsets31;
-    if (!p.persistent && few_fits(N, K, M, num_cus) && (uint64_t)(N + kFewFeatures) * rb < (1ull << 32)) {
-        p.few = true;
-        return p;
+    const bool few_ok = !p.persistent && few_fits(wtype, N, K, M);
+    if (few_ok && M <= kSkinnyMaxTokens) {
+        p.few_features = few_features(xtype, N, K, M, num_cus);
+        if (p.few_features) {
+            p.few = true;
+            return p;
+        }
     }
-    if (!p.persistent && M <= 256 && K % kStageK == 0 && N % 4 == 0 && offsets31) {
+    if (!p.persistent && M <= kSkinnyMaxTokens && K % kStageK == 0 && N % 4 == 0 && offsets31) {
         // few tokens over few features: the skinny kernel (one workgroup per
         // CU: its LDS), K split so the launch fills the CUs in one round (at
         // least kSplitMinStages stages per split), as far as the partials fit
@@ -225,7 +267,12 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
         }
     }
     if (K % kStageK == 0 && N % 4 == 0 && offsets31 && M < kW16MinTokens) {
-        const SplitPlan sp = plan_split(wtype, N, K, M, num_cus, p.persistent);
+        const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent);
+        if (few_ok && few_us(wtype, xtype, N, K, M, num_cus) < 0.97 * sp.us) {
+            p.few = true;
+            p.few_features = kFewNarrow;
+            return p;
+        }
         const size_t x16 = xtype == kF32 ? align256((size_t)M * K * 2u) : 0u;
         const size_t ws = x16 + (size_t)(tiles - sp.full) * sp.splits * kPartTile;
         if (sp.splits > 1 && ws <= ws_limit) {

@@ -1569,7 +1569,7 @@ hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uin
         return wtype == kGgmlQ4K ? launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, st)
                                  : launch_gemv_q8(w, xtype, x, y, N, K, M, row_offset, st);
     const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit);
-    if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, st);
+    if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, pl.few_features, st);
     if (pl.skinny) return launch_gemm_skinny(w, wtype, x, xtype, y, N, K, M, row_offset, pl.splits, ws, st);
     if (pl.split > 1) return launch_split(w, wtype, x, xtype, y, N, K, M, row_offset, pl, num_cus, ws, st);
     if (!pl.persistent) {

@@ -1,6 +1,7 @@
 // Dequant-GEMM for few tokens (M <= 256): batch_matmul_q8 / batch_matmul_q4k
-// (llm.slang:1639-1767, :2277-2365) when the output has too few 256 x 256
-// tiles for the persistent kernels, e.g. a single linear over 256 tokens.
+// (llm.slang:1639-1767, :2277-2365) with f32 activations and rows past K = 8192,
+// where re-reading them per 32 features costs more than packing them once
+// (plan::few_features).
 //
 // Workgroup (n tile, split z) computes all M tokens x 64 features over the K
 // stages [z per, min(S, (z + 1) per)): the activations are read by N / 64

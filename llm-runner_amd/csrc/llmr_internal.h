@@ -126,10 +126,11 @@ hipError_t launch_splitk_reduce(const float* part, float* y, uint64_t mn, uint32
 // ranges. Workspace: f32 activations rounded to fp16 (skinny_x_bytes), then,
 // for splits > 1, the partials (splits * M * N floats) reduced into y.
 using plan::skinny_x_bytes;
-// The few-token GEMM with no K split (gemm_few.hip): M <= 256, K % 64 == 0,
-// f32 / f16 / bf16 activations read in place; no workspace.
+// The few-token GEMM with no K split (gemm_few.hip): M <= 512, K % 64 == 0,
+// f32 / f16 / bf16 activations read in place; no workspace. features: of a
+// workgroup's tile, 32 or 96.
 hipError_t launch_gemm_few(const void* w, uint32_t wtype, const void* x, uint32_t xtype, float* y, uint32_t N,
-                           uint32_t K, uint32_t M, uint32_t row_offset, hipStream_t st);
+                           uint32_t K, uint32_t M, uint32_t row_offset, uint32_t features, hipStream_t st);
 hipError_t launch_gemm_skinny(const void* w, uint32_t wtype, const void* x, uint32_t xtype, float* y, uint32_t N,
                               uint32_t K, uint32_t M, uint32_t row_offset, uint32_t splits, void* ws,
                               hipStream_t st);

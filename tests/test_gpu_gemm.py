@@ -304,6 +304,39 @@ def test_persistent_every_tile(dev, wtype, M, N, K, xtype, row_offset):
     assert torch.equal(y, y2)
 
 
+@pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", [
+    (12, 77, 3077, 1024, 30, 8),   # 32-feature tiles: a last one of 5, N % 4 != 0
+    (8, 33, 1000, 576, 0, 4),      # nine stages over eight waves, f32 as fp16
+    (8, 5, 36, 64, 1, 0),          # one stage: seven waves without
+    (12, 300, 1030, 768, 0, 0),    # past 256 tokens, f32 as bf16
+    (8, 512, 1024, 1088, 30, 2),   # the most tokens, 17 stages
+    (8, 250, 3072, 640, 30, 0),    # 96-feature tiles
+])
+def test_few_token_tiles(dev, wtype, M, N, K, xtype, row_offset):
+    """The few-token kernel's two tile widths at ragged tokens, features and
+    stage counts: every 32 x 32 block within the GEMM bar of the f32 product
+    of the dequantized weight (a wave's stages left out are off by 1 / sqrt(17)
+    or more), nothing written past the output."""
+    import torch
+    from llmr_amd import ops
+    w = _weights(dev, wtype, N + row_offset, K, 370 + wtype)
+    x = torch.randn(M, K, generator=torch.Generator(device="cpu").manual_seed(M + N + K))
+    x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
+    buf = torch.full((M * N + 64,), 7.0, device=dev)
+    y = buf[:M * N].view(M, N)
+    ops.batch_matmul(w, wtype, x, N, row_offset=row_offset, out=y)
+    ref = x.float() @ ops.dequant(w, wtype, N, K, row_offset).t()
+    torch.cuda.synchronize()
+    assert bool((buf[M * N:] == 7.0).all())
+    tm, tn = (M + 31) // 32, (N + 31) // 32
+    pad = (0, tn * 32 - N, 0, tm * 32 - M)
+    d2 = torch.nn.functional.pad((y - ref).double() ** 2, pad).view(tm, 32, tn, 32).sum((1, 3))
+    r2 = torch.nn.functional.pad(ref.double() ** 2, pad).view(tm, 32, tn, 32).sum((1, 3))
+    err = float((d2 / r2).sqrt().max())
+    print(f"few tokens wtype={wtype} M={M} N={N} K={K}: worst block rel_l2={err:.3e}")
+    assert err <= TOL
+
+
 # Launches below 2048 tokens whose last round of tiles is cut along K.
 SPLIT_TILE_CASES = [
     # (wtype, M, N, K, xtype, row_offset)
