@@ -574,19 +574,31 @@ __global__ void __launch_bounds__(256, 1) gemm_q_persist(const PersistArgs args)
         for (int i = 0; i < X_DMAS; i++) dma(xr, Xs, i, cx.s * 128u);
         advance(cx, nx);
     };
-    // A stage's loads in issue order: the W_LOADS weight loads of W(g+3),
-    // then the X_DMAS activation DMAs of X(g+2); part p of 4 issues the
-    // slice [p n / 4, (p+1) n / 4) of that list.
+    // A stage's loads in issue order: the X_DMAS activation DMAs of X(g+2),
+    // then the W_LOADS weight loads of W(g+3). The memory counter counts loads
+    // in order, so the stage's last barrier, which needs X(g+1), must not have
+    // the weight rows of W(g+3) (scattered, from HBM) in front of it: with the
+    // weights first and everything spread over the stage the SwiGLU of 1101 x
+    // 10240 x 3840 took 256 us, with the activations first and all of them in the
+    // stage's first k step 216. Q4_K, with fewer and lighter weight loads, gains
+    // most with the loads spread over the four parts (1536 x 9216 x 3072 105 ->
+    // 100 us, 1536 x 21504 x 3072 205 -> 203).
     constexpr int N_OPS = W_LOADS + X_DMAS;
+    constexpr bool EARLY = WT == kGgmlQ8_0;
+    // no part mixes the two kinds: the compiler may reorder loads within a part,
+    // and the barriers count on the order of the kinds
+    static_assert(EARLY || N_OPS / 4 == X_DMAS || N_OPS / 2 == X_DMAS || 3 * N_OPS / 4 == X_DMAS);
     auto issue_part = [&](auto PART, rsrc_t wr, uint32_t ws, rsrc_t xr, uint32_t xso, uint8_t* Xs,
                           WRow<WT, XT>& U) {
         constexpr int p = decltype(PART)::value;
-        static_for<p * N_OPS / 4, (p + 1) * N_OPS / 4>([&](auto I) {
+        constexpr int first = EARLY ? (p == 0 ? 0 : p == 1 ? X_DMAS : N_OPS) : p * N_OPS / 4;
+        constexpr int last = EARLY ? (p == 0 ? X_DMAS : N_OPS) : (p + 1) * N_OPS / 4;
+        static_for<first, last>([&](auto I) {
             constexpr int i = decltype(I)::value;
-            if constexpr (i < W_LOADS)
-                U.template load<i>(wr, wvoff, ws);
+            if constexpr (i < X_DMAS)
+                dma(xr, Xs, i, xso);
             else
-                dma(xr, Xs, i - W_LOADS, xso);
+                U.template load<i - X_DMAS>(wr, wvoff, ws);
         });
     };
 
@@ -619,17 +631,21 @@ __global__ void __launch_bounds__(256, 1) gemm_q_persist(const PersistArgs args)
     };
 
     // prologue, issued in the steady state's order (a stage issues the
-    // weights of g+3, then the activations of g+2): W0 | W1 X0 | W2 X1; then
+    // activations of g+2, then the weights of g+3): W0 | X0 W1 | X1 W2; then
     // stage 0's weights are dequantized and its activations have landed
     x_tile(cx, 0);
     w_tile(cw, 0);
     x_tile(nx, 1);
     w_tile(nw, 1);
     issue_w_all(R0);
-    issue_w_all(R1);
+    __builtin_amdgcn_sched_barrier(0);  // the waits below count loads: their order is fixed
     issue_x_all(X0);
-    issue_w_all(R2);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w_all(R1);
+    __builtin_amdgcn_sched_barrier(0);
     issue_x_all(X1);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w_all(R2);
     LLMR_WAIT_VMCNT(2 * W_LOADS + 2 * X_DMAS);
     {
         const auto sc0 = R0.scale(0);
@@ -638,20 +654,21 @@ __global__ void __launch_bounds__(256, 1) gemm_q_persist(const PersistArgs args)
         R0.template store<2>(W0, sc0, wbase);
         R0.template store<3>(W0, sc0, wbase);
     }
-    LLMR_STAGE_BARRIER(IN_FLIGHT);
+    LLMR_STAGE_BARRIER(IN_FLIGHT + W_LOADS);
 
     Frags F0, F1;
 
     // Global stage g: slots X[g%3], W[g%2]; W(g+1) is in register row R[(g+1)%3].
-    //   wait for W(g+1) (issued first two stages ago: the activation DMAs of
-    //   that stage and all of last stage's loads may stay in flight);
+    //   wait for W(g+1) (issued last two stages ago: all of last stage's loads
+    //   may stay in flight);
     //   k step A: MFMA (g-1,3), frags (g,0), dequant part 0, loads part 0
     //   k step B: MFMA (g,0), frags (g,1), dequant part 1, loads part 1
     //   k step C: MFMA (g,1), frags (g,2), dequant part 2, loads part 2
     //   k step D: MFMA (g,2), frags (g,3), dequant part 3, loads part 3
-    //   (loads: weights of g+3 -> R[g%3], then activations of g+2 -> X[(g+2)%3]);
-    //   barrier once X(g+1) has landed (issued last in the previous stage:
-    //   this stage's loads may stay in flight) and the LDS writes are done.
+    //   (loads: activations of g+2 -> X[(g+2)%3], then weights of g+3 -> R[g%3]);
+    //   barrier once X(g+1) has landed (issued first in the previous stage:
+    //   that stage's weights and this stage's loads may stay in flight) and the
+    //   LDS writes are done.
     // Loads run ahead across tile boundaries (each stream walks the
     // workgroup's tiles on its own), so a tile's first stages are already in
     // flight when its predecessor's results are stored.
@@ -660,14 +677,14 @@ __global__ void __launch_bounds__(256, 1) gemm_q_persist(const PersistArgs args)
         const rsrc_t wr_ = make_rsrc(cw.base, cw.s < S ? cw.size : 0u);                      \
         const rsrc_t xr_ = make_rsrc(cx.base, cx.s < S ? cx.size : 0u);                      \
         const uint32_t ws_ = cw.s, xso_ = cx.s * 128u;                                      \
-        LLMR_WAIT_VMCNT(X_DMAS + IN_FLIGHT);                                                \
+        LLMR_WAIT_VMCNT(IN_FLIGHT);                                                         \
         __builtin_amdgcn_sched_barrier(0);                                                  \
         const auto sc_ = RN.scale(NEXT);                                                    \
         issue_part(std::integral_constant<int, 0>{}, wr_, ws_, xr_, xso_, XD, RL);          \
         read_frags(F0, XC, WC, 0);                                                          \
         mfma_step(F1);                                                                      \
         RN.template store<0>(WNX, sc_, wbase);                                              \
-        LLMR_STEP_SCHEDULE_A;                                                               \
+        if constexpr (EARLY) { LLMR_STEP_SCHEDULE_X; } else { LLMR_STEP_SCHEDULE_A; }       \
         __builtin_amdgcn_sched_barrier(0);                                                  \
         issue_part(std::integral_constant<int, 1>{}, wr_, ws_, xr_, xso_, XD, RL);          \
         read_frags(F1, XC, WC, 1);                                                          \
@@ -689,7 +706,7 @@ __global__ void __launch_bounds__(256, 1) gemm_q_persist(const PersistArgs args)
         __builtin_amdgcn_sched_barrier(0);                                                  \
         advance(cw, nw);                                                                    \
         advance(cx, nx);                                                                    \
-        LLMR_STAGE_BARRIER(IN_FLIGHT);                                                      \
+        LLMR_STAGE_BARRIER(IN_FLIGHT + W_LOADS);                                            \
     }
     for (uint32_t k = 0; k < n_tiles; k++) {
         if (k > 0) {  // the load cursors have moved on to tile k: prepare tile k+1
@@ -820,14 +837,15 @@ struct WHalf<kGgmlQ8_0, OT> {
     }
 };
 
-// One 16-wide k step of the 8-wave kernel: 8 MFMAs, the next step's six
-// fragment reads after the first six, the dequantization's VALU, its LDS
-// write and the step's loads in between.
+// One 16-wide k step of the 8-wave kernel: 8 MFMAs, the step's loads after the
+// first, the next step's six fragment reads after the first six, the
+// dequantization's VALU between them and its LDS write at the end.
 #define LLMR8_SLOT_R LLMR_SGB(0x008, 1); LLMR_SGB(0x100, 1); LLMR_SGB(0x002, 2)
 #define LLMR8_STEP_SCHEDULE                                                                 \
-    LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R;     \
-    LLMR_SGB(0x008, 1); LLMR_SGB(0x002, 4); LLMR_SGB(0x200, 1);                             \
-    LLMR_SGB(0x008, 1); LLMR_SGB(0x002, 4); LLMR_SGB(0x020, 2)
+    LLMR_SGB(0x008, 1); LLMR_SGB(0x020, 4); LLMR_SGB(0x100, 1);                             \
+    LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R; LLMR8_SLOT_R;                   \
+    LLMR_SGB(0x008, 1); LLMR_SGB(0x002, 6);                                                 \
+    LLMR_SGB(0x008, 1); LLMR_SGB(0x002, 6); LLMR_SGB(0x200, 1)
 
 struct Frags8 {
     f16x8 x[4], w[2];
@@ -972,16 +990,19 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         for (int i = 0; i < X_DMAS; i++) dma(xr, Xs, i, cx.s * 128u);
         advance(cx, nx);
     };
+    // the activation DMAs of X(g+2) with the stage's first k step, the weight
+    // loads of W(g+3) with its second (see gemm_q_persist: weights first and
+    // spread over the stage, 1101 x 20480 x 3840 Q8_0 took 238 us, this 211)
     constexpr int N_OPS = W_LOADS + X_DMAS;
     auto issue_part = [&](auto PART, rsrc_t wr, uint32_t ws, rsrc_t xr, uint32_t xso, uint8_t* Xs,
                           WHalf<WT, XT>& U) {
         constexpr int p = decltype(PART)::value;
-        static_for<p * N_OPS / 4, (p + 1) * N_OPS / 4>([&](auto I) {
+        static_for<(p == 0 ? 0 : p == 1 ? X_DMAS : N_OPS), (p == 0 ? X_DMAS : N_OPS)>([&](auto I) {
             constexpr int i = decltype(I)::value;
-            if constexpr (i < W_LOADS)
-                U.template load<i>(wr, wvoff, ws, wh);
+            if constexpr (i < X_DMAS)
+                dma(xr, Xs, i, xso);
             else
-                dma(xr, Xs, i - W_LOADS, xso);
+                U.template load<i - X_DMAS>(wr, wvoff, ws, wh);
         });
     };
 
@@ -1078,7 +1099,7 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         }
     };
 
-    // prologue, as gemm_q_persist's: W0 | W1 X0 | W2 X1, then stage 0's
+    // prologue, as gemm_q_persist's: W0 | X0 W1 | X1 W2, then stage 0's
     // weights are dequantized and its activations have landed
     x_tile(cx, 0);
     w_tile(cw, 0);
@@ -1087,10 +1108,14 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         w_tile(nw, 1);
     }
     issue_w_all(R0);
-    issue_w_all(R1);
+    __builtin_amdgcn_sched_barrier(0);  // the waits below count loads: their order is fixed
     issue_x_all(X0);
-    issue_w_all(R2);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w_all(R1);
+    __builtin_amdgcn_sched_barrier(0);
     issue_x_all(X1);
+    __builtin_amdgcn_sched_barrier(0);
+    issue_w_all(R2);
     LLMR_WAIT_VMCNT(2 * W_LOADS + 2 * X_DMAS);
     {
         const auto sc0 = R0.scale(S0, wh);
@@ -1099,7 +1124,7 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         R0.template store<2>(W0, sc0, wbase, wh);
         R0.template store<3>(W0, sc0, wbase, wh);
     }
-    LLMR_STAGE_BARRIER(IN_FLIGHT);
+    LLMR_STAGE_BARRIER(IN_FLIGHT + W_LOADS);
 
     Frags8 F0, F1;
     // the stage of gemm_q_persist with this kernel's fragments and schedule
@@ -1108,7 +1133,7 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         const rsrc_t wr_ = make_rsrc(cw.base, cw.s < S ? cw.size : 0u);                      \
         const rsrc_t xr_ = make_rsrc(cx.base, cx.s < S ? cx.size : 0u);                      \
         const uint32_t ws_ = cw.s, xso_ = cx.s * 128u;                                      \
-        LLMR_WAIT_VMCNT(X_DMAS + IN_FLIGHT);                                                \
+        LLMR_WAIT_VMCNT(IN_FLIGHT);                                                         \
         __builtin_amdgcn_sched_barrier(0);                                                  \
         const auto sc_ = RN.scale(NEXT, wh);                                                \
         issue_part(std::integral_constant<int, 0>{}, wr_, ws_, xr_, xso_, XD, RL);          \
@@ -1137,7 +1162,7 @@ __global__ void __launch_bounds__(512, 1) gemm_q_persist8(const PersistArgs args
         __builtin_amdgcn_sched_barrier(0);                                                  \
         advance(cw, nw);                                                                    \
         advance(cx, nx);                                                                    \
-        LLMR_STAGE_BARRIER(IN_FLIGHT);                                                      \
+        LLMR_STAGE_BARRIER(IN_FLIGHT + W_LOADS);                                            \
     }
     for (uint32_t k = 0; k < n_tiles; k++) {
         if (k > 0) {

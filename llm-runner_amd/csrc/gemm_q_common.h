@@ -338,6 +338,13 @@ struct WRow<kGgmlQ8_0, OT> {
     LLMR_SLOT_R; LLMR_SLOT_R; LLMR_SLOT_L; LLMR_SLOT_V; LLMR_SLOT_W; LLMR_SLOT_L;             \
     LLMR_SLOT_V; LLMR_SLOT_W; LLMR_SLOT_L; LLMR_SLOT_L
 
+// the first step of a stage whose eight activation DMAs all go with it
+#define LLMR_SLOT_RX LLMR_SGB(0x008, 1); LLMR_SGB(0x100, 1); LLMR_SGB(0x020, 1); LLMR_SGB(0x002, 5)
+#define LLMR_STEP_SCHEDULE_X                                                                \
+    LLMR_SLOT_RX; LLMR_SLOT_RX; LLMR_SLOT_RX; LLMR_SLOT_RX; LLMR_SLOT_RX; LLMR_SLOT_RX;       \
+    LLMR_SLOT_RX; LLMR_SLOT_RX; LLMR_SLOT_VA; LLMR_SLOT_VA; LLMR_SLOT_WA; LLMR_SLOT_VA;       \
+    LLMR_SLOT_VA; LLMR_SLOT_WA; LLMR_SLOT_VA; LLMR_SLOT_VA
+
 struct Frags {
     f16x8 x[4], w[4];
 };
