@@ -30,29 +30,34 @@ constexpr int kD = 128;
 // NB blocks of 32 queries (NB = 1: 8 waves, two per SIMD; the kernel is
 // written for any NB, and with NB = 2 every K or V fragment read from LDS
 // feeds two MFMAs). K and V tiles of 64 keys go HBM -> LDS by buffer DMA
-// (no staging registers, no VALU) into 3-slot rings, K three tiles and V two
-// tiles ahead of use; V stays row-major in LDS and the V^T operand is read
+// (no staging registers, no VALU) into rings of four K and three V slots, K
+// four tiles and V two tiles ahead; V stays row-major in LDS and the V^T operand is read
 // with the transposing ds_read_b64_tr_b16 (lane i of a 16-lane group gets
 // V[key0 + e][d0 + i], e = 0..3).
 //
 // Scores live in three 32-key halves used in rotation, so the MFMAs of
 // S(t+1) = K(t+1) Q^T go to a free half while S(t) is exponentiated. Per
-// tile t a wave: DMAs K(t+3) and V(t+2); computes S(t+1) on the matrix
+// tile t a wave: DMAs K(t+4) and V(t+2); computes S(t+1) on the matrix
 // cores while the vector ALU exponentiates S(t) into the fp16 P(t);
-// accumulates O^T += V(t)^T P(t)^T while taking the row max of S(t+1);
-// rescales O if a running max grew by more than 2^8 (lazily: O and the row
+// accumulates O^T += V(t)^T P(t)^T while taking the row max of S(t+1), then
+// reads the first fragments of K(t+2), so that the next tile starts without
+// waiting for LDS; rescales O if a running max grew by more than 2^8 (lazily: O and the row
 // sum keep a stale max until then, exp2 of at most 2^8 cannot overflow);
-// then one barrier. The main loop is unrolled by 3 (the
-// halves) and walks the LDS rings with scalar slot offsets. It runs while
+// then one barrier. Bound: per tile and SIMD the two waves have 2048 cycles of
+// MFMA and about 1400 of vector ALU and take 3090 (counters at H = 24, S =
+// 4608; 3180 with a three-slot K ring read only after the barrier, the row max
+// after the last MFMA and an address computed for most of the transposing
+// reads: 253.3 -> 250.3 us, S = 2048 63.6 -> 62.1). The main loop is unrolled
+// by 3 (the halves) and walks the LDS rings with scalar slot offsets. It runs while
 // S(t+1) has no keys past the sequence end; one masked iteration follows
 // when the last tile is partial, then a final iteration that only
 // exponentiates and accumulates.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kBQ64 = 256;            // queries per workgroup
 constexpr uint32_t kTile64 = 64u * 256u;   // one K or V tile: 64 keys x 128 fp16
-// LDS of a workgroup: the K and V rings (6 tiles), or the epilogue's
+// LDS of a workgroup: the K and V rings (4 + 3 tiles), or the epilogue's
 // staging of the output rows (kBQ64 queries x 128 f32)
-constexpr uint32_t kFaLds = kBQ64 * 128u * 4u > 6u * kTile64 ? kBQ64 * 128u * 4u : 6u * kTile64;
+constexpr uint32_t kFaLds = kBQ64 * 128u * 4u > 7u * kTile64 ? kBQ64 * 128u * 4u : 7u * kTile64;
 
 // LDS rows are 256 bytes (16 chunks of 8 fp16). K: chunk c of key r at
 // c ^ (r & 15) (a 16-lane fragment read touches 16 distinct bank quads).
@@ -72,7 +77,8 @@ __device__ __forceinline__ float xhalf_sum(float x) {
 }
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) f16x8 lds_f16x8;
 
 // QT: type of Q (F16, or F32 / BF16 rounded to fp16 as the fragments are
 // loaded: Q is read once per workgroup, so it needs no conversion pass)
@@ -83,7 +89,7 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
                                           const _Float16* __restrict__ V, void* __restrict__ O, uint32_t ostride,
                                           uint32_t S,
                                           uint32_t H, float scale_log2, uint32_t n_qb) {
-    // K ring in slots 0..2, V ring in slots 3..5
+    // K ring in slots 0..3, V ring in slots 4..6
     // (after the key loop the epilogue stages O in it: 16 KiB per 32 queries)
     __shared__ __attribute__((aligned(16))) uint8_t lds[kFaLds];
     constexpr uint32_t ROW = kD * 2u;  // bytes per token row of one head
@@ -213,32 +219,53 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
         for (int dt = 0; dt < 4; dt++) o[dt][b] = f32x16{};
     }
 
+    // the lane's fragment addresses in a K or V slot, in registers of their own:
+    // every read of a tile is then one of them plus an immediate (left to
+    // itself the compiler forms the 32 transposing reads' addresses one by one)
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)lds;
+    auto kaddr = [&](uint32_t slot, uint32_t (&ka)[4][2]) {
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+                ka[c][st] = lds0 + slot * kTile64 + kfo[c][st];
+                asm("" : "+v"(ka[c][st]));
+            }
+    };
+    auto vaddr = [&](uint32_t slot, uint32_t (&va)[4]) {
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            va[dt] = lds0 + (4u + slot) * kTile64 + vto[dt];
+            asm("" : "+v"(va[dt]));
+        }
+    };
+
     // Score halves: the scores of one 32-key block of a tile for both query
     // blocks; h[b] at lane l holds key 32kb + 8(i/4) + 4kh + i%4 of the
     // tile (kb = the block), query 32b + l32.
     //
     // K fragment f = 0..15 of the tile at Ks: key block f/8, d chunk
     // (c, st) = ((f%8)/2, f%2)
-    auto kfrag = [&](const uint8_t* Ks, int f) -> f16x8 {
-        return *(const f16x8*)(Ks + 32u * (uint32_t)(f / 8) * ROW + kfo[(f % 8) / 2][f % 2]);
+    auto kfrag = [&](const uint32_t (&ka)[4][2], int f) -> f16x8 {
+        return *(const lds_f16x8*)(uintptr_t)(ka[(f % 8) / 2][f % 2] + 32u * (uint32_t)(f / 8) * ROW);
     };
     // V^T fragment f = 0..15 of the tile at Vs: key block kb = f/8, keys
     // 32kb + 16c + {4kh..4kh+3, 8+4kh..8+4kh+3} with c = (f%8)/4, dims
     // 32dt + l32 with dt = f%4
-    auto vfrag = [&](const uint8_t* Vs, int f) -> f16x8 {
+    auto vfrag = [&](const uint32_t (&va)[4], int f) -> f16x8 {
         const uint32_t R = 32u * (uint32_t)(f / 8) + 16u * (uint32_t)((f % 8) / 4);
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(Vs + R * ROW + vto[f % 4]));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)(Vs + (R + 8u) * ROW + vto[f % 4]));
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(va[f % 4] + R * ROW));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)(va[f % 4] + (R + 8u) * ROW));
         return __builtin_bit_cast(
             f16x8, (short __attribute__((ext_vector_type(8)))){lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w});
     };
-    // S of the tile at Ks into the halves (h0: keys 0..31, h1: keys 32..63)
-    auto qk_all = [&](const uint8_t* Ks, f32x16 (&h0)[NB], f32x16 (&h1)[NB]) {
+    // S of the tile in K slot 0 into the halves (h0: keys 0..31, h1: keys 32..63)
+    auto qk_all = [&](f32x16 (&h0)[NB], f32x16 (&h1)[NB]) {
+        uint32_t ka[4][2];
+        kaddr(0, ka);
         static_for<0, 16>([&](auto F) {
             constexpr int f = F, kb = f / 8, c = (f % 8) / 2, st = f % 2;
-            const f16x8 a = kfrag(Ks, f);
+            const f16x8 a = kfrag(ka, f);
             static_for<0, NB>([&](auto B) {
                 constexpr int b = B;
                 f32x16& s = kb == 0 ? h0[b] : h1[b];
@@ -273,11 +300,8 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
     // raise m_ref where the tile whose scores are in (n0, n1) exceeds it by
     // more than 2^8 (lazily: exp2 of at most 2^8 cannot overflow), and shift
     // those scores to the new m_ref (the next tile's MFMAs start from it)
-    auto rescale = [&](const float (&mx)[NB], f32x16 (&n0)[NB], f32x16 (&n1)[NB]) {
-        bool grow = false;
-#pragma unroll
-        for (int b = 0; b < NB; b++) grow = grow || mx[b] > 8.0f;
-        if (__builtin_amdgcn_ballot_w64(grow) != 0) {
+    auto rescale = [&](uint64_t grow, const float (&mx)[NB], f32x16 (&n0)[NB], f32x16 (&n1)[NB]) {
+        if (grow != 0) {
 #pragma unroll
             for (int b = 0; b < NB; b++) {
                 const float d = fmaxf(mx[b], 0.0f);
@@ -309,66 +333,79 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
 
     // One tile t. S(t) is in (c0, c1); S(t+1) = K(t+1) Q^T goes to (n0, c0)
     // (n0 free; c0's block-0 scores are exponentiated before its first
-    // write). K(t+1) is in LDS slot ks, V(t) in V slot vs; K(t+3) is DMAed
-    // to K slot kd and V(t+2) to V slot vd.
+    // write). K(t+1) is in K slot (t+1) % 4, V(t) in V slot vs; K(t+4) is
+    // DMAed to K slot t % 4 and V(t+2) to V slot vd.
     // The 32 NB MFMAs (16 NB for S(t+1), then 16 NB for O^T += V(t)^T P(t)^T)
     // are issued in a fixed order with the vector work spread between them:
     // the exponentials of block 0 under the first 8 NB, those of block 1
     // under the next 16 NB (P's block 0 is complete before its accumulation
-    // starts), then the row max of S(t+1) under the accumulation MFMAs.
+    // starts), the row max of S(t+1) under the next 8 NB, the first fragment reads
+    // of K(t+2) (landed at the last barrier) under the rest.
     // Fragment reads run PF fragments ahead of their MFMAs. sched_barrier
     // fences keep that order.
-    auto tile = [&](f32x16 (&c0)[NB], f32x16 (&c1)[NB], f32x16 (&n0)[NB], uint32_t t, uint32_t ks, uint32_t vs,
-                    uint32_t kd, uint32_t vd, auto masked) {
-        dma(Kh, kvo, t + 3u, kd);
-        dma(Vh, vvo, t + 2u, 3u + vd);
-        const uint8_t* Ks = lds + ks * kTile64;
-        const uint8_t* Vs = lds + (3u + vs) * kTile64;
+    constexpr int PF = 3;  // fragments in flight ahead of their MFMAs
+    uint32_t ka[4][2];     // K(t+1)'s fragment addresses
+    f16x8 kf[PF + 1];      // its fragments in flight: the first PF are read before the tile starts
+    auto tile = [&](f32x16 (&c0)[NB], f32x16 (&c1)[NB], f32x16 (&n0)[NB], uint32_t t, uint32_t vs, uint32_t vd,
+                    auto masked) {
+        dma(Kh, kvo, t + 4u, t & 3u);
+        dma(Vh, vvo, t + 2u, 4u + vd);
+        uint32_t va[4];
+        vaddr(vs, va);
         f16x8 p[NB][2][2];
-        constexpr int PF = 3;  // fragments in flight ahead of their MFMAs
         constexpr int QS = 16 * NB;  // steps of the score MFMAs (then as many accumulation steps)
-        f16x8 kf[PF + 1], vf[PF + 1];
+        f16x8 vf[PF + 1];
         float rs[NB], mt[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
             rs[b] = 0.0f;
             mt[b] = -INFINITY;
         }
-        static_for<0, PF>([&](auto F) { kf[F] = kfrag(Ks, F); });
+        float mx[NB];
+        uint64_t grow = 0;
         static_for<0, 2 * QS>([&](auto J) {
             constexpr int j = J;
             if constexpr (j < QS) {
                 constexpr int f = j / NB, b = j % NB, kb = f / 8, c = (f % 8) / 2, st = f % 2;
-                if constexpr (b == 0 && f + PF < 16) kf[(f + PF) % (PF + 1)] = kfrag(Ks, f + PF);
+                if constexpr (b == 0 && f + PF < 16) kf[(f + PF) % (PF + 1)] = kfrag(ka, f + PF);
                 f32x16& s = kb == 0 ? n0[b] : c0[b];
                 s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[f % (PF + 1)], qf[b][c][st],
                                                            (c == 0 && st == 0) ? f32x16{} - m_ref[b] : s, 0, 0,
                                                            0);
             } else {
                 constexpr int f = (j - QS) / NB, b = j % NB, kb = f / 8, c = (f % 8) / 4, dt = f % 4;
-                if constexpr (b == 0 && f + PF < 16) vf[(f + PF) % (PF + 1)] = vfrag(Vs, f + PF);
+                if constexpr (b == 0 && f + PF < 16) vf[(f + PF) % (PF + 1)] = vfrag(va, f + PF);
                 o[dt][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[f % (PF + 1)], p[b][kb][c], o[dt][b], 0, 0, 0);
             }
-            if constexpr (j >= QS - PF && j < QS) vf[j - (QS - PF)] = vfrag(Vs, j - (QS - PF));
+            if constexpr (j >= QS - PF && j < QS) vf[j - (QS - PF)] = vfrag(va, j - (QS - PF));
             if constexpr (j < 8 * NB) exp_pair(c0, 0, j, p, rs);
             if constexpr (j >= 8 * NB && j < 24 * NB && j % 2 == 0) exp_pair(c1, 1, (j - 8 * NB) / 2, p, rs);
             if constexpr (decltype(masked)::value && j == QS - 1) mask(n0, c0, t + 1u);
-            if constexpr (j >= QS && j % 2 == 0) {
+            if constexpr (j >= QS && j < 24 * NB) {
                 // row max item k: half k/(4NB) (n0, then c0), query block (k%(4NB))/4, scores 4(k%4)..+3
-                constexpr int k = (j - QS) / 2, b = (k % (4 * NB)) / 4, i = 4 * (k % 4);
+                constexpr int k = j - QS, b = (k % (4 * NB)) / 4, i = 4 * (k % 4);
                 const f32x16& s = k < 4 * NB ? n0[b] : c0[b];
                 mt[b] = fmaxf(fmaxf(mt[b], s[i]), s[i + 1]);
                 mt[b] = fmaxf(fmaxf(mt[b], s[i + 2]), s[i + 3]);
             }
+            if constexpr (j == 24 * NB) {
+#pragma unroll
+                for (int b = 0; b < NB; b++) mx[b] = xhalf_max(mt[b]);
+            }
+            if constexpr (j == 24 * NB + 1) {
+                bool g = false;
+#pragma unroll
+                for (int b = 0; b < NB; b++) g = g || mx[b] > 8.0f;
+                grow = __builtin_amdgcn_ballot_w64(g);
+            }
+            if constexpr (j == 24 * NB + 2) kaddr((t + 2u) & 3u, ka);
+            if constexpr (j >= 24 * NB + 3 && j < 24 * NB + 3 + PF)  // K(t+2): this tile's successor starts with it
+                kf[j - (24 * NB + 3)] = kfrag(ka, j - (24 * NB + 3));
             __builtin_amdgcn_sched_barrier(0);
         });
-        float mx[NB];
 #pragma unroll
-        for (int b = 0; b < NB; b++) {
-            l_i[b] += rs[b];
-            mx[b] = xhalf_max(mt[b]);
-        }
-        rescale(mx, n0, c0);
+        for (int b = 0; b < NB; b++) l_i[b] += rs[b];
+        rescale(grow, mx, n0, c0);
         LLMR_STAGE_BARRIER(4 * NB);
     };
 
@@ -377,17 +414,18 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
     // iterations t whose S(t+1) has no key past the sequence end
     const uint32_t n_plain = partial ? (n_tiles >= 2u ? n_tiles - 2u : 0u) : n_tiles - 1u;
 
-    // prologue: K(0) V(0) K(1) V(1) K(2) in flight; S(0) and its max
+    // prologue: K(0) V(0) K(1) K(2) V(1) K(3) in flight; S(0) and its max
     dma(Kh, kvo, 0, 0);
-    dma(Vh, vvo, 0, 3);
+    dma(Vh, vvo, 0, 4);
     dma(Kh, kvo, 1, 1);
-    dma(Vh, vvo, 1, 4);
     dma(Kh, kvo, 2, 2);
-    LLMR_STAGE_BARRIER(8 * NB);  // K(0) has landed
+    dma(Vh, vvo, 1, 5);
+    dma(Kh, kvo, 3, 3);
+    LLMR_STAGE_BARRIER(10 * NB);  // K(0) has landed
     f32x16 h0[NB], h1[NB], h2[NB];
     {   // S(0) from zero; its row max becomes m_ref, S(0) relative to it
         float mx[NB];
-        qk_all(lds, h0, h1);
+        qk_all(h0, h1);
         if (n_tiles == 1u && partial) mask(h0, h1, 0);
         rowmax(h0, h1, mx);
 #pragma unroll
@@ -397,16 +435,17 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
             h1[b] -= mx[b];
         }
     }
-    LLMR_STAGE_BARRIER(4 * NB);  // K(1), V(0) have landed; every wave is done with K(0)
+    LLMR_STAGE_BARRIER(4 * NB);  // K(1), K(2), V(0) have landed; every wave is done with K(0)
+    kaddr(1, ka);
+    static_for<0, PF>([&](auto F) { kf[F] = kfrag(ka, F); });
 
-    // t % 3 = r0 names the ring slots: K(t+1) in r1, V(t) in r0; K(t+3) to
-    // r0 (K(t), last read in iteration t-1), V(t+2) to r2 (V(t-1)). The
+    // t % 3 = r0 names the V ring's slots: V(t) in r0, V(t+2) to r2 (V(t-1)). The
     // score halves rotate with period 3: S(t) in (h0, h1), (h2, h0), (h1, h2).
     uint32_t t = 0, r0 = 0;
     auto step = [&](f32x16 (&c0)[NB], f32x16 (&c1)[NB], f32x16 (&n0)[NB], auto masked) {
         const uint32_t r1 = r0 == 2u ? 0u : r0 + 1u;
         const uint32_t r2 = r0 == 0u ? 2u : r0 - 1u;
-        tile(c0, c1, n0, t, r1, r0, r0, r2, masked);
+        tile(c0, c1, n0, t, r0, r2, masked);
         t++;
         r0 = r1;
     };
@@ -440,10 +479,11 @@ __device__ __forceinline__ void fa64_body(const void* __restrict__ Q, const _Flo
         static_for<0, 8 * NB>([&](auto I) { exp_pair(h1, 1, I, p, rs); });
 #pragma unroll
         for (int b = 0; b < NB; b++) l_i[b] += rs[b];
-        const uint8_t* Vs = lds + (3u + r0) * kTile64;
+        uint32_t va[4];
+        vaddr(r0, va);
         static_for<0, 16>([&](auto F) {
             constexpr int f = F, kb = f / 8, c = (f % 8) / 4, dt = f % 4;
-            const f16x8 a = vfrag(Vs, f);
+            const f16x8 a = vfrag(va, f);
             static_for<0, NB>([&](auto B) {
                 o[dt][B] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, p[B][kb][c], o[dt][B], 0, 0, 0);
             });
