@@ -154,8 +154,8 @@ inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, u
     return 6.0 + rounds * ((double)K / t.splits) * per_k;
 }
 
-// Launches below kW16MinTokens tokens whose 256 x 256 tiles leave CUs idle in
-// their last round: the whole rounds of tiles run as they are (`full` of
+// Launches below kW16MinTokens tokens, or with too few tiles for the persistent
+// kernels, whose 256 x 256 tiles leave CUs idle in their last round: the whole rounds of tiles run as they are (`full` of
 // them) and every tile of the last round is cut along K into `splits`
 // workgroups, whose partial tiles a second launch adds up. The times are
 // estimates in us on MI355X (256 CUs), fitted to launches of 300-2000 tokens
@@ -166,7 +166,8 @@ inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, u
 // whole launch before -> after: 1101 x 3840 x 3840 Q8_0 (75 tiles x 3) 129 ->
 // 60 us, x 10240 348 -> 117; 520 x 9216 x 3072 Q4_K (108 x 2) 99 -> 60; 1536 x
 // 11520 x 3840 Q8_0 (256 whole tiles + 14 x 15) 236 -> 160; 2000 x 9216 x
-// 3072 Q4_K (256 + 32 x 8) 165 -> 139. Where the estimates are within 3%
+// 3072 Q4_K (256 + 32 x 8) 165 -> 139; 2048 x 3840 x 3840 Q8_0 (120 x 2) 123
+// -> 88, x 10240 256 -> 169. Where the estimates are within 3%
 // the launch stays whole (2000 x 12288 x 3072 Q4_K, 128 tiles in its last
 // round: 168 whole, 177 split).
 constexpr size_t kPartTile = 256u * 256u * sizeof(float);  // one partial tile
@@ -209,7 +210,7 @@ inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t
 //    activations rounded to operand_type() into the workspace first; from
 //    kW16MinTokens tokens two-pass (the 16-bit weight image after them in
 //    the workspace);
-//  * split: below kW16MinTokens tokens, where plan_split finds that cutting
+//  * split: below kW16MinTokens tokens or where not persistent, where plan_split finds that cutting
 //    the last round's tiles along K pays: [x16 | partial tiles];
 //  * otherwise the tiled kernel, split-K partials in the workspace.
 // With a workspace limit (the no-allocation entry point's fixed array) the
@@ -266,7 +267,7 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
             return p;
         }
     }
-    if (K % kStageK == 0 && N % 4 == 0 && offsets31 && M < kW16MinTokens) {
+    if (K % kStageK == 0 && N % 4 == 0 && offsets31 && (M < kW16MinTokens || !p.persistent)) {
         const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent);
         if (few_ok && few_us(wtype, xtype, N, K, M, num_cus) < 0.97 * sp.us) {
             p.few = true;

@@ -337,7 +337,8 @@ def test_few_token_tiles(dev, wtype, M, N, K, xtype, row_offset):
     assert err <= TOL
 
 
-# Launches below 2048 tokens whose last round of tiles is cut along K.
+# Launches below 2048 tokens, or with too few tiles for the persistent kernels,
+# whose last round of tiles is cut along K.
 SPLIT_TILE_CASES = [
     # (wtype, M, N, K, xtype, row_offset)
     (8, 1101, 3840, 3840, 0, 0),     # 75 tiles x 3 splits of 20 stages, f32 activations as fp16
@@ -346,6 +347,7 @@ SPLIT_TILE_CASES = [
     (12, 513, 2052, 5120, 1, 4),     # splits of unequal stage counts
     (8, 1536, 11520, 1088, 30, 0),   # 256 whole tiles, 14 cut into splits of 17 stages in all
     (12, 2047, 9216, 3072, 30, 0),   # 256 whole tiles, 32 x 8
+    (8, 2049, 2052, 2048, 1, 0),     # 81 tiles past 2048 tokens, one row and four features past a tile
 ]
 
 
