@@ -124,25 +124,41 @@ def test_gemv_against_64_bits(dev, wtype, M, N, K, xtype, row_offset):
         assert err < 1e-6
 
 
-@pytest.mark.parametrize("wtype", [8, 12])
-def test_gemv_nonfinite_activations(dev, wtype):
+@pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", [
+    (8, 3, 70, 512, 0, 0),         # the waves share 16 rows: six of the last workgroup's
+    (12, 3, 70, 512, 0, 0),
+    (12, 1, 8250, 256, 30, 3),     # 64 rows a workgroup, fewer pieces of 32 weights than a row's lanes
+    (8, 1, 8197, 768, 1, 1),
+    (12, 2, 8203, 2304, 1, 0),
+    (8, 4, 8192, 1280, 30, 0),
+])
+def test_gemv_nonfinite_activations(dev, wtype, M, N, K, xtype, row_offset):
     """An infinite or NaN activation gives the products of the dequantized
     weight (Inf of each weight's sign, NaN at a zero weight) for its token and
-    leaves the others as they are."""
+    leaves the others as they are (K / 16 additions per lane and token, 2^-24
+    each at random signs: 1e-6)."""
     import torch
     from llmr_amd import ops
-    M, N, K = 3, 70, 512
-    w = _weights(dev, wtype, N, K, 280 + wtype)
+    w = _weights(dev, wtype, N + row_offset, K, 280 + wtype)
     x = torch.randn(M, K, generator=torch.Generator(device="cpu").manual_seed(9))
-    good = ops.batch_matmul(w, wtype, x.to(dev), N).cpu()
+    x = x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)
+    wd = ops.dequant(w, wtype, N, K, row_offset)
+    good = (x.to(dev).double() @ wd.double().t()).cpu()
     x[0, 100] = float("inf")
-    x[2, 400] = float("nan")
-    y = ops.batch_matmul(w, wtype, x.to(dev), N).cpu()
-    col = ops.dequant(w, wtype, N, K).cpu()[:, 100]
+    if M == 3:
+        x[2, 200] = float("nan")
+    buf = torch.full((M * N + 64,), 7.0, device=dev)
+    y = buf[:M * N].view(M, N)
+    ops.batch_matmul(w, wtype, x.to(dev), N, row_offset=row_offset, out=y)
+    y = y.cpu()
+    assert bool((buf[M * N:] == 7.0).all())
+    col = wd.cpu()[:, 100]
     want = torch.where(col == 0, torch.tensor(float("nan")), torch.copysign(torch.tensor(float("inf")), col))
     assert torch.equal(torch.nan_to_num(y[0], nan=7.0), torch.nan_to_num(want, nan=7.0))
-    assert bool(torch.isnan(y[2]).all())
-    assert rel_l2(y[1].numpy(), good[1].numpy()) < 1e-6
+    if M == 3:
+        assert bool(torch.isnan(y[2]).all())
+    for m in (m for m in range(1, M) if M != 3 or m == 1):
+        assert rel_l2(y[m].numpy(), good[m].numpy()) < 1e-6
 
 
 @pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", CASES)
