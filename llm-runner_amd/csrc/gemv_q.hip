@@ -151,10 +151,13 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
 //    sub-block's largest lies in [2^29, 2^30) and rounded to an integer (31
 //    bits under the largest), is the sum of four signed base-256 digits; sums of
 //    quant x digit over a sub-block are exact in int32, and the four of them
-//    make one f32 with a single rounding;
-//  * Q4_K: the sums start at -8 times the sub-block's digit sums, so they are of
-//    the quants less 8, and acc += (d sc) sum (q - 8) x - (dmin mn - 8 d sc) sum x
-//    cancels little of what the two f32 terms round.
+//    make one f32 with a single rounding (Q8_0, whose pairs of sums pass 2^24:
+//    with up to three);
+//  * Q4_K: acc += (d sc) sum (q - c) x - (dmin mn - c d sc) sum x with c the quant
+//    whose weight is nearest zero; the first sum is exact (c times the
+//    activations' digit sums off the products). Both terms are then of the size of
+//    the weights times x, and a zero weight's activation is in neither: one 300
+//    times the rest of its sub-block leaves 0.9-2.1e-7 (8 for every c: 2-7e-6).
 // That is at least as exact as f32 FMAs on f32 activations (18432 x 3072: 1.4e-7
 // relative to 64 bits, the FMA kernel 2.5e-7). An infinite or NaN activation has
 // no digits: such a workgroup multiplies in f32 (gemv_f32_rows).
@@ -170,7 +173,7 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
 // Measured per call, before -> after (one token, FMA kernel; Q8_0, the few-token
 // GEMMs): 18432 x 3072 Q4_K 19.5 -> 9.7 us (3.3 TB/s), 38 of them grouped 328
 // -> 210 us (5.8 TB/s), 3072 x 15360 76 -> 12, two and four tokens of 18432 x
-// 3072 31 -> 16 and 56 -> 28 us; 11520 x 3840 Q8_0 54 -> 9.8 us (4.8 TB/s).
+// 3072 31 -> 15 and 56 -> 26 us; 11520 x 3840 Q8_0 54 -> 9.8 us (4.8 TB/s).
 // ---------------------------------------------------------------------------
 
 // Up to CAP projections of one shape [N, K] (each its own weight, input
@@ -196,16 +199,15 @@ struct GemvW {
 };
 
 // LDS of the activations per unit, T token slots (1, 2 or 4). Digits: 16 k at a
-// time, [digit][token][16 bytes]. Then per sub-block: Q4_K, the sums' start
-// [digit][token] (one token: [digit]); (1 / scale, activation sum) per token.
+// time, [digit][token][16 bytes]. Then per sub-block and token: Q4_K, the sums of
+// its two upper and two lower digits, 1 / scale, activation sum; Q8_0, 1 / scale.
 // Units are padded so the four a wave reads together lie 64 bytes apart in the
 // banks.
 template <uint32_t WT, int T>
 struct GemvX {
     static constexpr uint32_t kSub = GemvW<WT>::kK / 32u;
     static constexpr uint32_t kDigits = GemvW<WT>::kK / 16u * (64u * T);
-    static constexpr uint32_t kStart = WT == kGgmlQ4K ? (T == 1 ? 16u : 64u) : 0u;
-    static constexpr uint32_t kSubBytes = kStart + (T == 4 ? 32u : 16u);
+    static constexpr uint32_t kTok = WT == kGgmlQ4K ? 16u : 8u, kSubBytes = kTok * T;
     static constexpr uint32_t kUsed = kDigits + kSub * kSubBytes, kUnit = kUsed + (320u - kUsed % 256u) % 256u;
 };
 // the activations as f32 in the same region: 16 bytes of padding every 64 k, so
@@ -417,7 +419,7 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         const int e = min(126, max(-126, 156 - (int)((__float_as_uint(mx) >> 23) & 0xffu)));
         const float up = __uint_as_float((uint32_t)(127 + e) << 23), down = __uint_as_float((uint32_t)(127 - e) << 23);
         uint32_t dg[2][4];  // [four k][digit, lowest first]: a byte per k
-        int start[4] = {0, 0, 0, 0};
+        int sums[4] = {0, 0, 0, 0};
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             uint32_t v4[4];
@@ -439,14 +441,13 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
             dg[h][3] = __builtin_amdgcn_perm(c1, a1, 0x07060302u);
             if constexpr (WT == kGgmlQ4K)
 #pragma unroll
-                for (int p = 0; p < 4; p++) start[p] = __builtin_amdgcn_sdot4((int)dg[h][p], 0x01010101, start[p], false);
+                for (int p = 0; p < 4; p++) sums[p] = __builtin_amdgcn_sdot4((int)dg[h][p], 0x01010101, sums[p], false);
         }
         if constexpr (WT == kGgmlQ4K)
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                start[p] += __shfl_xor(start[p], 1, 64);
-                start[p] += __shfl_xor(start[p], 2, 64);
-                start[p] *= -8;
+                sums[p] += __shfl_xor(sums[p], 1, 64);
+                sums[p] += __shfl_xor(sums[p], 2, 64);
             }
         if (i >= total) return;
         const uint32_t m = T == 1 ? 0u : i / pieces, c = T == 1 ? i : i - m * pieces;  // chunk of 8 k
@@ -455,16 +456,11 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 #pragma unroll
         for (int p = 0; p < 4; p++) *(u32x2*)(dst + p * (16u * T)) = u32x2{dg[0][p], dg[1][p]};
         if (cu % 4u == 0u) {
-            uint8_t* const sb = smem + u * GX::kUnit + GX::kDigits + cu / 4u * GX::kSubBytes;
-            if constexpr (WT == kGgmlQ4K) {
-                if constexpr (T == 1) {
-                    *(i32x4*)sb = i32x4{start[0], start[1], start[2], start[3]};
-                } else {
-#pragma unroll
-                    for (int p = 0; p < 4; p++) *(int*)(sb + 16u * p + 4u * m) = start[p];  // (rows past T: unused)
-                }
-            }
-            *(f32x2*)(sb + GX::kStart + 8u * m) = f32x2{down, sum};
+            uint8_t* const sb = smem + u * GX::kUnit + GX::kDigits + cu / 4u * GX::kSubBytes + GX::kTok * m;
+            if constexpr (WT == kGgmlQ4K)
+                *(f32x4*)sb = f32x4{(float)(sums[3] * 256 + sums[2]), (float)(sums[1] * 256 + sums[0]), down, sum};
+            else
+                *(float*)sb = down;
         }
     };
 #pragma unroll
@@ -511,26 +507,23 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
                 d2[p] = __builtin_amdgcn_mfma_i32_4x4x4i8((int)a2[p][q], (int)w2[q], d2[p], 0, 0, 0);
         }
     };
-    auto begin = [&](i32x4 (&d)[P], const uint8_t* sb) __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            if constexpr (WT == kGgmlQ4K)
-                d[p] = *(const i32x4*)(sb + 16u * p);
-            else
-                d[p] = i32x4{0, 0, 0, 0};
-        }
-    };
-    // acc += ds (sum q x) - dm (sum x) of one sub-block
-    auto add = [&](const i32x4 (&d)[P], const uint8_t* sb, float ds, float dm) __attribute__((always_inline)) {
+    // acc += ds (sum (q - c) x) - dm (sum x) of one sub-block
+    auto add = [&](const i32x4 (&d)[P], const uint8_t* sb, float ds, float dm, float c) __attribute__((always_inline)) {
 #pragma unroll
         for (int m = 0; m < T; m++) {
-            const f32x2 s = *(const f32x2*)(sb + GX::kStart + 8u * m);
             const int d0 = T == 1 ? d[0].x : d[0][m], d1 = T == 1 ? d[0].y : d[1 % P][m];
             const int d2 = T == 1 ? d[0].z : d[2 % P][m], d3 = T == 1 ? d[0].w : d[3 % P][m];
-            // both pairs are below 2^24
-            const float t = __builtin_fmaf((float)(d3 * 256 + d2), 65536.0f, (float)(d1 * 256 + d0));
-            acc[m] = __builtin_fmaf(ds * t, s.x, acc[m]);
-            if constexpr (WT == kGgmlQ4K) acc[m] = __builtin_fmaf(-dm, s.y, acc[m]);
+            float hi = (float)(d3 * 256 + d2), lo = (float)(d1 * 256 + d0);
+            if constexpr (WT == kGgmlQ4K) {
+                // quants to 15: both pairs, c times the digits' and the differences
+                // are whole numbers below 2^24, so only t rounds
+                const f32x4 s = *(const f32x4*)(sb + GX::kTok * m);
+                const float t = __builtin_fmaf(__builtin_fmaf(-c, s.x, hi), 65536.0f, __builtin_fmaf(-c, s.y, lo));
+                acc[m] = __builtin_fmaf(-dm, s.w, __builtin_fmaf(ds * t, s.z, acc[m]));
+            } else {  // (quants to 127: the pairs reach 2^27 and round)
+                const float down = *(const float*)(sb + GX::kTok * m);
+                acc[m] = __builtin_fmaf(ds * __builtin_fmaf(hi, 65536.0f, lo), down, acc[m]);
+            }
         }
     };
 
@@ -554,23 +547,29 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
             // get_scale_min_k4 of the eight sub-blocks, four bytes at a time
             const uint32_t sc4[2] = {s0w & 0x3f3f3f3fu, (s2w & 0x0f0f0f0fu) | ((s0w >> 2) & 0x30303030u)};
             const uint32_t mn4[2] = {s1w & 0x3f3f3f3fu, ((s2w >> 4) & 0x0f0f0f0fu) | ((s1w >> 2) & 0x30303030u)};
+            float ds[8], dm[8], c[8];
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                ds[b] = dd * (float)((sc4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
+                dm[b] = dmin * (float)((mn4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
+                // (any c from 0 to 15 gives the same sum: a ds of 0 may take either end)
+                c[b] = (float)(uint32_t)__builtin_amdgcn_fmed3f(
+                    __builtin_fmaf(dm[b], __builtin_amdgcn_rcpf(ds[b]), 0.5f), 0.0f, 15.5f);
+                dm[b] = __builtin_fmaf(-c[b], ds[b], dm[b]);
+            }
 #pragma unroll
             for (int q = 0; q < 4; q++) {  // sub-blocks 2q (low nibbles) and 2q + 1 (high)
                 __builtin_amdgcn_sched_barrier(0);  // one quarter's operands at a time
                 const u32x4 qa = *(const u32x4*)(wl + 16u + 32u * q), qb = *(const u32x4*)(wl + 32u + 32u * q);
                 const u32x4 m4 = {0x0f0f0f0fu, 0x0f0f0f0fu, 0x0f0f0f0fu, 0x0f0f0f0fu};
                 i32x4 lo[P], hi[P];
-                begin(lo, sb + (2u * q) * GX::kSubBytes);
-                begin(hi, sb + (2u * q + 1u) * GX::kSubBytes);
+#pragma unroll
+                for (int p = 0; p < P; p++) lo[p] = hi[p] = i32x4{0, 0, 0, 0};
                 mul16(lo, xb + (4u * q) * (64u * T), qa & m4, hi, xb + (4u * q + 2u) * (64u * T), (qa >> 4) & m4);
                 mul16(lo, xb + (4u * q + 1u) * (64u * T), qb & m4, hi, xb + (4u * q + 3u) * (64u * T), (qb >> 4) & m4);
 #pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const uint32_t b = 2u * q + e;
-                    const float ds = dd * (float)((sc4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
-                    const float dm = dmin * (float)((mn4[b >> 2] >> (8u * (b & 3u))) & 0xffu);
-                    add(e ? hi : lo, sb + b * GX::kSubBytes, ds, __builtin_fmaf(-8.0f, ds, dm));
-                }
+                for (int e = 0; e < 2; e++)
+                    add(e ? hi : lo, sb + (2u * q + e) * GX::kSubBytes, ds[2 * q + e], dm[2 * q + e], c[2 * q + e]);
             }
         } else {
             // four blocks of 34 bytes: block b's scale at byte 34 b, its quants two bytes on
@@ -592,15 +591,15 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
                     q2[i] = wd[dw + 9 + i];
                 }
                 i32x4 t[P], t2[P];
-                begin(t, sb);
-                begin(t2, sb);
+#pragma unroll
+                for (int p = 0; p < P; p++) t[p] = t2[p] = i32x4{0, 0, 0, 0};
 #pragma unroll
                 for (int h = 0; h < 2; h++)
                     mul16(t, xb + (2u * b + h) * (64u * T), u32x4{q[4 * h], q[4 * h + 1], q[4 * h + 2], q[4 * h + 3]},
                           t2, xb + (2u * b + 2u + h) * (64u * T),
                           u32x4{q2[4 * h], q2[4 * h + 1], q2[4 * h + 2], q2[4 * h + 3]});
-                add(t, sb + b * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw] & 0xffffu) : 0.0f, 0.0f);
-                add(t2, sb + (b + 1) * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw + 8] >> 16) : 0.0f, 0.0f);
+                add(t, sb + b * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw] & 0xffffu) : 0.0f, 0.0f, 0.0f);
+                add(t2, sb + (b + 1) * GX::kSubBytes, live ? f16_bits_to_f32(wd[dw + 8] >> 16) : 0.0f, 0.0f, 0.0f);
             }
         }
     }

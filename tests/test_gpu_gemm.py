@@ -124,6 +124,50 @@ def test_gemv_against_64_bits(dev, wtype, M, N, K, xtype, row_offset):
         assert err < 1e-6
 
 
+def _weights_zero_at(dev, wtype, rows, K, at, seed):
+    """Random raw blocks whose element `at` of every 32 is exactly zero (Q4_K: with all mins zero)."""
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(seed)
+    if wtype == 12:
+        b = torch.randint(0, 256, (rows, K // 256, 144), generator=g, dtype=torch.uint8)
+        b[..., 0:2] = (torch.rand(rows, K // 256, 1, generator=g) * 2e-4 + 1e-4).half().view(torch.uint8)
+        b[..., 2:4] = (torch.rand(rows, K // 256, 1, generator=g) * 2e-4 + 1e-4).half().view(torch.uint8)
+        b[..., 8:12] = 0     # mins 0-3 and the top bits of mins 4-7
+        b[..., 12:16] &= 15  # the low bits of mins 4-7
+        b[..., 16 + at::32] = 0
+    else:
+        b = torch.randint(0, 256, (rows, K // 32, 34), generator=g, dtype=torch.uint8)
+        b[..., 0:2] = (torch.rand(rows, K // 32, 1, generator=g) * 2e-4 + 1e-4).half().view(torch.uint8)
+        b[..., 2 + at] = 0
+    return b.reshape(-1).to(dev)
+
+
+def _gemv_worst_token(dev, w, wtype, x, N):
+    """Worst token's relative L2 against float64 of the dequantized weight."""
+    from llmr_amd import ops
+    K = x.shape[1]
+    y = ops.batch_matmul(w, wtype, x, N)
+    ref = x.double() @ ops.dequant(w, wtype, N, K).double().t()
+    return float(((y - ref).norm(dim=1) / ref.norm(dim=1)).max())
+
+
+@pytest.mark.parametrize("M,N,K,xtype", [(1, 8256, 2304, 0), (1, 100, 3072, 30), (2, 77, 3072, 0), (4, 130, 1280, 1)])
+def test_gemv_activation_under_a_zero_weight(dev, M, N, K, xtype):
+    """An activation 300 times the others of its sub-block, under weights that
+    are exactly zero (Q4_K quant 0, min 0): it is in no term, so the error stays
+    that of the f32 additions over the sub-blocks, K / 32 / 4 a lane at 2^-24 each
+    and random signs: below 2^-24 sqrt(24) = 3e-7 (1.1e-7; where the large
+    activation enters two terms that cancel, 2e-6)."""
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(M + N)
+    x = (torch.rand(M, K, generator=g) + 0.5) * torch.where(torch.rand(M, K, generator=g) < 0.5, -1.0, 1.0)
+    x[:, 5::32] *= 300
+    x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
+    err = _gemv_worst_token(dev, _weights_zero_at(dev, 12, N, K, 5, M), 12, x, N)
+    print(f"gemv zero weight M={M} N={N} K={K}: {err:.2e}")
+    assert err < 3e-7
+
+
 @pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", [
     (8, 3, 70, 512, 0, 0),         # the waves share 16 rows: six of the last workgroup's
     (12, 3, 70, 512, 0, 0),
