@@ -159,8 +159,15 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
 //    the weights times x, and a zero weight's activation is in neither: one 300
 //    times the rest of its sub-block leaves 0.9-2.1e-7 (8 for every c: 2-7e-6).
 // That is at least as exact as f32 FMAs on f32 activations (18432 x 3072: 1.4e-7
-// relative to 64 bits, the FMA kernel 2.5e-7). An infinite or NaN activation has
-// no digits: such a workgroup multiplies in f32 (gemv_f32_rows).
+// relative to 64 bits, the FMA kernel 2.5e-7), as long as the digits hold what is
+// multiplied. Where they do not, a workgroup multiplies in f32 (gemv_f32_rows): an
+// infinite or NaN activation; a quarter or more of a sub-block's values, other
+// than zeros, below 2^20 units of the digits (2^9 to 2^10 under the largest: f32
+// values, that keep 20 bits there; f16 and bf16 are whole down to 2^10 and 2^7
+// units); a sub-block under 2^-97, for which no scale is a normal number. With an
+// activation 2^k times the rest of its sub-block under a zero weight the digits'
+// error was, for k = 8, 10, 12 and 20, 1.1e-7, 3.5e-7, 9.6e-7 and 7.7e-4, the
+// FMAs' 0.9e-7; with activations of 1e-33 2.8e-6 and 1.8e-7.
 // A wave owns 16 weight rows and walks them 4 units at a time: lane l = 16 rq +
 // 4 g + j has row 4 rq + j and unit g, so the four lanes of an MFMA block share
 // a unit. One token: the block's four rows of A are the token's digits; two to
@@ -351,7 +358,7 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t* const wsb = smem + nu4 * GX::kUnit;
     uint8_t* const ws = wsb + wave * GW::kStep;           // the wave's weight bytes of a step
-    uint32_t* const odd = (uint32_t*)(wsb + 4u * GW::kStep);  // an activation is infinite or NaN
+    uint32_t* const odd = (uint32_t*)(wsb + 4u * GW::kStep);  // the activations have no digits: f32 rows
     if (tid == 0) *odd = 0u;
 
     // activations: thread -> 8 k of one token, four neighbours a sub-block; the
@@ -402,6 +409,7 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     __syncthreads();  // odd is cleared
 
     bool bad = false;
+    constexpr float kLow = XT == kGgmlF32 ? 0x1p20f : XT == kGgmlF16 ? 0x1p10f : 0x1p7f;
     auto stage_x = [&](uint32_t i, const X8& v) __attribute__((always_inline)) {
         const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
         float mx = 0.0f, sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
@@ -420,6 +428,7 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         const float up = __uint_as_float((uint32_t)(127 + e) << 23), down = __uint_as_float((uint32_t)(127 - e) << 23);
         uint32_t dg[2][4];  // [four k][digit, lowest first]: a byte per k
         int sums[4] = {0, 0, 0, 0};
+        uint32_t low = 0u;  // values whose digits hold too few of their bits
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             uint32_t v4[4];
@@ -427,7 +436,9 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
             for (int q = 0; q < 4; q++) {
                 // |v| < 2^30 + 1: adding 0x808080 and flipping those bits turns the
                 // three low bytes into signed digits (the carries go up)
-                const int i32 = (int)rintf(x[4 * h + q] * up);
+                const float y = x[4 * h + q] * up;
+                const int i32 = (int)rintf(y);
+                low += x[4 * h + q] != 0.0f && __builtin_fabsf(y) < kLow ? 1u : 0u;
                 v4[q] = ((uint32_t)i32 + 0x00808080u) ^ 0x00808080u;
             }
             // 4 x 4 byte transpose
@@ -443,6 +454,9 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 #pragma unroll
                 for (int p = 0; p < 4; p++) sums[p] = __builtin_amdgcn_sdot4((int)dg[h][p], 0x01010101, sums[p], false);
         }
+        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0xb1, 15, 15, false);  // lane ^ 1
+        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4e, 15, 15, false);  // lane ^ 2
+        bad = bad || low >= 8u || (mx > 0.0f && mx < 0x1p-97f);
         if constexpr (WT == kGgmlQ4K)
 #pragma unroll
             for (int p = 0; p < 4; p++) {

@@ -168,6 +168,33 @@ def test_gemv_activation_under_a_zero_weight(dev, M, N, K, xtype):
     assert err < 3e-7
 
 
+@pytest.mark.parametrize("wtype", [8, 12])
+@pytest.mark.parametrize("M,N,K,xtype,outliers,scale", [
+    (1, 8256, 1024, 0, 1e6, 1.0),     # one in 32 above, 31 with few digits' bits
+    (1, 100, 3072, 0, 700.0, 1.0),    # little past the line
+    (3, 130, 1280, 0, 1e20, 1.0),
+    (2, 77, 768, 1, 4e4, 1e-2),
+    (2, 77, 768, 30, 1e8, 1.0),
+    (1, 8256, 256, 0, 1.0, 1e-33),    # too small for a scale
+    (4, 60, 512, 0, 1.0, 1e-36),
+])
+def test_gemv_activations_out_of_the_digits_range(dev, wtype, M, N, K, xtype, outliers, scale):
+    """Activations that four int8 digits under their sub-block's largest do not
+    hold, the largest under weights that are exactly zero, and activations near
+    the smallest normal numbers: the error is that of f32 additions, K / 16 a lane
+    at 2^-24 each and random signs: 2^-24 sqrt(192) = 8e-7 at most. (The last
+    token, within the digits' range, stays as exact beside them.)"""
+    import torch
+    g = torch.Generator(device="cpu").manual_seed(M + N)
+    x = (torch.rand(M, K, generator=g) + 0.5) * torch.where(torch.rand(M, K, generator=g) < 0.5, -1.0, 1.0) * scale
+    x[:max(1, M - 1), 5::32] *= outliers / scale if xtype == 1 else outliers
+    x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
+    assert bool(torch.isfinite(x).all())
+    err = _gemv_worst_token(dev, _weights_zero_at(dev, wtype, N, K, 5, M), wtype, x, N)
+    print(f"gemv out of range wtype={wtype} M={M} N={N} K={K}: {err:.2e}")
+    assert err < 8e-7
+
+
 @pytest.mark.parametrize("wtype,M,N,K,xtype,row_offset", [
     (8, 3, 70, 512, 0, 0),         # the waves share 16 rows: six of the last workgroup's
     (12, 3, 70, 512, 0, 0),
