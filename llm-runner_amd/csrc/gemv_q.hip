@@ -161,13 +161,14 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
 // That is at least as exact as f32 FMAs on f32 activations (18432 x 3072: 1.4e-7
 // relative to 64 bits, the FMA kernel 2.5e-7), as long as the digits hold what is
 // multiplied. Where they do not, a workgroup multiplies in f32 (gemv_f32_rows): an
-// infinite or NaN activation; a quarter or more of a sub-block's values, other
-// than zeros, below 2^20 units of the digits (2^9 to 2^10 under the largest: f32
-// values, that keep 20 bits there; f16 and bf16 are whole down to 2^10 and 2^7
-// units); a sub-block under 2^-97, for which no scale is a normal number. With an
+// infinite or NaN activation; f16 and bf16 values, other than zeros, that are not
+// whole (below 2^10 and 2^7 units of the digits); f32 values below 2^20 units, 2^9
+// to 2^10 under their sub-block's largest, that fill a quarter of it, or one below
+// 2^8; a sub-block under 2^-97, for which no scale is a normal number. With an
 // activation 2^k times the rest of its sub-block under a zero weight the digits'
-// error was, for k = 8, 10, 12 and 20, 1.1e-7, 3.5e-7, 9.6e-7 and 7.7e-4, the
-// FMAs' 0.9e-7; with activations of 1e-33 2.8e-6 and 1.8e-7.
+// error is, for k = 8, 10, 12 and 20, 1.1e-7, 3.5e-7, 9.6e-7 and 7.7e-4, the
+// FMAs' 0.9e-7; with activations of 1e-33 2.8e-6 and 1.8e-7. (Of 3072 normal
+// deviates one lies below 2^8 units in 1 of 500 draws.)
 // A wave owns 16 weight rows and walks them 4 units at a time: lane l = 16 rq +
 // 4 g + j has row 4 rq + j and unit g, so the four lanes of an MFMA block share
 // a unit. One token: the block's four rows of A are the token's digits; two to
@@ -410,14 +411,13 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 
     bool bad = false;
     constexpr float kLow = XT == kGgmlF32 ? 0x1p20f : XT == kGgmlF16 ? 0x1p10f : 0x1p7f;
+    constexpr float kTiny = XT == kGgmlF32 ? 0x1p8f : kLow;
     auto stage_x = [&](uint32_t i, const X8& v) __attribute__((always_inline)) {
         const float x[8] = {v.a.x, v.a.y, v.a.z, v.a.w, v.b.x, v.b.y, v.b.z, v.b.w};
         float mx = 0.0f, sum = ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+        bad = bad || !(__builtin_fabsf(sum) < INFINITY);  // (sums that overflow: the f32 rows too)
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            bad = bad || !(__builtin_fabsf(x[e]) < INFINITY);
-            mx = fmaxf(mx, __builtin_fabsf(x[e]));
-        }
+        for (int e = 0; e < 8; e++) mx = fmaxf(mx, __builtin_fabsf(x[e]));
 #pragma unroll
         for (int o = 1; o < 4; o <<= 1) {
             mx = fmaxf(mx, __shfl_xor(mx, o, 64));
@@ -426,9 +426,21 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         // scale 2^e with 2^e mx in [2^29, 2^30), e kept where 2^e and 2^-e are normal
         const int e = min(126, max(-126, 156 - (int)((__float_as_uint(mx) >> 23) & 0xffu)));
         const float up = __uint_as_float((uint32_t)(127 + e) << 23), down = __uint_as_float((uint32_t)(127 - e) << 23);
+        // values whose digits hold too few of their bits, zeros aside (magnitude
+        // bits less one: a zero's are the largest)
+        const uint32_t low_bits = 2u * __float_as_uint(kLow * down) - 1u;
+        uint32_t low = 0u, least = ~0u;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            const uint32_t b = 2u * __float_as_uint(x[q]) - 1u;
+            low += b < low_bits ? 1u : 0u;
+            least = min(least, b);
+        }
+        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0xb1, 15, 15, false);  // lane ^ 1
+        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4e, 15, 15, false);  // lane ^ 2
+        bad = bad || low >= 8u || least < 2u * __float_as_uint(kTiny * down) - 1u || (mx > 0.0f && mx < 0x1p-97f);
         uint32_t dg[2][4];  // [four k][digit, lowest first]: a byte per k
         int sums[4] = {0, 0, 0, 0};
-        uint32_t low = 0u;  // values whose digits hold too few of their bits
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             uint32_t v4[4];
@@ -436,9 +448,7 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
             for (int q = 0; q < 4; q++) {
                 // |v| < 2^30 + 1: adding 0x808080 and flipping those bits turns the
                 // three low bytes into signed digits (the carries go up)
-                const float y = x[4 * h + q] * up;
-                const int i32 = (int)rintf(y);
-                low += x[4 * h + q] != 0.0f && __builtin_fabsf(y) < kLow ? 1u : 0u;
+                const int i32 = (int)rintf(x[4 * h + q] * up);
                 v4[q] = ((uint32_t)i32 + 0x00808080u) ^ 0x00808080u;
             }
             // 4 x 4 byte transpose
@@ -454,9 +464,6 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 #pragma unroll
                 for (int p = 0; p < 4; p++) sums[p] = __builtin_amdgcn_sdot4((int)dg[h][p], 0x01010101, sums[p], false);
         }
-        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0xb1, 15, 15, false);  // lane ^ 1
-        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4e, 15, 15, false);  // lane ^ 2
-        bad = bad || low >= 8u || (mx > 0.0f && mx < 0x1p-97f);
         if constexpr (WT == kGgmlQ4K)
 #pragma unroll
             for (int p = 0; p < 4; p++) {

@@ -125,7 +125,7 @@ def test_gemv_against_64_bits(dev, wtype, M, N, K, xtype, row_offset):
 
 
 def _weights_zero_at(dev, wtype, rows, K, at, seed):
-    """Random raw blocks whose element `at` of every 32 is exactly zero (Q4_K: with all mins zero)."""
+    """Random raw blocks whose elements `at` of every 32 are exactly zero (Q4_K: with all mins zero)."""
     import torch
     g = torch.Generator(device="cpu").manual_seed(seed)
     if wtype == 12:
@@ -134,11 +134,13 @@ def _weights_zero_at(dev, wtype, rows, K, at, seed):
         b[..., 2:4] = (torch.rand(rows, K // 256, 1, generator=g) * 2e-4 + 1e-4).half().view(torch.uint8)
         b[..., 8:12] = 0     # mins 0-3 and the top bits of mins 4-7
         b[..., 12:16] &= 15  # the low bits of mins 4-7
-        b[..., 16 + at::32] = 0
+        for i in at:
+            b[..., 16 + i::32] = 0
     else:
         b = torch.randint(0, 256, (rows, K // 32, 34), generator=g, dtype=torch.uint8)
         b[..., 0:2] = (torch.rand(rows, K // 32, 1, generator=g) * 2e-4 + 1e-4).half().view(torch.uint8)
-        b[..., 2 + at] = 0
+        for i in at:
+            b[..., 2 + i] = 0
     return b.reshape(-1).to(dev)
 
 
@@ -163,7 +165,7 @@ def test_gemv_activation_under_a_zero_weight(dev, M, N, K, xtype):
     x = (torch.rand(M, K, generator=g) + 0.5) * torch.where(torch.rand(M, K, generator=g) < 0.5, -1.0, 1.0)
     x[:, 5::32] *= 300
     x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
-    err = _gemv_worst_token(dev, _weights_zero_at(dev, 12, N, K, 5, M), 12, x, N)
+    err = _gemv_worst_token(dev, _weights_zero_at(dev, 12, N, K, [5], M), 12, x, N)
     print(f"gemv zero weight M={M} N={N} K={K}: {err:.2e}")
     assert err < 3e-7
 
@@ -173,6 +175,8 @@ def test_gemv_activation_under_a_zero_weight(dev, M, N, K, xtype):
     (1, 8256, 1024, 0, 1e6, 1.0),     # one in 32 above, 31 with few digits' bits
     (1, 100, 3072, 0, 700.0, 1.0),    # little past the line
     (3, 130, 1280, 0, 1e20, 1.0),
+    (1, 8200, 512, 0, -1e20, 1.0),    # all but one in 32 above
+    (2, 77, 768, 1, -4e4, 1e-2),
     (2, 77, 768, 1, 4e4, 1e-2),
     (2, 77, 768, 30, 1e8, 1.0),
     (1, 8256, 256, 0, 1.0, 1e-33),    # too small for a scale
@@ -187,10 +191,14 @@ def test_gemv_activations_out_of_the_digits_range(dev, wtype, M, N, K, xtype, ou
     import torch
     g = torch.Generator(device="cpu").manual_seed(M + N)
     x = (torch.rand(M, K, generator=g) + 0.5) * torch.where(torch.rand(M, K, generator=g) < 0.5, -1.0, 1.0) * scale
-    x[:max(1, M - 1), 5::32] *= outliers / scale if xtype == 1 else outliers
+    at, big = [5], abs(outliers) / (scale if xtype == 1 else 1.0)
+    if outliers < 0:
+        at = [i for i in range(32) if i != 9]
+    for i in at:
+        x[:max(1, M - 1), i::32] *= big
     x = (x if xtype == 0 else x.to(torch.float16 if xtype == 1 else torch.bfloat16)).to(dev)
     assert bool(torch.isfinite(x).all())
-    err = _gemv_worst_token(dev, _weights_zero_at(dev, wtype, N, K, 5, M), wtype, x, N)
+    err = _gemv_worst_token(dev, _weights_zero_at(dev, wtype, N, K, at, M), wtype, x, N)
     print(f"gemv out of range wtype={wtype} M={M} N={N} K={K}: {err:.2e}")
     assert err < 8e-7
 
