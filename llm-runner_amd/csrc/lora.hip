@@ -309,8 +309,10 @@ __global__ void __launch_bounds__(256) lora_up_kernel(const float* __restrict__ 
 // thread gi owns output column o0 + gi, whose B row stays in registers (a chunk
 // at a time) for the workgroup's T tokens; their scratch rows are the same for
 // the whole wave, so they come as scalar loads and are scalar operands of the
-// FMAs, and all the output values are requested before the first sum (rows past
-// seq_len read zero and are not stored: the buffer ends there). Same arithmetic
+// FMAs, and all the output values are requested before the first sum. The buffer
+// ends at seq_len: rows past it read zero and are not stored. Their offset is the
+// lane's, which the range check covers on its own (whether it covers a scalar
+// offset past the buffer's end is not documented). Same arithmetic
 // as lora_up_kernel: the sum over ranks in rank order from 0, then y + scale *
 // sum. What bounds it is the output's read and write. With the scratch rows
 // through LDS (a broadcast read per 4 FMAs is as slow as they are), 16 tokens at
@@ -332,7 +334,7 @@ __global__ void __launch_bounds__(256) lora_up_reg_kernel(const float* __restric
     float yv[T];
 #pragma unroll
     for (uint32_t t = 0; t < T; t++)
-        yv[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yr, yo, t * out_dim * 4u, 0));
+        yv[t] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(yr, yo + t * out_dim * 4u, 0, 0));
     const uint32_t ld = CHUNKS ? rank : R;
     const float* const brow = B + (uint64_t)(weight_row_offset + min(o, b_rows - 1u)) * ld;
     float bv[R];
@@ -353,7 +355,7 @@ __global__ void __launch_bounds__(256) lora_up_reg_kernel(const float* __restric
         return a;
     };
     auto store = [&](uint32_t t, float a) __attribute__((always_inline)) {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(yv[t] + scale * a), yr, yo, t * out_dim * 4u, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(yv[t] + scale * a), yr, yo + t * out_dim * 4u, 0, 0);
     };
     if constexpr (!CHUNKS) {
         load_b(0);

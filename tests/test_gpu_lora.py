@@ -24,6 +24,14 @@ def _act(x_f32, xtype, dev):
     return t.to(dev)
 
 
+def _guarded(y0, dev):
+    """y0 on the device with 64 rows of 7.0 after it: (the output, those rows)."""
+    import torch
+    buf = torch.full((y0.shape[0] + 64, y0.shape[1]), 7.0, device=dev)
+    buf[:y0.shape[0]] = torch.from_numpy(y0).to(dev)
+    return buf[:y0.shape[0]], buf[y0.shape[0]:]
+
+
 @pytest.mark.parametrize("seq,in_dim,rank,out_dim,b_rows,row_off,w_off,xtype", [
     (37, 512, 8, 300, 200, 50, 30, 0),      # f32 input, sub-range of a wider output
     (64, 3072, 32, 3072, 0, 0, 0, 30),      # Flux dim, bf16 input, whole output
@@ -42,7 +50,7 @@ def test_lora_correction_bit_exact(orc, dev, seq, in_dim, rank, out_dim, b_rows,
     x = r.standard_normal((seq, in_dim)).astype(np.float32)
     xt = _act(x, xtype, dev)
     y0 = r.standard_normal((seq, out_dim)).astype(np.float32)
-    y = torch.from_numpy(y0).to(dev)
+    y, after = _guarded(y0, dev)
     scratch = torch.empty(seq * rank, device=dev)
     g = ops.default_graph()
     ops.dispatch_lora_correction(g, lora, scratch, ops.Tensor.from_torch(xt), ops.Tensor.from_torch(y), in_dim,
@@ -53,6 +61,7 @@ def test_lora_correction_bit_exact(orc, dev, seq, in_dim, rank, out_dim, b_rows,
     np.testing.assert_array_equal(scratch.cpu().numpy().reshape(seq, rank), s_ref)
     y_ref = orc.lora_up(B, s_ref, y0, 0.8, row_offset=row_off, weight_row_offset=w_off, b_rows=rows)
     np.testing.assert_array_equal(y.cpu().numpy(), y_ref)
+    assert bool((after == 7.0).all())
 
 
 @pytest.mark.parametrize("seq,in_dim,rank,out_dim,xtype,shift", [
@@ -74,7 +83,7 @@ def test_lora_correction_edges_bit_exact(orc, dev, seq, in_dim, rank, out_dim, x
     flat = _act(np.concatenate([np.zeros(shift, np.float32), x.ravel()]), xtype, dev)
     xt = flat[shift:].view(seq, in_dim)
     y0 = r.standard_normal((seq, out_dim)).astype(np.float32)
-    y = torch.from_numpy(y0).to(dev)
+    y, after = _guarded(y0, dev)
     scratch = torch.empty(seq * rank, device=dev)
     ops.dispatch_lora_correction(ops.default_graph(), lora, scratch, ops.Tensor.from_torch(xt),
                                  ops.Tensor.from_torch(y), in_dim, out_dim, seq)
@@ -82,6 +91,7 @@ def test_lora_correction_edges_bit_exact(orc, dev, seq, in_dim, rank, out_dim, x
     s_ref = orc.lora_down(A, xt.float().cpu().numpy())
     np.testing.assert_array_equal(scratch.cpu().numpy().reshape(seq, rank), s_ref)
     np.testing.assert_array_equal(y.cpu().numpy(), orc.lora_up(B, s_ref, y0, 0.7))
+    assert bool((after == 7.0).all())
 
 
 def test_batch_matmul_with_lora_equals_base_plus_correction(orc, dev):
