@@ -396,13 +396,16 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     struct Set {
         u32x4 v[GW::kLoads];
     };
-    // (the last step may read into the next row: those units are masked below)
+    // (the last step may read into the next row: those units are masked below; past
+    // the last row the buffer ends. The step's offset is in the descriptor, not a
+    // scalar offset, which the range check need not cover)
     auto load_w = [&](uint32_t s) __attribute__((always_inline)) {
         Set w;
-        const rsrc_t r = make_rsrc(W + (uint64_t)n0 * rb, s < steps ? wbytes : 0u);
+        const uint32_t at = 4u * GW::kBytes * s;
+        const rsrc_t r = make_rsrc(W + (uint64_t)n0 * rb + at, s < steps && at < wbytes ? wbytes - at : 0u);
 #pragma unroll
         for (uint32_t i = 0; i < GW::kLoads; i++)
-            w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i], 4u * GW::kBytes * s, 0));
+            w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i], 0, 0));
         return w;
     };
     const uint32_t s0 = wave % KS;
