@@ -90,11 +90,14 @@ inline size_t skinny_x_bytes(uint32_t xtype, uint32_t M, uint32_t K) {
 // The 4-wave tiled kernel's tile (64, 128 or 256 square) and K splits: the
 // largest tile that still gives every CU ~1.5 workgroups; launches with fewer
 // workgroups than kSplitWgsPerCu per CU split K (at least kSplitMinStages
-// stages per split, M * N % 4 == 0 for the reduction).
+// stages per split, M * N % 4 == 0 for the reduction, partials within ws_limit:
+// as many as fit, none if fewer than two).
+constexpr size_t kNoWorkspaceLimit = ~(size_t)0;
 struct TilePlan {
     uint32_t bm, splits;
 };
-inline TilePlan plan_tiles(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+inline TilePlan plan_tiles(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
+                           size_t ws_limit = kNoWorkspaceLimit) {
     auto wgs = [&](uint32_t bm) { return (uint64_t)((M + bm - 1) / bm) * ((N + bm - 1) / bm); };
     const uint64_t want = (uint64_t)num_cus * 3 / 2;
     TilePlan t{64, 1};
@@ -105,6 +108,8 @@ inline TilePlan plan_tiles(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, i
     const uint32_t S = K / kStageK;
     if (w < target && S >= 2 * kSplitMinStages && ((uint64_t)M * N) % 4 == 0)
         t.splits = nonempty_splits(S, (uint32_t)std::min<uint64_t>((target + w - 1) / w, S / kSplitMinStages));
+    const size_t fit = ws_limit / ((size_t)M * N * sizeof(float));
+    if (t.splits > fit) t.splits = fit >= 2 ? nonempty_splits(S, (uint32_t)fit) : 1u;
     return t;
 }
 
@@ -146,8 +151,9 @@ inline double few_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uin
 }
 // Time in us of the tiled kernel: two of its workgroups per CU run at full
 // speed, its 64 x 64 tiles four at a time (three with f32 activations).
-inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
-    const TilePlan t = plan_tiles(wtype, N, K, M, num_cus);
+inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
+                       size_t ws_limit) {
+    const TilePlan t = plan_tiles(wtype, N, K, M, num_cus, ws_limit);
     const double wgs = (double)((M + t.bm - 1) / t.bm) * ((N + t.bm - 1) / t.bm) * t.splits, c = (double)num_cus;
     const double rounds = wgs <= 2 * c ? 1.0 : wgs <= (xtype == kF32 ? 3 : 4) * c ? 1.8 : std::max(3.1, 0.55 * wgs / c);
     const double per_k = (t.bm == 64 ? 1.0 : t.bm == 128 ? 2.8 : 8.0) * (wtype == kQ8_0 ? 0.0105 : 0.0090);
@@ -177,20 +183,23 @@ constexpr uint32_t kSplitMax = 16;
 constexpr uint32_t kSplitTileMinStages = 16;
 struct SplitPlan {
     uint32_t full, splits;  // splits 1: no split
+    size_t x16;             // bytes of f32 activations rounded to 16 bits, before the partial tiles
     double us;              // of the launch, split or whole
+    size_t ws(uint64_t tiles) const { return x16 + (size_t)(tiles - full) * splits * kPartTile; }
 };
-inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus, bool persistent) {
+inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
+                            bool persistent, size_t ws_limit) {
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
     const uint32_t S = K / kStageK;
     const uint64_t full = tiles / num_cus * num_cus, rem = tiles - full;
-    SplitPlan p{(uint32_t)full, 1, 0.0};
+    SplitPlan p{(uint32_t)full, 1, xtype == kF32 ? align256((size_t)M * K * 2u) : 0u, 0.0};
     const double whole = persistent
                              ? (double)((tiles + num_cus - 1) / num_cus) * S * (wtype == kQ8_0 ? 1.93 : 1.7) + 6.0
-                             : tiled_us(wtype, xtype, N, K, M, num_cus);
+                             : tiled_us(wtype, xtype, N, K, M, num_cus, ws_limit);
     p.us = whole;
     double best = 0.97 * whole;
     for (uint32_t s = 2; rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
-        if (nonempty_splits(S, s) != s) continue;
+        if (nonempty_splits(S, s) != s || p.x16 + (size_t)rem * s * kPartTile > ws_limit) continue;
         const double rounds = (double)((rem * s + num_cus - 1) / num_cus);
         const double us = (double)(full / num_cus) * (S * 2.0 + 8.0) + rounds * ((S + s - 1) / s * 2.0 + 8.0) + 3.0 +
                           (double)rem * kPartTile * (s + 1) / 5e6;
@@ -215,9 +224,11 @@ inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t
 //  * otherwise the tiled kernel, split-K partials in the workspace.
 // With a workspace limit (the no-allocation entry point's fixed array) the
 // plan keeps within it: the two-pass path only when its image fits, as many
-// splits as fit (none if fewer than two), and the tiled kernel (which reads
-// f32 activations in place) when the 16-bit copy of f32 activations for the
-// persistent kernels does not fit.
+// splits as fit (none if fewer than two), and the kernels that read f32
+// activations in place (tiled, few-token) when the 16-bit copy of f32
+// activations for the others does not fit. The estimates are of what fits: with
+// 32 MiB, 323 x 3072 x 15360 Q8_0 f16 ran the tiled kernel, 1.5 times the
+// few-token kernel's time, as the split it was compared with did not fit.
 struct GemmPlan {
     bool persistent, two_pass, convert_x, skinny, few;
     uint32_t xt;                  // activation type the kernel reads
@@ -228,8 +239,6 @@ struct GemmPlan {
     size_t x16_off, img_off, ws;  // workspace: [x16 | image] (persistent), [packed x | partials]
                                   // (skinny), split-K partials (tiled)
 };
-constexpr size_t kNoWorkspaceLimit = ~(size_t)0;
-
 inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
                           size_t ws_limit = kNoWorkspaceLimit) {
     GemmPlan p{};
@@ -240,7 +249,8 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
     const uint64_t rb = row_bytes_of(wtype, K);
     const bool offsets31 = (uint64_t)M * K * 2u < (1ull << 31) && (uint64_t)N * rb < (1ull << 31);
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
-    p.persistent = K % kStageK == 0 && N % 4 == 0 && 2 * tiles >= (uint64_t)num_cus && offsets31;
+    p.persistent = K % kStageK == 0 && N % 4 == 0 && 2 * tiles >= (uint64_t)num_cus && offsets31 &&
+                   (xtype != kF32 || align256((size_t)M * K * 2u) <= ws_limit);
     const bool few_ok = !p.persistent && few_fits(wtype, N, K, M);
     if (few_ok && M <= kSkinnyMaxTokens) {
         p.few_features = few_features(xtype, N, K, M, num_cus);
@@ -268,35 +278,26 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
         }
     }
     if (K % kStageK == 0 && N % 4 == 0 && offsets31 && (M < kW16MinTokens || !p.persistent)) {
-        const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent);
+        const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent, ws_limit);
         if (few_ok && few_us(wtype, xtype, N, K, M, num_cus) < 0.97 * sp.us) {
             p.few = true;
             p.few_features = kFewNarrow;
             return p;
         }
-        const size_t x16 = xtype == kF32 ? align256((size_t)M * K * 2u) : 0u;
-        const size_t ws = x16 + (size_t)(tiles - sp.full) * sp.splits * kPartTile;
-        if (sp.splits > 1 && ws <= ws_limit) {
+        if (sp.splits > 1) {
             p.persistent = false;
             p.split = sp.splits;
             p.split_full = sp.full;
             p.convert_x = xtype == kF32;
             p.xt = operand_type(wtype, xtype);
-            p.img_off = x16;  // the partial tiles
-            p.ws = ws;
+            p.img_off = sp.x16;  // the partial tiles
+            p.ws = sp.ws(tiles);
             return p;
         }
     }
-    if (p.persistent && xtype == kF32 && align256((size_t)M * K * 2u) > ws_limit) p.persistent = false;
     if (!p.persistent) {
-        p.tiles = plan_tiles(wtype, N, K, M, num_cus);
-        const size_t part = (size_t)M * N * sizeof(float);
-        if (p.tiles.splits > 1 && (size_t)p.tiles.splits * part > ws_limit) {
-            const size_t fit = ws_limit / part;
-            p.tiles.splits = fit >= 2 ? nonempty_splits(K / kStageK, (uint32_t)std::min<size_t>(fit, p.tiles.splits))
-                                      : 1u;
-        }
-        p.ws = p.tiles.splits > 1 ? (size_t)p.tiles.splits * part : 0u;
+        p.tiles = plan_tiles(wtype, N, K, M, num_cus, ws_limit);
+        p.ws = p.tiles.splits > 1 ? (size_t)p.tiles.splits * M * N * sizeof(float) : 0u;
         return p;
     }
     p.convert_x = xtype == kF32;

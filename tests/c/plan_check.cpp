@@ -28,10 +28,12 @@ static void check(uint32_t wt, uint32_t xt, uint32_t N, uint32_t K, uint32_t M, 
     const GemmPlan p = plan_gemm(wt, xt, N, K, M, cus, limit);
     const uint32_t S = K / kStageK;
     n_checked++;
-    if (p.few + p.skinny + p.persistent > 1) fail("more than one kernel", wt, xt, N, K, M, cus, limit);
+    if (p.few + p.skinny + p.persistent + (p.split > 1) > 1) fail("more than one kernel", wt, xt, N, K, M, cus, limit);
     if (p.ws > limit) fail("workspace beyond the limit", wt, xt, N, K, M, cus, limit);
     if (p.few) {
         if (M > kFewMaxTokens || K % kStageK || p.ws != 0) fail("few-token plan", wt, xt, N, K, M, cus, limit);
+        if (p.few_features != kFewNarrow && p.few_features != kFewFeatures)
+            fail("few-token tile width", wt, xt, N, K, M, cus, limit);
         return;
     }
     if (p.skinny) {
@@ -46,6 +48,23 @@ static void check(uint32_t wt, uint32_t xt, uint32_t N, uint32_t K, uint32_t M, 
         if (p.two_pass && M < kW16MinTokens) fail("two-pass below its token count", wt, xt, N, K, M, cus, limit);
         return;
     }
+    if (p.split > 1) {
+        const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
+        if (!splits_nonempty(S, p.split)) fail("tile cut without stages", wt, xt, N, K, M, cus, limit);
+        if (p.split_full >= tiles || p.split_full % cus || tiles - p.split_full > (uint64_t)cus)
+            fail("tiles cut are not the last round's", wt, xt, N, K, M, cus, limit);
+        if (N % 4 || K % kStageK) fail("tile cut of a ragged launch", wt, xt, N, K, M, cus, limit);
+        const size_t x16 = xt == kF32 ? align256((size_t)M * K * 2) : 0;
+        if (p.convert_x != (xt == kF32) || p.xt != operand_type(wt, xt) || p.img_off != x16)
+            fail("tile cut's activations", wt, xt, N, K, M, cus, limit);
+        if (p.ws != x16 + (tiles - p.split_full) * p.split * kPartTile)
+            fail("tile cut's workspace", wt, xt, N, K, M, cus, limit);
+        return;
+    }
+    // the tiled kernel: where the few-token kernel could run instead, not by much the slower of the two
+    if (M > kSkinnyMaxTokens && few_fits(wt, N, K, M) && N % 4 == 0 &&
+        few_us(wt, xt, N, K, M, cus) < 0.8 * tiled_us(wt, xt, N, K, M, cus, limit))
+        fail("tiled in place of the few-token kernel", wt, xt, N, K, M, cus, limit);
     // the tiled kernel (or, Q8_0 with K % 64 == 32, the generic one: no splits)
     if (wt == kQ8_0 && K % kStageK) {
         if (p.tiles.splits != 1) fail("generic kernel split", wt, xt, N, K, M, cus, limit);
@@ -81,6 +100,16 @@ int main() {
     if (f32_operand_type(kQ8_0) != kF16 || f32_operand_type(kQ4K) != kBF16) {
         std::printf("FAIL f32 operand types\n");
         return 1;
+    }
+    // a limit that holds fewer parts than the launch is cut into without one
+    {
+        const GemmPlan a = plan_gemm(kQ8_0, kBF16, 3840, 3840, 1101, 256);
+        const GemmPlan b = plan_gemm(kQ8_0, kBF16, 3840, 3840, 1101, 256, (size_t)40 << 20);
+        n_checked++;
+        if (a.split != 3 || b.split != 2) {
+            std::printf("FAIL 1101 x 3840 x 3840: cut into %u, %u with 40 MiB\n", a.split, b.split);
+            return 1;
+        }
     }
     const uint32_t Ms[] = {1, 2, 4, 5, 17, 31, 32, 33, 64, 100, 200, 255, 256, 257, 320, 500, 512, 1000,
                            1024, 2047, 2048, 3000, 4096, 4352, 4608, 9000};
