@@ -143,32 +143,50 @@ inline uint32_t few_features(uint32_t xtype, uint32_t N, uint32_t K, uint32_t M,
     const double f = long_f32 ? 1.6 : xtype == kF32 ? 1.3 : 1.03;
     return f * narrow + 0.7 * c < 3.0 * c * ((wide + c - 1) / c) ? kFewNarrow : kFewFeatures;
 }
-// Time in us of the 32-feature tiles past kSkinnyMaxTokens tokens (300 x 3072
-// x 3072 Q4_K bf16: 960 tiles), for the choice against plan_split and the tiled kernel.
-inline double few_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
-    const double tiles = (double)((M + kFewTokens - 1) / kFewTokens) * ((N + kFewNarrow - 1) / kFewNarrow);
-    return 5.0 + (xtype == kF32 ? 7.0 : wtype == kQ8_0 ? 4.6 : 4.3) * K / 3072.0 * tiles / num_cus;
+// Time in us of the 32-feature tiles past kSkinnyMaxTokens tokens, for the choice
+// against plan_split and the tiled kernel: a wave's K / 512 stages one after
+// the other, or the tiles a CU has times their stages (with f32 activations a
+// second tile on a CU doubles the time), more past K = 8192, where the activation
+// rows leave the L2. Measured: 300 x 3072 x 3072 Q4_K bf16 19 us, 257 x 9216 x 256
+// Q8_0 12.6, 288 x 64 x 15360 f32 34.
+inline double few_us(uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
+    const bool f32 = xtype == kF32;
+    double q = (double)((M + kFewTokens - 1) / kFewTokens) * ((N + kFewNarrow - 1) / kFewNarrow) / num_cus;
+    if (f32 && q < 2.0) q = q <= 1.0 ? 1.0 : 2.0;
+    const double stages = K / 512.0, far = std::max(0.0, (K - 8192.0) / 4096.0), n = (K + 511) / 512;
+    const double tiles = 4.0 + q * (0.5 + (f32 ? 1.03 : 0.68) * std::max(stages, 0.5) + (f32 ? 7.7 : 3.2) * far);
+    return std::max({7.6, tiles, f32 ? 1.16 * n : 1.4 + 0.79 * n});
 }
 // Time in us of the tiled kernel: two of its workgroups per CU run at full
 // speed, its 64 x 64 tiles four at a time (three with f32 activations).
 inline double tiled_us(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
                        size_t ws_limit) {
     const TilePlan t = plan_tiles(wtype, N, K, M, num_cus, ws_limit);
+    const bool f32 = xtype == kF32;
     const double wgs = (double)((M + t.bm - 1) / t.bm) * ((N + t.bm - 1) / t.bm) * t.splits, c = (double)num_cus;
-    const double rounds = wgs <= 2 * c ? 1.0 : wgs <= (xtype == kF32 ? 3 : 4) * c ? 1.8 : std::max(3.1, 0.55 * wgs / c);
-    const double per_k = (t.bm == 64 ? 1.0 : t.bm == 128 ? 2.8 : 8.0) * (wtype == kQ8_0 ? 0.0105 : 0.0090);
+    const double rounds = wgs <= 2 * c ? 1.0 : wgs <= (f32 ? 3 : 4) * c ? 1.8 : std::max(3.1, 0.55 * wgs / c);
+    const double per_k = (t.bm == 64 ? 1.0 : t.bm == 128 ? 2.8 : 8.0) * (wtype == kQ8_0 ? 0.0105 : 0.0090) *
+                         (!f32 ? 1.0 : K < 8192 ? 1.05 : 1.26);
     return 6.0 + rounds * ((double)K / t.splits) * per_k;
+}
+// What its split-K sum (the output's stores where it has none) adds to that.
+inline double tiled_sum_us(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M, int num_cus, size_t ws_limit) {
+    const TilePlan t = plan_tiles(wtype, N, K, M, num_cus, ws_limit);
+    const double y = (double)M * N * sizeof(float) / 5e6;
+    return t.splits > 1 ? 3.0 + 0.25 * t.splits + y * (t.splits + 1) : 0.3 * y;
 }
 
 // Launches below kW16MinTokens tokens, or with too few tiles for the persistent
-// kernels, whose 256 x 256 tiles leave CUs idle in their last round: the whole rounds of tiles run as they are (`full` of
-// them) and every tile of the last round is cut along K into `splits`
-// workgroups, whose partial tiles a second launch adds up. The times are
-// estimates in us on MI355X (256 CUs), fitted to launches of 300-2000 tokens
-// x 3072-21504 features: a K stage of a tile takes 2.0 us on the 8-wave
-// kernel that also runs the splits (1.93 and 1.7 for Q8_0 and Q4_K where
-// tiles follow each other in the persistent kernels), a workgroup 8 us around
-// its stages, and the partial tiles are written and read at ~5 TB/s. Measured,
+// kernels, whose 256 x 256 tiles leave CUs idle in their last round: the whole
+// rounds of tiles run as they are (`full` of them) and every tile of the last
+// round is cut along K into `splits` workgroups, whose partial tiles a second
+// launch adds up. The times are estimates in us on MI355X (256 CUs), fitted to
+// 1500 launches of 257-9000 tokens x 64-21504 features: a K stage of a tile takes
+// 2.0 us on the 8-wave kernel that also runs the splits (1.93 and 1.7 for Q8_0 and
+// Q4_K where tiles follow each other in the persistent kernels, down to three
+// quarters of it where most CUs have none), a workgroup 8 us around its stages,
+// the partial tiles are written and read at ~5 TB/s, and f32 activations, which
+// the tiled kernel reads in place, are rounded by a launch of their own. Measured,
 // whole launch before -> after: 1101 x 3840 x 3840 Q8_0 (75 tiles x 3) 129 ->
 // 60 us, x 10240 348 -> 117; 520 x 9216 x 3072 Q4_K (108 x 2) 99 -> 60; 1536 x
 // 11520 x 3840 Q8_0 (256 whole tiles + 14 x 15) 236 -> 160; 2000 x 9216 x
@@ -194,15 +212,17 @@ inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t
     const uint64_t full = tiles / num_cus * num_cus, rem = tiles - full;
     SplitPlan p{(uint32_t)full, 1, xtype == kF32 ? align256((size_t)M * K * 2u) : 0u, 0.0};
     const double whole = persistent
-                             ? (double)((tiles + num_cus - 1) / num_cus) * S * (wtype == kQ8_0 ? 1.93 : 1.7) + 6.0
+                             ? (full == 0 ? 0.75 + 0.25 * rem / num_cus : (double)((tiles + num_cus - 1) / num_cus)) *
+                                       S * (wtype == kQ8_0 ? 1.93 : 1.7) + 6.0
                              : tiled_us(wtype, xtype, N, K, M, num_cus, ws_limit);
     p.us = whole;
     double best = 0.97 * whole;
+    const double round_x = xtype == kF32 && !persistent ? (double)M * K * 6.0 / 8e6 : 0.0;
     for (uint32_t s = 2; rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
         if (nonempty_splits(S, s) != s || p.x16 + (size_t)rem * s * kPartTile > ws_limit) continue;
         const double rounds = (double)((rem * s + num_cus - 1) / num_cus);
         const double us = (double)(full / num_cus) * (S * 2.0 + 8.0) + rounds * ((S + s - 1) / s * 2.0 + 8.0) + 3.0 +
-                          (double)rem * kPartTile * (s + 1) / 5e6;
+                          (double)rem * kPartTile * (s + 1) / 5e6 + round_x;
         if (us < best) best = p.us = us, p.splits = s;
     }
     return p;
@@ -279,7 +299,8 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
     }
     if (K % kStageK == 0 && N % 4 == 0 && offsets31 && (M < kW16MinTokens || !p.persistent)) {
         const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent, ws_limit);
-        if (few_ok && few_us(wtype, xtype, N, K, M, num_cus) < 0.97 * sp.us) {
+        const double sum = sp.splits > 1 ? 0.0 : tiled_sum_us(wtype, N, K, M, num_cus, ws_limit);
+        if (few_ok && few_us(xtype, N, K, M, num_cus) < 0.9 * (sp.us + sum)) {
             p.few = true;
             p.few_features = kFewNarrow;
             return p;

@@ -63,7 +63,7 @@ static void check(uint32_t wt, uint32_t xt, uint32_t N, uint32_t K, uint32_t M, 
     }
     // the tiled kernel: where the few-token kernel could run instead, not by much the slower of the two
     if (M > kSkinnyMaxTokens && few_fits(wt, N, K, M) && N % 4 == 0 &&
-        few_us(wt, xt, N, K, M, cus) < 0.8 * tiled_us(wt, xt, N, K, M, cus, limit))
+        few_us(xt, N, K, M, cus) < 0.8 * tiled_us(wt, xt, N, K, M, cus, limit))
         fail("tiled in place of the few-token kernel", wt, xt, N, K, M, cus, limit);
     // the tiled kernel (or, Q8_0 with K % 64 == 32, the generic one: no splits)
     if (wt == kQ8_0 && K % kStageK) {
@@ -100,6 +100,22 @@ int main() {
     if (f32_operand_type(kQ8_0) != kF16 || f32_operand_type(kQ4K) != kBF16) {
         std::printf("FAIL f32 operand types\n");
         return 1;
+    }
+    // launches of either kernel that the estimates once took for the other's
+    // (measured few-token : tiled, 15.5 : 8.9 us, 65 : 45, 34.9 : 25, 8.9 : 12.7)
+    {
+        struct {
+            uint32_t wt, xt, N, K, M;
+            bool few;
+        } const c[] = {{kQ8_0, kF16, 12288, 256, 257, false}, {kQ8_0, kF32, 1024, 15360, 257, false},
+                       {kQ4K, kF32, 64, 15360, 288, false}, {kQ8_0, kF32, 128, 3840, 350, true}};
+        for (const auto& s : c) {
+            n_checked++;
+            if (plan_gemm(s.wt, s.xt, s.N, s.K, s.M, 256).few != s.few) {
+                std::printf("FAIL %u x %u x %u: few-token kernel %d\n", s.M, s.N, s.K, !s.few);
+                return 1;
+            }
+        }
     }
     // a limit that holds fewer parts than the launch is cut into without one
     {
