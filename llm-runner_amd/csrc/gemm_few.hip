@@ -16,8 +16,8 @@
 //
 // Workgroup = 8 waves (two per SIMD) over one tile of 32 tokens x FF features,
 // 96 or 32 (plan::few_features holds the rule and the figures): 96 where a
-// launch has whole rounds of them, 32 where it has not, as three 32-feature
-// workgroups share a CU (50 KiB of LDS each) and hide each other's latency.
+// launch has whole rounds of them, 32 where it has not, as two 32-feature
+// workgroups share a CU (83 to 115 registers a lane) and hide each other's latency.
 // Wave w takes the K stages w, w + 8, w + 16, ... (64 k each) and keeps the
 // whole tile in FF / 32 32x32x16 MFMA accumulators; at the end the eight
 // partial tiles meet in LDS and are summed in wave order (deterministic).

@@ -123,24 +123,34 @@ inline bool few_fits(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M) {
 }
 
 // The few-token kernel's tile width up to kSkinnyMaxTokens tokens (0: the
-// skinny kernel). 96-feature tiles read the fewest bytes per CU but hold it
-// alone (102 KiB of LDS), so their cost is whole rounds over the CUs;
-// 32-feature tiles share a CU three at a time and cost by their number (f32
-// activations, re-read by every tile, more so past K = 8192), plus a fixed part
-// of a round. In units of a 32-feature tile; measured on 256 CUs, 96 -> 32
-// features: 77 x 9216 x 3072 Q4_K bf16 27.2 -> 19.2 us, 200 x 3840 x 3840 31.0 -> 22.7,
-// 64 x 9216 x 3072 15.2 / 15.7, 200 x 3072 x 3072 15.2 / 15.4, Q8_0 f32 15.7 / 21.0.
-// Below half the CUs' worth of 96-feature tiles the skinny kernel (packed
-// activations, K splits, partial sums: three launches) is the better one only
-// for f32 activations with long rows (77 x 3072 x 12288 43 against 48 us); the
-// 32-feature tiles take 77 x 3072 x 4096 Q4_K bf16 in 12.8 us against 19.5, 32 x
-// 3840 x 3840 8.7 against 19.6, 5 x 9216 x 3072 10.5 against 43.
+// skinny kernel, or the tiled one where N % 4). 96-feature tiles read the fewest
+// bytes per CU but hold it alone (102 KiB of LDS), so their cost is whole rounds
+// over the CUs; 32-feature tiles share a CU two at a time and cost by their number
+// (f32 activations, re-read by every tile, more so past K = 8192, as 16-bit ones a
+// little), plus a fixed part of a round. In units of a 32-feature tile; measured on
+// 256 CUs, 96 -> 32 features: 77 x 9216 x 3072 Q4_K bf16 27.2 -> 19.2 us, 200 x 3840
+// x 3840 31.0 -> 22.7, 64 x 9216 x 3072 15.2 / 15.7, 200 x 3072 x 3072 15.2 / 15.4,
+// Q8_0 f32 15.7 / 21.0, 200 x 21504 x 15360 Q8_0 bf16 414 / 508.
+// Below half the CUs' worth of 96-feature tiles the 32-feature tiles take 77 x 3072
+// x 4096 Q4_K bf16 in 12.8 us against the skinny kernel's 19.5 (packed activations,
+// K splits, partial sums: three launches), 32 x 3840 x 3840 8.7 against 19.6, 5 x
+// 9216 x 3072 10.5 against 43. The skinny kernel is the better one where a wave's K
+// stages, one after the other, are most of the time: f32 activations with long rows
+// (77 x 3072 x 12288 43 against 48 us; past 12288 with few features too, 150 x 64 x
+// 15360 28 against 34, tiled 23), 16-bit ones past 12288 where its splits still fill
+// the CUs with whole rounds (5 x 512 x 15360 19.6 against 23.6; x 256 and x 1024
+// 0.86-0.97 the other way), and long rows where some CUs get a second tile (200 x
+// 1536 x 8192 26 against 35, 150 x 2048 x 15360 bf16 36 against 48).
 inline uint32_t few_features(uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
     const uint64_t tm = (M + kFewTokens - 1) / kFewTokens, c = (uint64_t)num_cus;
     const uint64_t wide = tm * ((N + kFewFeatures - 1) / kFewFeatures), narrow = tm * ((N + kFewNarrow - 1) / kFewNarrow);
-    const bool long_f32 = xtype == kF32 && K > 8192;
-    if (2 * wide < c) return long_f32 && N >= 512 && N % 4 == 0 ? 0u : kFewNarrow;
-    const double f = long_f32 ? 1.6 : xtype == kF32 ? 1.3 : 1.03;
+    const bool f32 = xtype == kF32, long_rows = K > 8192;
+    if (2 * wide < c) {
+        const bool skinny = N % 4 == 0 && ((f32 && long_rows && N >= 512) || (narrow > c && K >= 8192 && N < 3072) ||
+                                           (K > 12288 && N > 256 && N < 1024));
+        return skinny || (f32 && K > 12288) ? 0u : kFewNarrow;
+    }
+    const double f = f32 ? (long_rows ? 1.6 : 1.3) : long_rows ? 1.14 : 1.03;
     return f * narrow + 0.7 * c < 3.0 * c * ((wide + c - 1) / c) ? kFewNarrow : kFewFeatures;
 }
 // Time in us of the 32-feature tiles past kSkinnyMaxTokens tokens, for the choice

@@ -117,6 +117,23 @@ int main() {
             }
         }
     }
+    // up to 256 tokens: which of the two few-token kernels, and its tile width (0: not the few-token kernel;
+    // measured the other way: 35 : 26 us, 48 : 36, 508 : 414, 34 : 28, 23.6 : 19.6, 17.2 : 20.5)
+    {
+        struct {
+            uint32_t wt, xt, N, K, M, features;
+        } const c[] = {{kQ8_0, kF32, 1536, 8192, 200, 0},   {kQ8_0, kBF16, 2048, 15360, 150, 0},
+                       {kQ8_0, kBF16, 21504, 15360, 200, 96}, {kQ8_0, kF32, 64, 15360, 150, 0},
+                       {kQ8_0, kF16, 512, 15360, 5, 0},     {kQ4K, kBF16, 128, 10240, 64, 32}};
+        for (const auto& s : c) {
+            const GemmPlan p = plan_gemm(s.wt, s.xt, s.N, s.K, s.M, 256);
+            n_checked++;
+            if (p.skinny != (s.features == 0) || (p.few ? p.few_features : 0u) != s.features) {
+                std::printf("FAIL %u x %u x %u: few-token tiles of %u features\n", s.M, s.N, s.K, p.few_features);
+                return 1;
+            }
+        }
+    }
     // a limit that holds fewer parts than the launch is cut into without one
     {
         const GemmPlan a = plan_gemm(kQ8_0, kBF16, 3840, 3840, 1101, 256);
