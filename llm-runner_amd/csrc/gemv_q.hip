@@ -397,15 +397,24 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         u32x4 v[GW::kLoads];
     };
     // (the last step may read into the next row: those units are masked below; past
-    // the last row the buffer ends. The step's offset is in the descriptor, not a
-    // scalar offset, which the range check need not cover)
+    // the last row the buffer ends, and there the step's offset is added to the
+    // lane's, as the range check need not cover a scalar offset. Added at every step
+    // it took 3% longer, 9216 x 12288 Q8_0 22.4 -> 23.0 us, a descriptor moved by it
+    // 28.7; with 16 rows shared by the waves the branch costs more, 3072 x 8192 8.0
+    // -> 8.7)
     auto load_w = [&](uint32_t s) __attribute__((always_inline)) {
         Set w;
         const uint32_t at = 4u * GW::kBytes * s;
-        const rsrc_t r = make_rsrc(W + (uint64_t)n0 * rb + at, s < steps && at < wbytes ? wbytes - at : 0u);
+        const rsrc_t r = make_rsrc(W + (uint64_t)n0 * rb, s < steps ? wbytes : 0u);
+        if (KS > 1u || 4u * (s + 1u) > nu) {
 #pragma unroll
-        for (uint32_t i = 0; i < GW::kLoads; i++)
-            w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i], 0, 0));
+            for (uint32_t i = 0; i < GW::kLoads; i++)
+                w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i] + at, 0, 0));
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < GW::kLoads; i++)
+                w.v[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, voff[i], at, 0));
+        }
         return w;
     };
     const uint32_t s0 = wave % KS;
