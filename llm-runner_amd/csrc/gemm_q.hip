@@ -1591,8 +1591,8 @@ hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uin
     if (seq_len == 0 || out_dim == 0) return hipSuccess;
     const uint32_t N = out_dim, K = in_dim, M = seq_len;
     if (runs_gemv(wtype, K, M))
-        return wtype == kGgmlQ4K ? launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, st)
-                                 : launch_gemv_q8(w, xtype, x, y, N, K, M, row_offset, st);
+        return wtype == kGgmlQ4K ? launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, num_cus, st)
+                                 : launch_gemv_q8(w, xtype, x, y, N, K, M, row_offset, num_cus, st);
     const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit);
     if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, pl.few_features, st);
     if (pl.skinny) return launch_gemm_skinny(w, wtype, x, xtype, y, N, K, M, row_offset, pl.splits, ws, st);

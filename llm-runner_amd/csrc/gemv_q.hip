@@ -227,9 +227,9 @@ static_assert(gemv_xs_fits<kGgmlQ4K, 1> && gemv_xs_fits<kGgmlQ4K, 2> && gemv_xs_
               gemv_xs_fits<kGgmlQ8_0, 1> && gemv_xs_fits<kGgmlQ8_0, 2> && gemv_xs_fits<kGgmlQ8_0, 4>);
 constexpr uint32_t kGemvLdsLimit = 160u * 1024u;
 template <uint32_t WT, int T>
-constexpr uint32_t gemv_lds_bytes(uint32_t K) {
+constexpr uint32_t gemv_lds_bytes(uint32_t K, uint32_t waves) {
     const uint32_t nu4 = (K / GemvW<WT>::kK + 3u) / 4u * 4u;
-    return nu4 * GemvX<WT, T>::kUnit + 4u * GemvW<WT>::kStep + 16u;
+    return nu4 * GemvX<WT, T>::kUnit + waves * GemvW<WT>::kStep + 16u;
 }
 
 // The same rows in f32, for activations that have no digits: each weight with
@@ -342,9 +342,10 @@ __device__ __forceinline__ void gemv_f32_rows(const uint8_t* W, const float* xs,
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
+// `waves`: of a workgroup, 4 to 8 (KS == 1; gemv_waves), else 4.
 template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
-__global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const GemvJobs<CAP> jobs, uint32_t N, uint32_t K,
-                                                          uint32_t ldy, uint32_t bpj) {
+__global__ void __launch_bounds__(512, T == 1 ? 3 : 2) gemv_i8_kernel(const GemvJobs<CAP> jobs, uint32_t N, uint32_t K,
+                                                          uint32_t ldy, uint32_t bpj, uint32_t waves) {
     static_assert(T == 1 || T == 2 || T == 4, "one token, two, or up to four");
     typedef GemvW<WT> GW;
     typedef GemvX<WT, T> GX;
@@ -355,11 +356,12 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     const uint32_t M = jobs.m[job];
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t nu = K / GW::kK, steps = (nu + 3u) / 4u, nu4 = 4u * steps;
+    const uint32_t nw = KS == 1u ? waves : 4u, threads = 64u * nw, rows = 16u * nw / KS;  // of the workgroup
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint8_t* const wsb = smem + nu4 * GX::kUnit;
     uint8_t* const ws = wsb + wave * GW::kStep;           // the wave's weight bytes of a step
-    uint32_t* const odd = (uint32_t*)(wsb + 4u * GW::kStep);  // the activations have no digits: f32 rows
+    uint32_t* const odd = (uint32_t*)(wsb + nw * GW::kStep);  // the activations have no digits: f32 rows
     if (tid == 0) *odd = 0u;
 
     // activations: thread -> 8 k of one token, four neighbours a sub-block; the
@@ -381,10 +383,10 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     constexpr uint32_t kAhead = T == 1 ? 2u : T == 2 ? 4u : 8u;
     X8 xa[kAhead];
 #pragma unroll
-    for (uint32_t q = 0; q < kAhead; q++) xa[q] = load_x(tid + 256u * q);
+    for (uint32_t q = 0; q < kAhead; q++) xa[q] = load_x(tid + threads * q);
 
     // the wave's 16 rows as a buffer: rows past N read as zero
-    const uint32_t n0 = blk * (64u / KS) + wave / KS * 16u, rb = nu * GW::kBytes;
+    const uint32_t n0 = blk * rows + wave / KS * 16u, rb = nu * GW::kBytes;
     const uint8_t* const W = jobs.w[job] + (uint64_t)jobs.row_offset[job] * rb;
     const uint32_t wbytes = n0 < N ? min(16u, N - n0) * rb : 0u;
     uint32_t voff[GW::kLoads];  // piece c = 64 i + lane of a step: row c / kRowPieces, 16 (c % kRowPieces) bytes in
@@ -498,16 +500,16 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
     };
 #pragma unroll
     for (uint32_t q = 0; q < kAhead; q++)
-        if (256u * q < total) stage_x(tid + 256u * q, xa[q]);
-    for (uint32_t i = 256u * kAhead + tid; i < (total + 255u) / 256u * 256u; i += 256u) stage_x(i, load_x(i));
+        if (threads * q < total) stage_x(tid + threads * q, xa[q]);
+    for (uint32_t i = threads * kAhead; i < total; i += threads) stage_x(i + tid, load_x(i + tid));  // (whole waves)
     if (bad) *odd = 1u;
     __syncthreads();
     if (*odd != 0u) {  // a whole workgroup's branch: nothing below waits for it
         // (the last read of odd and of the digits lies behind every thread's barrier)
         float* const xs = (float*)smem;
-        for (uint32_t i = 4u * tid; i < M * K; i += 1024u) *(f32x4*)(xs + gemv_xs(i)) = load_x4<XT>(X, i);
+        for (uint32_t i = 4u * tid; i < M * K; i += 4u * threads) *(f32x4*)(xs + gemv_xs(i)) = load_x4<XT>(X, i);
         __syncthreads();
-        gemv_f32_rows<WT, T, 4 / KS>(W, xs, Y, blk * (64u / KS) + wave * (16u / KS), N, K, rb, M, ldy, lane);
+        gemv_f32_rows<WT, T, 4 / KS>(W, xs, Y, blk * rows + wave * (16u / KS), N, K, rb, M, ldy, lane);
         return;
     }
 
@@ -651,8 +653,8 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 #pragma unroll
             for (int m = 0; m < T; m++) red[(wave * T + m) * 16u + r] = acc[m];
         __syncthreads();
-        for (uint32_t i = tid; i < 64u / KS * T; i += 256u) {
-            const uint32_t row = i % (64u / KS), m = i / (64u / KS), w0 = row / 16u * KS, n = blk * (64u / KS) + row;
+        for (uint32_t i = tid; i < rows * T; i += threads) {
+            const uint32_t row = i % rows, m = i / rows, w0 = row / 16u * KS, n = blk * rows + row;
             float v = red[(w0 * T + m) * 16u + row % 16u];
 #pragma unroll
             for (uint32_t w = 1; w < KS; w++) v += red[((w0 + w) * T + m) * 16u + row % 16u];
@@ -670,19 +672,34 @@ __global__ void __launch_bounds__(256, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
 template <uint32_t WT>
 bool gemv_fits(uint32_t K, uint32_t M) {
     if (M == 0 || M > kGemvMaxTokens || K % 256u || K == 0 || K > (1u << 20)) return false;
-    return (M == 1 ? gemv_lds_bytes<WT, 1>(K) : M == 2 ? gemv_lds_bytes<WT, 2>(K) : gemv_lds_bytes<WT, 4>(K)) <=
+    return (M == 1 ? gemv_lds_bytes<WT, 1>(K, 4u) : M == 2 ? gemv_lds_bytes<WT, 2>(K, 4u) : gemv_lds_bytes<WT, 4>(K, 4u)) <=
            kGemvLdsLimit;
+}
+
+// Waves of a workgroup, 16 rows each, for one projection: as few from 4 on as
+// give every CU at most one workgroup (beside the activations' digits the LDS holds
+// one to three of 4 waves, and each cuts the digits anew), 4 where 8 do not.
+// 18432 rows are 288 workgroups of 4 and 231 of 5: x 3072 Q8_0 at one, two and four
+// tokens 13.8, 18.2, 29.5 -> 12.3, 15.6, 18.5 us, x 6144 24, 44, 55 -> 22, 28, 34, x
+// 12288 Q4_K at one 47 -> 30. With two full rounds more waves gain nothing (36864 x
+// 3072 Q4_K, two tokens: 24.5 us with 4, 28.6 with 5).
+template <uint32_t WT, int T>
+uint32_t gemv_waves(uint32_t N, uint32_t K, int num_cus) {
+    for (uint32_t w = 4; w <= 8 && gemv_lds_bytes<WT, T>(K, w) <= kGemvLdsLimit; w++)
+        if ((N + 16u * w - 1u) / (16u * w) <= (uint32_t)num_cus) return w;
+    return 4;
 }
 
 template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
 hipError_t launch_gemv_k(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
-                         hipStream_t st) {
+                         uint32_t waves, hipStream_t st) {
     auto kern = gemv_i8_kernel<WT, XT, T, CAP, KS>;
     static const hipError_t attr =
         hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvLdsLimit);
     if (attr != hipSuccess) return attr;
-    const uint32_t rows = 64u / KS, bpj = (N + rows - 1u) / rows;
-    hipLaunchKernelGGL(kern, dim3(bpj * n_jobs), dim3(256), (gemv_lds_bytes<WT, T>(K)), st, jobs, N, K, ldy, bpj);
+    const uint32_t rows = 16u * waves / KS, bpj = (N + rows - 1u) / rows;
+    hipLaunchKernelGGL(kern, dim3(bpj * n_jobs), dim3(64u * waves), (gemv_lds_bytes<WT, T>(K, waves)), st, jobs, N, K,
+                       ldy, bpj, waves);
     return hipGetLastError();
 }
 
@@ -693,19 +710,20 @@ hipError_t launch_gemv_k(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N,
 // against 25 us; one token, 18432 x 3072: 9.7 against 11.1).
 template <uint32_t WT, uint32_t XT, int T, uint32_t CAP>
 hipError_t launch_gemv_t(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
-                         hipStream_t st) {
-    if ((N + 63u) / 64u * n_jobs < 128u) return launch_gemv_k<WT, XT, T, CAP, 4>(jobs, n_jobs, N, K, ldy, st);
-    return launch_gemv_k<WT, XT, T, CAP, 1>(jobs, n_jobs, N, K, ldy, st);
+                         int num_cus, hipStream_t st) {
+    if ((N + 63u) / 64u * n_jobs < 128u) return launch_gemv_k<WT, XT, T, CAP, 4>(jobs, n_jobs, N, K, ldy, 4u, st);
+    const uint32_t waves = CAP == 1u ? gemv_waves<WT, T>(N, K, num_cus) : 4u;
+    return launch_gemv_k<WT, XT, T, CAP, 1>(jobs, n_jobs, N, K, ldy, waves, st);
 }
 
 template <uint32_t WT, uint32_t CAP>
 hipError_t launch_gemv(uint32_t xtype, const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
-                       uint32_t max_m, hipStream_t st) {
+                       uint32_t max_m, int num_cus, hipStream_t st) {
     auto by_x = [&](auto xt) {
         constexpr uint32_t XT = decltype(xt)::value;
-        return max_m <= 1   ? launch_gemv_t<WT, XT, 1, CAP>(jobs, n_jobs, N, K, ldy, st)
-               : max_m <= 2 ? launch_gemv_t<WT, XT, 2, CAP>(jobs, n_jobs, N, K, ldy, st)
-                            : launch_gemv_t<WT, XT, 4, CAP>(jobs, n_jobs, N, K, ldy, st);
+        return max_m <= 1   ? launch_gemv_t<WT, XT, 1, CAP>(jobs, n_jobs, N, K, ldy, num_cus, st)
+               : max_m <= 2 ? launch_gemv_t<WT, XT, 2, CAP>(jobs, n_jobs, N, K, ldy, num_cus, st)
+                            : launch_gemv_t<WT, XT, 4, CAP>(jobs, n_jobs, N, K, ldy, num_cus, st);
     };
     switch (xtype) {
         case kGgmlF32: return by_x(std::integral_constant<uint32_t, kGgmlF32>{});
@@ -743,16 +761,16 @@ hipError_t launch_gemv_q4k_multi(uint32_t xtype, const GemmJob* jobs, uint32_t n
     }
     if (max_m == 0) return hipSuccess;
     if (!gemv_fits<kGgmlQ4K>(K, max_m)) return hipErrorNotSupported;
-    return launch_gemv<kGgmlQ4K>(xtype, t, n_jobs, N, K, ldy, max_m, st);
+    return launch_gemv<kGgmlQ4K>(xtype, t, n_jobs, N, K, ldy, max_m, 0, st);
 }
 
 hipError_t launch_gemv_q4k(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K,
-                           uint32_t M, uint32_t row_offset, hipStream_t st) {
+                           uint32_t M, uint32_t row_offset, int num_cus, hipStream_t st) {
     if (M == 0 || N == 0) return hipSuccess;
     if (M > kGemvMaxTokens) return hipErrorInvalidValue;
     if (gemv_fits<kGgmlQ4K>(K, M)) {
         const GemvJobs<1> one{{(const uint8_t*)w}, {x}, {y}, {M}, {row_offset}};
-        return launch_gemv<kGgmlQ4K>(xtype, one, 1u, N, K, N, M, st);
+        return launch_gemv<kGgmlQ4K>(xtype, one, 1u, N, K, N, M, num_cus, st);
     }
     switch (xtype) {
         case kGgmlF32: return launch_t<kGgmlF32>(w, x, y, N, K, M, row_offset, st);
@@ -764,11 +782,11 @@ hipError_t launch_gemv_q4k(const void* w, uint32_t xtype, const void* x, float* 
 bool gemv_q8_fits(uint32_t K, uint32_t M) { return gemv_fits<kGgmlQ8_0>(K, M); }
 
 hipError_t launch_gemv_q8(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K, uint32_t M,
-                          uint32_t row_offset, hipStream_t st) {
+                          uint32_t row_offset, int num_cus, hipStream_t st) {
     if (M == 0 || N == 0) return hipSuccess;
     if (!gemv_fits<kGgmlQ8_0>(K, M)) return hipErrorInvalidValue;
     const GemvJobs<1> one{{(const uint8_t*)w}, {x}, {y}, {M}, {row_offset}};
-    return launch_gemv<kGgmlQ8_0>(xtype, one, 1u, N, K, N, M, st);
+    return launch_gemv<kGgmlQ8_0>(xtype, one, 1u, N, K, N, M, num_cus, st);
 }
 
 }  // namespace llmr

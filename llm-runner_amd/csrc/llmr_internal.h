@@ -98,12 +98,12 @@ hipError_t launch_q8_lora_merge(void* base, const float* A, const float* B, uint
 // HBM-bound weight stream, taken by launch_batch_matmul for such M.
 using plan::kGemvMaxTokens;
 hipError_t launch_gemv_q4k(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K,
-                           uint32_t M, uint32_t row_offset, hipStream_t st);
+                           uint32_t M, uint32_t row_offset, int num_cus, hipStream_t st);
 
 // The same for Q8_0 weights, where gemv_q8_fits.
 bool gemv_q8_fits(uint32_t K, uint32_t M);
 hipError_t launch_gemv_q8(const void* w, uint32_t xtype, const void* x, float* y, uint32_t N, uint32_t K, uint32_t M,
-                          uint32_t row_offset, hipStream_t st);
+                          uint32_t row_offset, int num_cus, hipStream_t st);
 
 // SwiGLU of two Q8_0 GEMMs (batch_matmul_swiglu_q8). `ws` must hold
 // swiglu_workspace_bytes(...) bytes (may be 0).

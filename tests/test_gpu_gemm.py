@@ -95,6 +95,8 @@ def test_small_m_q4k_f32_matches_reference_arithmetic(orc, dev, M, N, K, row_off
     (8, 3, 8195, 1792, 1, 2),      # 14 units
     (8, 2, 130, 768, 30, 0),
     (8, 4, 33, 3840, 0, 5),
+    (8, 4, 16390, 512, 30, 1),     # more row blocks than CUs: workgroups of five waves, six rows in the last
+    (12, 1, 28700, 768, 0, 0),     # of eight waves, part-filled steps
 ])
 def test_gemv_against_64_bits(dev, wtype, M, N, K, xtype, row_offset):
     """At most four tokens: int8 digits of the activations times the quants,
@@ -210,6 +212,7 @@ def test_gemv_activations_out_of_the_digits_range(dev, wtype, M, N, K, xtype, ou
     (8, 1, 8197, 768, 1, 1),
     (12, 2, 8203, 2304, 1, 0),
     (8, 4, 8192, 1280, 30, 0),
+    (8, 2, 16390, 256, 0, 0),      # workgroups of five waves
 ])
 def test_gemv_nonfinite_activations(dev, wtype, M, N, K, xtype, row_offset):
     """An infinite or NaN activation gives the products of the dequantized
