@@ -342,6 +342,14 @@ __device__ __forceinline__ void gemv_f32_rows(const uint8_t* W, const float* xs,
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
+// v of lane ^ 1 or lane ^ 2, without the LDS round trip of a shuffle
+template <int X, typename V>
+__device__ __forceinline__ V quad_xor(V v) {
+    static_assert(X == 1 || X == 2, "within a quad");
+    return __builtin_bit_cast(
+        V, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), X == 1 ? 0xb1 : 0x4e, 15, 15, false));
+}
+
 // `waves`: of a workgroup, 4 to 8 (KS == 1; gemv_waves), else 4.
 template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
 __global__ void __launch_bounds__(512, T == 1 ? 3 : 2) gemv_i8_kernel(const GemvJobs<CAP> jobs, uint32_t N, uint32_t K,
@@ -432,11 +440,10 @@ __global__ void __launch_bounds__(512, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         bad = bad || !(__builtin_fabsf(sum) < INFINITY);  // (sums that overflow: the f32 rows too)
 #pragma unroll
         for (int e = 0; e < 8; e++) mx = fmaxf(mx, __builtin_fabsf(x[e]));
-#pragma unroll
-        for (int o = 1; o < 4; o <<= 1) {
-            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-            sum += __shfl_xor(sum, o, 64);
-        }
+        mx = fmaxf(mx, quad_xor<1>(mx));
+        sum += quad_xor<1>(sum);
+        mx = fmaxf(mx, quad_xor<2>(mx));
+        sum += quad_xor<2>(sum);
         // scale 2^e with 2^e mx in [2^29, 2^30), e kept where 2^e and 2^-e are normal
         const int e = min(126, max(-126, 156 - (int)((__float_as_uint(mx) >> 23) & 0xffu)));
         const float up = __uint_as_float((uint32_t)(127 + e) << 23), down = __uint_as_float((uint32_t)(127 - e) << 23);
@@ -450,8 +457,8 @@ __global__ void __launch_bounds__(512, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
             low += b < low_bits ? 1u : 0u;
             least = min(least, b);
         }
-        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0xb1, 15, 15, false);  // lane ^ 1
-        low += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)low, 0x4e, 15, 15, false);  // lane ^ 2
+        low += quad_xor<1>(low);
+        low += quad_xor<2>(low);
         bad = bad || low >= 8u || least < 2u * __float_as_uint(kTiny * down) - 1u || (mx > 0.0f && mx < 0x1p-97f);
         uint32_t dg[2][4];  // [four k][digit, lowest first]: a byte per k
         int sums[4] = {0, 0, 0, 0};
@@ -481,8 +488,8 @@ __global__ void __launch_bounds__(512, T == 1 ? 3 : 2) gemv_i8_kernel(const Gemv
         if constexpr (WT == kGgmlQ4K)
 #pragma unroll
             for (int p = 0; p < 4; p++) {
-                sums[p] += __shfl_xor(sums[p], 1, 64);
-                sums[p] += __shfl_xor(sums[p], 2, 64);
+                sums[p] += quad_xor<1>(sums[p]);
+                sums[p] += quad_xor<2>(sums[p]);
             }
         if (i >= total) return;
         const uint32_t m = T == 1 ? 0u : i / pieces, c = T == 1 ? i : i - m * pieces;  // chunk of 8 k
