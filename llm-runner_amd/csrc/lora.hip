@@ -421,7 +421,16 @@ hipError_t launch_lora_correction(const float* A, const float* B, uint32_t rank,
                                   uint32_t seq_len, uint32_t b_rows, uint32_t row_offset, uint32_t weight_row_offset,
                                   hipStream_t st) {
     if (rank == 0 || seq_len == 0) return hipSuccess;
-    const bool wide = in_dim % 4u == 0u && ((uintptr_t)A & 15u) == 0u && ((uintptr_t)x & 15u) == 0u;
+    // One wave walks a whole row for 8 ranks, so with one such group of ranks (two,
+    // with long rows and many tokens) a workgroup of the LDS form is the faster one
+    // where the walk is long and waves are few: both hops at rank 8, LDS : wave, 1 x
+    // 3072 22 : 32 us at K = 15360, 2048 x 1024 1.0 : 1.2 at 3072, 4608 x 1024 1.0 :
+    // 0.95, 1.0 : 1.0 or less at K = 1024; rank 16, 4608 tokens 1.0 : 1.14 at 15360,
+    // 1.0 : 0.89 at 8192; rank 12, one token 1.0 : 0.89 at 3072.
+    const bool few_waves = rank <= 8u    ? in_dim >= 2048u && (in_dim > 4096u || seq_len < 4096u)
+                           : rank <= 16u ? in_dim > 12288u && seq_len >= 4096u
+                                         : false;
+    const bool wide = !few_waves && in_dim % 4u == 0u && ((uintptr_t)A & 15u) == 0u && ((uintptr_t)x & 15u) == 0u;
     auto down = [&](auto xt) {
         constexpr uint32_t XT = decltype(xt)::value;
         if (wide) {

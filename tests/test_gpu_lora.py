@@ -68,6 +68,7 @@ def test_lora_correction_bit_exact(orc, dev, seq, in_dim, rank, out_dim, b_rows,
     (35, 1028, 12, 300, 30, 0),   # part-filled token and rank groups, one lane's last pass
     (6, 254, 5, 64, 0, 0),        # in_dim % 4 != 0: the LDS form of hop 1
     (9, 512, 8, 264, 1, 1),       # activations one element past 16 bytes: the same
+    (6, 2048, 8, 64, 30, 0),      # the LDS form by its rule: one group of ranks, a long row
     (33, 256, 32, 257, 30, 0),    # one token and one column past a hop-2 workgroup
     (18, 260, 96, 300, 0, 0),     # three chunks of 32 ranks
     (1030, 64, 4, 33000, 30, 0),  # enough workgroups for 32 tokens each
