@@ -328,7 +328,9 @@ __global__ void __launch_bounds__(256) lora_up_reg_kernel(const float* __restric
                                                            uint32_t b_rows) {
     typedef __attribute__((address_space(4))) const float cfloat;
     const uint32_t o = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t s0 = blockIdx.y * T, nt = min(T, seq_len - s0);
+    const uint32_t group = blockIdx.z * gridDim.y + blockIdx.y;  // of T tokens
+    if (group >= (seq_len + T - 1u) / T) return;
+    const uint32_t s0 = group * T, nt = min(T, seq_len - s0);
     const rsrc_t yr = make_rsrc(out + (uint64_t)s0 * out_dim, (uint64_t)nt * out_dim * 4u);
     const uint32_t yo = o < b_rows ? (row_offset + o) * 4u : 0x80000000u;
     float yv[T];
@@ -457,18 +459,23 @@ hipError_t launch_lora_correction(const float* A, const float* B, uint32_t rank,
         // with 16, 1536 x 9216 x 32 52 against 49, 300 x 3072 x 16 23 against 17
         const uint32_t cols = (b_rows + 255u) / 256u;
         const bool wide_t = (uint64_t)cols * ((seq_len + 31u) / 32u) >= 4096u;
+        // (a grid's y ends at 65535 workgroups: 1048560 tokens of 16)
+        auto grid = [&](uint32_t t) {
+            const uint32_t groups = (seq_len - 1u) / t + 1u, y = min(groups, 65535u);
+            return dim3(cols, y, (groups + y - 1u) / y);
+        };
         auto go = [&](auto r) {
             constexpr uint32_t R = decltype(r)::value;
             if (rank > R)
-                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, true>), dim3(cols, (seq_len + 15u) / 16u), dim3(256), 0,
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, true>), grid(16u), dim3(256), 0,
                                    st, B, (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
                                    weight_row_offset, b_rows);
             else if (wide_t)
-                hipLaunchKernelGGL((lora_up_reg_kernel<R, 32, false>), dim3(cols, (seq_len + 31u) / 32u), dim3(256), 0, st, B,
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 32, false>), grid(32u), dim3(256), 0, st, B,
                                    (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
                                    weight_row_offset, b_rows);
             else
-                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, false>), dim3(cols, (seq_len + 15u) / 16u), dim3(256), 0, st, B,
+                hipLaunchKernelGGL((lora_up_reg_kernel<R, 16, false>), grid(16u), dim3(256), 0, st, B,
                                    (const float*)scratch, out, rank, out_dim, seq_len, scale, row_offset,
                                    weight_row_offset, b_rows);
         };

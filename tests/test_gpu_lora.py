@@ -72,6 +72,7 @@ def test_lora_correction_bit_exact(orc, dev, seq, in_dim, rank, out_dim, b_rows,
     (33, 256, 32, 257, 30, 0),    # one token and one column past a hop-2 workgroup
     (18, 260, 96, 300, 0, 0),     # three chunks of 32 ranks
     (1030, 64, 4, 33000, 30, 0),  # enough workgroups for 32 tokens each
+    (1048580, 4, 64, 4, 30, 0),   # more groups of 16 tokens than a grid's y holds
 ])
 def test_lora_correction_edges_bit_exact(orc, dev, seq, in_dim, rank, out_dim, xtype, shift):
     """The correction at the edges of its token, rank and column groups and at
