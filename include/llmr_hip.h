@@ -183,7 +183,9 @@ LLMR_API int llmr_batch_matmul_pc(llmr_context* ctx, const void* weight, uint32_
  * plan needs more, the call takes the form that fits: the one-pass kernels
  * instead of the weight image (the same bits), fewer K splits (the same
  * result to f32 summation order), the tiled kernel reading f32 activations
- * in place instead of their 16-bit copy (the same operands). Every call on
+ * in place instead of their 16-bit copy (the same operands). On a stream that
+ * is being captured, this call and llmr_batch_matmul cut no tiles along K, so
+ * that launches that need no workspace uncut need none there. Every call on
  * one GPU uses that GPU's one array, whose contents persist between calls.
  * Calls of one context on different streams (llmr_set_stream) are ordered
  * as its workspace is: a call on another stream than the last one waits

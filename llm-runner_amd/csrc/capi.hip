@@ -320,6 +320,16 @@ static int release_workspace(llmr_context* ctx, size_t need) {
     return LLMR_OK;
 }
 
+// Whether a GEMM whose plan takes `need` bytes with tiles cut along K and `whole`
+// without keeps to the latter: while the current stream is being captured a call
+// allocates nothing more than the tiled kernel's plan does, waits for no other
+// stream, and leaves no more of the workspace's addresses in the graph.
+static bool captures_whole(llmr_context* ctx, size_t need, size_t whole) {
+    if (need == whole) return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->cur, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // Argument checks of llmr_batch_matmul and its no-allocation variant.
 static int check_batch_matmul(llmr_context* ctx, const void* weight, uint32_t wtype, const void* input,
                               uint32_t xtype, const float* output, uint32_t out_dim, uint32_t in_dim,
@@ -343,10 +353,18 @@ int llmr_batch_matmul(llmr_context* ctx, const void* weight, uint32_t wtype, con
     if (int r = check_batch_matmul(ctx, weight, wtype, input, xtype, output, out_dim, in_dim, seq_len, row_offset))
         return r;
     if (seq_len == 0 || out_dim == 0) return ok();
-    const size_t need = llmr::batch_matmul_workspace_bytes(wtype, xtype, out_dim, in_dim, seq_len, ctx->num_cus);
+    auto bytes = [&](bool cut) {
+        return llmr::batch_matmul_workspace_bytes(wtype, xtype, out_dim, in_dim, seq_len, ctx->num_cus,
+                                                  llmr::kNoWorkspaceLimit, cut);
+    };
+    size_t need = bytes(true);
+    const size_t whole = need ? bytes(false) : 0u;
+    const bool cut = !captures_whole(ctx, need, whole);
+    if (!cut) need = whole;
     if (int r = acquire_workspace(ctx, need)) return r;
     hipError_t e = llmr::launch_batch_matmul(weight, wtype, input, xtype, output, out_dim, in_dim, seq_len,
-                                             row_offset, ctx->num_cus, ctx->ws, ctx->cur);
+                                             row_offset, ctx->num_cus, ctx->ws, ctx->cur, llmr::kNoWorkspaceLimit,
+                                             cut);
     if (e != hipSuccess) return fail(LLMR_ERR_HIP, "batch_matmul launch: %s", hipGetErrorString(e));
     if (int r = release_workspace(ctx, need)) return r;
     return ok();
@@ -368,8 +386,14 @@ int llmr_batch_matmul_noalloc(llmr_context* ctx, const void* weight, uint32_t wt
     // the plan keeps within the scratch: smaller forms (one-pass kernels
     // instead of a weight image, fewer K splits, the tiled kernel reading f32
     // activations in place) where the usual plan needs more
-    const size_t need = llmr::batch_matmul_workspace_bytes(wtype, xtype, out_dim, in_dim, seq_len, ctx->num_cus,
-                                                           kNoAllocScratchBytes);
+    auto bytes = [&](bool cut) {
+        return llmr::batch_matmul_workspace_bytes(wtype, xtype, out_dim, in_dim, seq_len, ctx->num_cus,
+                                                  kNoAllocScratchBytes, cut);
+    };
+    size_t need = bytes(true);
+    const size_t whole = need ? bytes(false) : 0u;
+    const bool cut = !captures_whole(ctx, need, whole);
+    if (!cut) need = whole;
     if (need > kNoAllocScratchBytes)
         return fail(LLMR_ERR_INVALID_ARG, "this GEMM needs %zu bytes of scratch, beyond the %zu the no-allocation "
                     "entry point holds; call llmr_batch_matmul", need, kNoAllocScratchBytes);
@@ -378,7 +402,7 @@ int llmr_batch_matmul_noalloc(llmr_context* ctx, const void* weight, uint32_t wt
     if (need > 0 && ctx->scr_used && ctx->scr_stream != ctx->cur)
         LLMR_HIP_CHECK(hipStreamWaitEvent(ctx->cur, ctx->scr_done, 0));
     hipError_t e = llmr::launch_batch_matmul(weight, wtype, input, xtype, output, out_dim, in_dim, seq_len, row_offset,
-                                             ctx->num_cus, ptr, ctx->cur, kNoAllocScratchBytes);
+                                             ctx->num_cus, ptr, ctx->cur, kNoAllocScratchBytes, cut);
     if (e != hipSuccess) return fail(LLMR_ERR_HIP, "batch_matmul launch: %s", hipGetErrorString(e));
     if (need > 0) {
         ctx->scr_stream = ctx->cur;
@@ -620,11 +644,17 @@ static int batch_matmul_multi_impl(llmr_context* ctx, uint32_t wtype, uint32_t x
                              heads->n_heads, heads->seq_len, heads->out_type, heads->eps};
     const llmr::GemmEpilogue ge{e.kind, e.ldy, e.ldy2, e.split, has2 ? e.output2_type : (uint32_t)LLMR_GGML_BF16,
                                 heads ? &gh : nullptr};
-    const size_t need = llmr::batch_matmul_multi_workspace_bytes(wtype, xtype, out_dim, in_dim, gj, n_jobs, ge,
-                                                                 ctx->num_cus, images != nullptr);
+    auto bytes = [&](bool cut_tiles) {
+        return llmr::batch_matmul_multi_workspace_bytes(wtype, xtype, out_dim, in_dim, gj, n_jobs, ge, ctx->num_cus,
+                                                        images != nullptr, cut_tiles);
+    };
+    size_t need = bytes(true);
+    const size_t whole = need ? bytes(false) : 0u;
+    const bool cut = !captures_whole(ctx, need, whole);
+    if (!cut) need = whole;
     if (int r = acquire_workspace(ctx, need)) return r;
     hipError_t err = llmr::launch_batch_matmul_multi(wtype, xtype, out_dim, in_dim, gj, n_jobs, ge, ctx->num_cus,
-                                                     ctx->ws, ctx->cur, images, next ? &nx : nullptr);
+                                                     ctx->ws, ctx->cur, images, next ? &nx : nullptr, cut);
     if (err != hipSuccess) return fail(LLMR_ERR_HIP, "batch_matmul_multi launch: %s", hipGetErrorString(err));
     if (int r = release_workspace(ctx, need)) return r;
     return ok();

@@ -216,7 +216,7 @@ struct SplitPlan {
     size_t ws(uint64_t tiles) const { return x16 + (size_t)(tiles - full) * splits * kPartTile; }
 };
 inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
-                            bool persistent, size_t ws_limit) {
+                            bool persistent, size_t ws_limit, bool cut_tiles) {
     const uint64_t tiles = (uint64_t)((M + 255) / 256) * ((N + 255) / 256);
     const uint32_t S = K / kStageK;
     const uint64_t full = tiles / num_cus * num_cus, rem = tiles - full;
@@ -228,7 +228,7 @@ inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t
     p.us = whole;
     double best = 0.97 * whole;
     const double round_x = xtype == kF32 && !persistent ? (double)M * K * 6.0 / 8e6 : 0.0;
-    for (uint32_t s = 2; rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
+    for (uint32_t s = 2; cut_tiles && rem && S >= kSplitTileMinStages && s <= std::min(kSplitMax, S / kSplitMinStages); s++) {
         if (nonempty_splits(S, s) != s || p.x16 + (size_t)rem * s * kPartTile > ws_limit) continue;
         const double rounds = (double)((rem * s + num_cus - 1) / num_cus);
         const double us = (double)(full / num_cus) * (S * 2.0 + 8.0) + rounds * ((S + s - 1) / s * 2.0 + 8.0) + 3.0 +
@@ -259,6 +259,9 @@ inline SplitPlan plan_split(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t
 // activations for the others does not fit. The estimates are of what fits: with
 // 32 MiB, 323 x 3072 x 15360 Q8_0 f16 ran the tiled kernel, 1.5 times the
 // few-token kernel's time, as the split it was compared with did not fit.
+// Without cut_tiles (a stream being captured, which allocates and waits for
+// nothing) no tile is cut along K: such a launch needs a workspace where the tiled
+// kernel mostly needs none.
 struct GemmPlan {
     bool persistent, two_pass, convert_x, skinny, few;
     uint32_t xt;                  // activation type the kernel reads
@@ -270,7 +273,7 @@ struct GemmPlan {
                                   // (skinny), split-K partials (tiled)
 };
 inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus,
-                          size_t ws_limit = kNoWorkspaceLimit) {
+                          size_t ws_limit = kNoWorkspaceLimit, bool cut_tiles = true) {
     GemmPlan p{};
     p.xt = xtype;
     p.tiles = TilePlan{64, 1};
@@ -308,7 +311,7 @@ inline GemmPlan plan_gemm(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K
         }
     }
     if (K % kStageK == 0 && N % 4 == 0 && offsets31 && (M < kW16MinTokens || !p.persistent)) {
-        const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent, ws_limit);
+        const SplitPlan sp = plan_split(wtype, xtype, N, K, M, num_cus, p.persistent, ws_limit, cut_tiles);
         const double sum = sp.splits > 1 ? 0.0 : tiled_sum_us(wtype, N, K, M, num_cus, ws_limit);
         if (few_ok && few_us(xtype, N, K, M, num_cus) < 0.9 * (sp.us + sum)) {
             p.few = true;

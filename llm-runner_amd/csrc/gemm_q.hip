@@ -1425,9 +1425,9 @@ bool runs_gemv(uint32_t wtype, uint32_t K, uint32_t M) {
 }  // namespace
 
 size_t batch_matmul_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M,
-                                    int num_cus, size_t ws_limit) {
+                                    int num_cus, size_t ws_limit, bool cut_tiles) {
     if (M == 0 || N == 0 || runs_gemv(wtype, K, M)) return 0;
-    return plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit).ws;
+    return plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit, cut_tiles).ws;
 }
 
 namespace {
@@ -1587,13 +1587,14 @@ hipError_t launch_split(const void* w, uint32_t wtype, const void* x, uint32_t x
 
 hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uint32_t xtype,
                                float* y, uint32_t out_dim, uint32_t in_dim, uint32_t seq_len,
-                               uint32_t row_offset, int num_cus, void* ws, hipStream_t st, size_t ws_limit) {
+                               uint32_t row_offset, int num_cus, void* ws, hipStream_t st, size_t ws_limit,
+                               bool cut_tiles) {
     if (seq_len == 0 || out_dim == 0) return hipSuccess;
     const uint32_t N = out_dim, K = in_dim, M = seq_len;
     if (runs_gemv(wtype, K, M))
         return wtype == kGgmlQ4K ? launch_gemv_q4k(w, xtype, x, y, N, K, M, row_offset, num_cus, st)
                                  : launch_gemv_q8(w, xtype, x, y, N, K, M, row_offset, num_cus, st);
-    const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit);
+    const GemmPlan pl = plan_gemm(wtype, xtype, N, K, M, num_cus, ws_limit, cut_tiles);
     if (pl.few) return launch_gemm_few(w, wtype, x, xtype, y, N, K, M, row_offset, pl.few_features, st);
     if (pl.skinny) return launch_gemm_skinny(w, wtype, x, xtype, y, N, K, M, row_offset, pl.splits, ws, st);
     if (pl.split > 1) return launch_split(w, wtype, x, xtype, y, N, K, M, row_offset, pl, num_cus, ws, st);
@@ -1754,10 +1755,13 @@ hipError_t launch_persist_multi(const PersistArgs& a, int num_cus, hipStream_t s
 // workspace `t` (directly into the output for an unstrided store), then
 // the epilogue as glue passes. `gemm_ws` is the GEMM's own workspace.
 hipError_t run_job_fallback(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, const GemmJob& j,
-                            const GemmEpilogue& epi, int num_cus, float* t, void* gemm_ws, hipStream_t st) {
+                            const GemmEpilogue& epi, int num_cus, float* t, void* gemm_ws, bool cut_tiles,
+                            hipStream_t st) {
     if (epi.kind == kEpiStore && epi.ldy == N)
-        return launch_batch_matmul(j.w, wtype, j.x, xtype, j.y, N, K, j.M, j.row_offset, num_cus, gemm_ws, st);
-    hipError_t e = launch_batch_matmul(j.w, wtype, j.x, xtype, t, N, K, j.M, j.row_offset, num_cus, gemm_ws, st);
+        return launch_batch_matmul(j.w, wtype, j.x, xtype, j.y, N, K, j.M, j.row_offset, num_cus, gemm_ws, st,
+                                   kNoWorkspaceLimit, cut_tiles);
+    hipError_t e = launch_batch_matmul(j.w, wtype, j.x, xtype, t, N, K, j.M, j.row_offset, num_cus, gemm_ws, st,
+                                       kNoWorkspaceLimit, cut_tiles);
     if (e != hipSuccess) return e;
     if (epi.kind == kEpiResidual) {
         ResidualArgs r{j.y, t, nullptr, j.gate, epi.ldy, N, j.M, N, 0.0f};
@@ -1808,7 +1812,7 @@ size_t fallback_t_bytes(uint32_t N, const GemmJob* jobs, uint32_t n_jobs, const 
 
 size_t batch_matmul_multi_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K,
                                           const GemmJob* jobs, uint32_t n_jobs, const GemmEpilogue& epi,
-                                          int num_cus, bool prebuilt_images) {
+                                          int num_cus, bool prebuilt_images, bool cut_tiles) {
     const size_t t = fallback_t_bytes(N, jobs, n_jobs, epi, wtype, xtype, K, num_cus);
     size_t need = 0;
     for (uint32_t i = 0; i < n_jobs; i += 2) {
@@ -1818,7 +1822,8 @@ size_t batch_matmul_multi_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32
             continue;
         }
         for (uint32_t q = i; q < i + n; q++)
-            need = max(need, t + batch_matmul_workspace_bytes(wtype, xtype, N, K, jobs[q].M, num_cus));
+            need = max(need, t + batch_matmul_workspace_bytes(wtype, xtype, N, K, jobs[q].M, num_cus, kNoWorkspaceLimit,
+                                                              cut_tiles));
     }
     return need;
 }
@@ -1872,7 +1877,7 @@ hipError_t finish_next_images(const NextImageSet& nx, uint32_t otype, uint32_t f
 
 hipError_t launch_batch_matmul_multi(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, const GemmJob* jobs,
                                      uint32_t n_jobs, const GemmEpilogue& epi, int num_cus, void* ws,
-                                     hipStream_t st, const void* const* images, const NextImageSet* next) {
+                                     hipStream_t st, const void* const* images, const NextImageSet* next, bool cut_tiles) {
     if (next && (next->count == 0 || next->count > kMaxNextImages || (xtype != kGgmlF16 && xtype != kGgmlBF16)))
         return hipErrorInvalidValue;
     uint32_t fused = 0;  // next-image items the last group's GEMM builds
@@ -1935,7 +1940,7 @@ hipError_t launch_batch_matmul_multi(uint32_t wtype, uint32_t xtype, uint32_t N,
         } else {
             for (uint32_t q = i; q < i + n && e == hipSuccess; q++)
                 e = run_job_fallback(wtype, xtype, N, K, jobs[q], epi, num_cus, (float*)ws,
-                                     (uint8_t*)ws + t_bytes, st);
+                                     (uint8_t*)ws + t_bytes, cut_tiles, st);
         }
         if (e != hipSuccess) return e;
     }

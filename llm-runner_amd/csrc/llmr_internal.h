@@ -22,15 +22,15 @@ hipError_t launch_dequant_operand_f16(const void* w, uint32_t wtype, uint32_t n_
 // to fp16, split-K partials of launches with few tiles and, from a few
 // thousand tokens, the 16-bit weight image of the two-pass path. With a
 // ws_limit the plan keeps within it where a smaller form exists (the
-// one-pass kernels instead of the image, fewer splits); pass the same limit
-// to both calls.
+// one-pass kernels instead of the image, fewer splits), without cut_tiles no
+// tile is cut along K; pass the same limit and cut_tiles to both calls.
 using plan::kNoWorkspaceLimit;
 size_t batch_matmul_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, uint32_t M,
-                                    int num_cus, size_t ws_limit = kNoWorkspaceLimit);
+                                    int num_cus, size_t ws_limit = kNoWorkspaceLimit, bool cut_tiles = true);
 hipError_t launch_batch_matmul(const void* w, uint32_t wtype, const void* x, uint32_t xtype,
                                float* y, uint32_t out_dim, uint32_t in_dim, uint32_t seq_len,
                                uint32_t row_offset, int num_cus, void* ws, hipStream_t st,
-                               size_t ws_limit = kNoWorkspaceLimit);
+                               size_t ws_limit = kNoWorkspaceLimit, bool cut_tiles = true);
 
 // Several GEMMs of one shape (N, K, weight and activation types) with a
 // shared epilogue (kind kEpi* of gemm_q.hip: 0 store, 1 gated residual
@@ -69,7 +69,7 @@ struct NextImageSet;  // the next GEMM group's weight images (below)
 // (launch_batch_matmul_multi's `images`), so the workspace holds none.
 size_t batch_matmul_multi_workspace_bytes(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K,
                                           const GemmJob* jobs, uint32_t n_jobs, const GemmEpilogue& epi,
-                                          int num_cus, bool prebuilt_images = false);
+                                          int num_cus, bool prebuilt_images = false, bool cut_tiles = true);
 // Q4_K projections of at most kGemvMaxTokens tokens, one launch for up to
 // 64 jobs of one shape [N, K] with plain stores (rows ldy apart);
 // hipErrorNotSupported when a job does not fit the LDS-staged kernel.
@@ -81,7 +81,7 @@ hipError_t launch_gemv_q4k_multi(uint32_t xtype, const GemmJob* jobs, uint32_t n
 hipError_t launch_batch_matmul_multi(uint32_t wtype, uint32_t xtype, uint32_t N, uint32_t K, const GemmJob* jobs,
                                      uint32_t n_jobs, const GemmEpilogue& epi, int num_cus, void* ws,
                                      hipStream_t st, const void* const* images = nullptr,
-                                     const NextImageSet* next = nullptr);
+                                     const NextImageSet* next = nullptr, bool cut_tiles = true);
 
 // LoRA (lora.hip): the two-hop correction appended to a base GEMM output and
 // the load-time Q8_0 merge. Ranks above kMaxLoraRank are not taken (the

@@ -28,6 +28,10 @@ static void check(uint32_t wt, uint32_t xt, uint32_t N, uint32_t K, uint32_t M, 
     const GemmPlan p = plan_gemm(wt, xt, N, K, M, cus, limit);
     const uint32_t S = K / kStageK;
     n_checked++;
+    const GemmPlan w = plan_gemm(wt, xt, N, K, M, cus, limit, false);
+    if (w.split > 1 || w.ws > limit) fail("plan without cut tiles", wt, xt, N, K, M, cus, limit);
+    if (p.split <= 1 && (w.ws != p.ws || w.few != p.few || w.persistent != p.persistent || w.skinny != p.skinny))
+        fail("cut_tiles changes a plan that cuts none", wt, xt, N, K, M, cus, limit);
     if (p.few + p.skinny + p.persistent + (p.split > 1) > 1) fail("more than one kernel", wt, xt, N, K, M, cus, limit);
     if (p.ws > limit) fail("workspace beyond the limit", wt, xt, N, K, M, cus, limit);
     if (p.few) {

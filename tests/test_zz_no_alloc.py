@@ -148,3 +148,51 @@ def test_noalloc_two_streams_of_one_context(dev):
     ctx.close()
     for y, r in zip(ys, refs):
         assert torch.equal(y, r)
+
+
+def test_captured_gemm_takes_no_workspace(dev):
+    """Launches whose tiles are cut along K outside a capture (partial tiles in
+    the workspace) need none under one: a context that holds no workspace
+    captures llmr_batch_matmul, and llmr_batch_matmul_noalloc after the scratch
+    was used on another stream; every replay, with the context's own work and a
+    larger workspace between, gives the eager result to f32 summation order."""
+    from conftest import rel_l2
+    from llmr_amd import capi, ops
+    wtype, N, K, M = 12, 3840, 5120, 600  # 45 tiles cut into 3, 2 within the scratch
+    w, x = _weights(dev, wtype, N, K, 41), _x(dev, M, K, BF16, 42)
+    ws, xs = _weights(dev, wtype, 512, 10240, 43), _x(dev, 64, 10240, F32, 44)  # split-K partials
+    g = ops.default_graph()
+    g.bind_stream()
+    y_ref = torch.empty((M, N), device=dev)
+    g.ctx.batch_matmul(w.data_ptr(), wtype, x.data_ptr(), BF16, y_ref.data_ptr(), N, K, M, 0)
+    ys = torch.empty((64, 512), device=dev)
+    ctx = capi.Context(0)
+    side = torch.cuda.Stream()
+    main = torch.cuda.current_stream().cuda_stream
+
+    def scratch_call():
+        ctx.batch_matmul_noalloc(ws.data_ptr(), wtype, xs.data_ptr(), F32, ys.data_ptr(), 512, 10240, 64, 0)
+
+    ctx.set_stream(main)
+    scratch_call()
+    torch.cuda.synchronize()
+    ctx.set_stream(side.cuda_stream)
+    y, y_na = (torch.empty((M, N), device=dev) for _ in range(2))
+    graph = torch.cuda.CUDAGraph()
+    print("capture of 600 x 3840 x 5120 Q4_K bf16", flush=True)
+    with torch.cuda.graph(graph, stream=side):
+        ctx.batch_matmul(w.data_ptr(), wtype, x.data_ptr(), BF16, y.data_ptr(), N, K, M, 0)
+        ctx.batch_matmul_noalloc(w.data_ptr(), wtype, x.data_ptr(), BF16, y_na.data_ptr(), N, K, M, 0)
+    ctx.set_stream(main)
+    y_big = torch.empty((2 * M, N), device=dev)
+    for i in range(3):
+        y.fill_(7.0)
+        y_na.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        for t in (y, y_na):
+            assert rel_l2(t.cpu().numpy(), y_ref.cpu().numpy()) <= 1e-5, i
+        scratch_call()
+        ctx.batch_matmul(w.data_ptr(), wtype, x.data_ptr(), BF16, y_big[i * 4:].data_ptr(), N, K, M - 100 * (2 - i), 0)
+        torch.cuda.synchronize()
+    ctx.close()
