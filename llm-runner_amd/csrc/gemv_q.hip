@@ -13,6 +13,7 @@
 // is (d*sc)*q - dmin*mn with one rounding (the FMA; both products are exact).
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <type_traits>
 
 #include "llmr_device.h"
@@ -701,9 +702,17 @@ template <uint32_t WT, uint32_t XT, int T, uint32_t CAP, uint32_t KS>
 hipError_t launch_gemv_k(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
                          uint32_t waves, hipStream_t st) {
     auto kern = gemv_i8_kernel<WT, XT, T, CAP, KS>;
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvLdsLimit);
-    if (attr != hipSuccess) return attr;
+    // more than 64 KiB of LDS: an attribute of the kernel on each device
+    static std::atomic<uint64_t> allowed{0};  // by device
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = dev < 64 ? 1ull << dev : 0ull;
+    if (!(allowed.load(std::memory_order_acquire) & bit)) {
+        e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGemvLdsLimit);
+        if (e != hipSuccess) return e;
+        allowed.fetch_or(bit, std::memory_order_release);
+    }
     const uint32_t rows = 16u * waves / KS, bpj = (N + rows - 1u) / rows;
     hipLaunchKernelGGL(kern, dim3(bpj * n_jobs), dim3(64u * waves), (gemv_lds_bytes<WT, T>(K, waves)), st, jobs, N, K,
                        ldy, bpj, waves);
