@@ -138,6 +138,46 @@ int main() {
             }
         }
     }
+    // what the GPU tests' launches run, so that each reaches the kernel it names
+    {
+        enum Route { kTiled, kFew32, kFew96, kSkinny, kCut, kPersist };
+        const size_t none = kNoWorkspaceLimit, scratch = LLMR_NOALLOC_SCRATCH_BYTES;
+        struct {
+            uint32_t wt, xt, N, K, M;
+            size_t limit;
+            Route route;
+            bool ws;
+        } const c[] = {
+            // test_gpu_gemm.py: test_gemm_parity, test_few_token_tiles, test_split_tiles
+            {kQ8_0, kF32, 516, 8256, 33, none, kSkinny, true},    {kQ4K, kF32, 512, 8448, 100, none, kSkinny, true},
+            {kQ8_0, kF16, 640, 12352, 17, none, kSkinny, true},   {kQ4K, kBF16, 1540, 8192, 200, none, kSkinny, true},
+            {kQ4K, kBF16, 3077, 1024, 77, none, kFew32, false},   {kQ4K, kF32, 1028, 768, 300, none, kFew32, false},
+            {kQ8_0, kBF16, 1024, 1088, 512, none, kFew32, false}, {kQ8_0, kBF16, 3072, 640, 250, none, kFew96, false},
+            {kQ8_0, kF32, 3840, 3840, 1101, none, kCut, true},    {kQ4K, kF32, 3072, 3072, 1101, none, kCut, true},
+            {kQ8_0, kBF16, 2052, 5120, 513, none, kCut, true},    {kQ4K, kF16, 2052, 5120, 513, none, kCut, true},
+            {kQ8_0, kBF16, 11520, 1088, 1536, none, kCut, true},  {kQ4K, kBF16, 9216, 3072, 2047, none, kCut, true},
+            {kQ8_0, kF16, 2052, 2048, 2049, none, kCut, true},
+            // test_zz_no_alloc.py
+            {kQ8_0, kF32, 3072, 3072, 64, scratch, kFew32, false},
+            {kQ4K, kF32, 3840, 10240, 64, scratch, kSkinny, true}, {kQ4K, kF32, 3840, 10240, 33, scratch, kSkinny, true},
+            {kQ4K, kF32, 4096, 1024, 2304, scratch, kPersist, true}, {kQ4K, kBF16, 12288, 3072, 2560, scratch, kPersist, false},
+            {kQ4K, kBF16, 3072, 3072, 4608, scratch, kPersist, true}, {kQ4K, kBF16, 3072, 3072, 2048, scratch, kTiled, false},
+            {kQ8_0, kF16, 1000, 12352, 200, scratch, kSkinny, true}, {kQ8_0, kF16, 1000, 12352, 40, scratch, kSkinny, true},
+            {kQ8_0, kBF16, 3840, 5120, 600, scratch, kCut, true},  {kQ8_0, kBF16, 3840, 5120, 513, scratch, kCut, true},
+            {kQ4K, kF32, 512, 10240, 64, scratch, kSkinny, true},  {kQ4K, kF32, 4096, 4096, 4608, scratch, kTiled, false},
+        };
+        for (const auto& s : c) {
+            const GemmPlan p = plan_gemm(s.wt, s.xt, s.N, s.K, s.M, 256, s.limit);
+            const Route r = p.few ? (p.few_features == kFewNarrow ? kFew32 : kFew96)
+                            : p.skinny ? kSkinny : p.split > 1 ? kCut : p.persistent ? kPersist : kTiled;
+            n_checked++;
+            if (r != s.route || (p.ws > 0) != s.ws) {
+                std::printf("FAIL %u x %u x %u: a test's launch runs kernel %d (%zu bytes), not %d\n", s.M, s.N, s.K, r,
+                            p.ws, s.route);
+                return 1;
+            }
+        }
+    }
     // a limit that holds fewer parts than the launch is cut into without one
     {
         const GemmPlan a = plan_gemm(kQ8_0, kBF16, 3840, 3840, 1101, 256);

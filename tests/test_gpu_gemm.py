@@ -42,14 +42,14 @@ CASES = [
     (8, 65, 130, 256, 1, 64),        # f16, row_offset into a fused weight
     (8, 7, 33, 96, 0, 3),            # K % 64 == 32: generic kernel; N not a multiple of 4
     (8, 1, 64, 64, 30, 0),           # one token
-    (8, 300, 520, 1024, 30, 8),      # 128x128 tiles, ragged
+    (8, 300, 520, 1024, 30, 8),      # ragged, past 256 tokens
     (12, 77, 130, 512, 0, 0),        # Q4_K f32
     (12, 129, 256, 1024, 30, 256),   # Q4_K bf16 with row_offset
     (12, 513, 1032, 768, 1, 0),      # Q4_K f16, ragged
     (12, 1, 17, 256, 30, 1),         # one token, odd N (small-M Q4_K kernel)
     (12, 3, 1000, 768, 1, 4),        # small-M Q4_K kernel, f16, row_offset
     (12, 4, 130, 512, 30, 0),        # small-M Q4_K kernel at its largest M
-    (12, 5, 72, 512, 30, 0),         # one token more: the tiled kernel again
+    (12, 5, 72, 512, 30, 0),         # one token more: the few-token kernel
     # few tokens with at least half the CUs' worth of 32 x 96 tiles: the
     # few-token kernel (one launch, the waves of a workgroup split K)
     (8, 250, 3001, 3264, 30, 5),     # ragged M, odd N, 51 stages (not a multiple of the 8 waves), bf16
@@ -57,18 +57,25 @@ CASES = [
     (8, 129, 4000, 1024, 1, 0),      # one token in the last token tile, f16
     (12, 64, 12288, 512, 1, 0),      # Q4_K f16, two token tiles
     (12, 256, 3072, 3072, 30, 0),    # Q4_K bf16 at the single-linear size
-    # few tokens over few features, N % 4 == 0: the skinny kernel (all tokens x
-    # 64 features per workgroup, K split across workgroups)
+    # few tokens over few features: 32-feature tiles
     (8, 200, 1000, 768, 30, 8),      # ragged M and N, bf16, row_offset
-    (8, 33, 64, 4096, 0, 0),         # one feature tile: 16 K splits, f32
-    (12, 250, 3072, 3072, 1, 0),     # Q4_K f16 at the single-linear size
-    (12, 256, 21504, 1024, 30, 0),   # 336 feature tiles: no split
-    (8, 17, 128, 192, 1, 0),         # three stages: one split, short pipeline
-    (12, 100, 256, 1024, 0, 256),    # Q4_K, f32 activations packed to fp16, row_offset
+    (8, 33, 64, 4096, 0, 0),         # two feature tiles, f32
+    (12, 250, 3072, 3072, 1, 0),     # Q4_K f16 at the single-linear size (96-feature tiles)
+    (12, 256, 21504, 1024, 30, 0),   # 1792 tiles of 96 features
+    (8, 17, 128, 192, 1, 0),         # three stages: five waves without
+    (12, 100, 256, 1024, 0, 256),    # Q4_K, f32 activations as bf16, row_offset
+    # the skinny kernel (all tokens x 64 features per workgroup, K split across
+    # workgroups)
+    (8, 33, 516, 8256, 0, 4),        # f32 as fp16: 26 splits of 129 stages, four features past a tile
+    (12, 100, 512, 8448, 0, 0),      # f32 as bf16
+    (8, 17, 640, 12352, 1, 0),       # f16, read in place
+    (12, 200, 1540, 8192, 30, 8),    # bf16, row_offset, ragged M and N
 ]
 
 
-@pytest.mark.parametrize("M,N,K,row_offset", [(1, 18432, 3072, 0), (1, 3072, 256, 0), (4, 264, 4096, 16)])
+@pytest.mark.parametrize("M,N,K,row_offset", [(1, 18432, 3072, 0), (1, 3072, 256, 0), (4, 264, 4096, 16),
+                                              # rows whose digits do not fit the LDS: the f32 kernel
+                                              (2, 72, 15360, 0), (3, 41, 6400, 8), (4, 130, 12288, 16)])
 def test_small_m_q4k_f32_matches_reference_arithmetic(orc, dev, M, N, K, row_offset):
     """M <= 4 Q4_K launches keep the activations in f32 and sum the
     f32 products of batch_matmul_q4k's dequantized weights (per sub-block as
@@ -406,7 +413,7 @@ def test_persistent_every_tile(dev, wtype, M, N, K, xtype, row_offset):
     (12, 77, 3077, 1024, 30, 8),   # 32-feature tiles: a last one of 5, N % 4 != 0
     (8, 33, 1000, 576, 0, 4),      # nine stages over eight waves, f32 as fp16
     (8, 5, 36, 64, 1, 0),          # one stage: seven waves without
-    (12, 300, 1030, 768, 0, 0),    # past 256 tokens, f32 as bf16
+    (12, 300, 1028, 768, 0, 0),    # past 256 tokens, f32 as bf16
     (8, 512, 1024, 1088, 30, 2),   # the most tokens, 17 stages
     (8, 250, 3072, 640, 30, 0),    # 96-feature tiles
 ])
@@ -441,7 +448,7 @@ SPLIT_TILE_CASES = [
     # (wtype, M, N, K, xtype, row_offset)
     (8, 1101, 3840, 3840, 0, 0),     # 75 tiles x 3 splits of 20 stages, f32 activations as fp16
     (12, 1101, 3072, 3072, 0, 8),    # 60 tiles x 4, f32 activations as bf16, row_offset
-    (8, 257, 1028, 2048, 30, 0),     # one row and four features past a tile
+    (8, 513, 2052, 5120, 30, 0),     # one row and four features past a tile
     (12, 513, 2052, 5120, 1, 4),     # splits of unequal stage counts
     (8, 1536, 11520, 1088, 30, 0),   # 256 whole tiles, 14 cut into splits of 17 stages in all
     (12, 2047, 9216, 3072, 30, 0),   # 256 whole tiles, 32 x 8

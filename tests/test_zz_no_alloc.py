@@ -45,19 +45,23 @@ def _both(dev, w, wtype, x, xtype, N, row_offset=0):
 # scratch holds). Where llmr_batch_matmul's plan fits the array both calls run
 # the same kernels (same bits); a launch whose weight image does not fit runs
 # the one-pass kernels (same bits as the two-pass path); one whose split-K
-# partials do not fit runs fewer splits (the same sums in another order:
-# compared to f32 rounding, far inside the GEMM bar of relative L2 1e-2).
+# partials or partial tiles do not fit runs fewer splits or another kernel (the
+# same sums in another order: compared to f32 rounding, far inside the GEMM bar
+# of relative L2 1e-2; `exact` False for that launch). tests/c/plan_check.cpp
+# pins what each of these launches holds in the scratch.
 CASES = [
-    (8, F32, 3072, 3072, (256, 64), 0, "nothing (the single Q8_0 linear), then split-K partials"),
-    (12, F32, 4096, 1024, (4096, 2304), 8, "f32 activations as bf16 + the weight image"),
-    (12, BF16, 12288, 3072, (2560, 2304), 0, "nothing: one-pass in place of a 75 MB weight image"),
-    (12, BF16, 3072, 3072, (4608, 2048), 0, "the weight image; then fewer splits than llmr_batch_matmul"),
-    (8, F16, 1000, 2048, (300, 40), 4, "split-K partials, ragged N"),
+    (8, F32, 3072, 3072, (256, 64), 0, (True, True), "nothing (the few-token kernel)"),
+    (12, F32, 3840, 10240, (64, 33), 0, (True, True), "packed activations and split-K partials"),
+    (12, F32, 4096, 1024, (4096, 2304), 8, (True, True), "f32 activations as bf16 + the weight image"),
+    (12, BF16, 12288, 3072, (2560, 2304), 0, (True, True), "nothing: one-pass in place of a 75 MB weight image"),
+    (12, BF16, 3072, 3072, (4608, 2048), 0, (True, False), "the weight image; then no partials"),
+    (8, F16, 1000, 12352, (200, 40), 4, (True, True), "split-K partials, ragged N"),
+    (8, BF16, 3840, 5120, (600, 513), 0, (False, False), "partial tiles, in fewer parts"),
 ]
 
 
-@pytest.mark.parametrize("wtype,xtype,N,K,Ms,row_offset,what", CASES)
-def test_noalloc_matches_batch_matmul_twice(dev, wtype, xtype, N, K, Ms, row_offset, what):
+@pytest.mark.parametrize("wtype,xtype,N,K,Ms,row_offset,exact,what", CASES)
+def test_noalloc_matches_batch_matmul_twice(dev, wtype, xtype, N, K, Ms, row_offset, exact, what):
     from conftest import rel_l2
     w = _weights(dev, wtype, N + row_offset, K, 60 + wtype)
     for i, M in enumerate(Ms):
@@ -67,11 +71,10 @@ def test_noalloc_matches_batch_matmul_twice(dev, wtype, xtype, N, K, Ms, row_off
         assert bool(torch.isfinite(y_ref).all())
         assert bool(torch.isfinite(y).all())
         err = rel_l2(y.cpu().numpy(), y_ref.cpu().numpy())
-        exact = torch.equal(y, y_ref)
-        print(f"  rel L2 {err:.2e}, identical {exact}")
+        same = torch.equal(y, y_ref)
+        print(f"  rel L2 {err:.2e}, identical {same}")
         assert err <= 1e-5, (M, err)
-        if not (wtype == 12 and xtype == BF16 and N == 3072 and M == 2048):
-            assert exact, M
+        assert same or not exact[i], M
 
 
 def test_noalloc_f32_beyond_scratch_runs_tiled(dev):
@@ -94,10 +97,11 @@ def test_noalloc_f32_beyond_scratch_runs_tiled(dev):
 def test_noalloc_allocates_nothing_on_a_fresh_context(dev):
     """A context that has never run a GEMM calls only llmr_batch_matmul_noalloc,
     on launches whose plans use scratch (split-K partials, a 16-bit copy of f32
-    activations, a weight image): the device's free memory is the same before
+    activations, a weight image, partial tiles): the device's free memory is the same before
     and after. (The kernels' code is loaded first through another context.)"""
     from llmr_amd import capi, ops
-    cases = [(8, F32, 3072, 3072, 64), (12, F32, 4096, 1024, 2304), (12, BF16, 3072, 3072, 4608)]
+    cases = [(12, F32, 512, 10240, 64), (12, F32, 4096, 1024, 2304), (12, BF16, 3072, 3072, 4608),
+             (8, BF16, 3840, 5120, 600)]
     data = []
     for wtype, xtype, N, K, M in cases:
         w = _weights(dev, wtype, N, K, 90 + wtype)
@@ -128,22 +132,22 @@ def test_noalloc_two_streams_of_one_context(dev):
     waits for the first stream's work up to the switch, so both results are
     llmr_batch_matmul's."""
     from llmr_amd import capi
-    N, K = 3072, 3072
-    w = _weights(dev, 8, N, K, 31)
+    N, K = 3840, 10240
+    w = _weights(dev, 12, N, K, 31)
     xs = [_x(dev, 64, K, F32, 11), _x(dev, 64, K, F32, 12)]
     ys = [torch.full((64, N), -1.0, device=dev) for _ in xs]
     refs = [torch.empty((64, N), device=dev) for _ in xs]
     ctx = capi.Context(0)
     s0, s1 = torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
-    print("noalloc on two streams of one context: 64 x 3072 x 3072 Q8_0 f32 (split-K partials)", flush=True)
+    print("noalloc on two streams of one context: 64 x 3840 x 10240 Q4_K f32 (split-K partials)", flush=True)
     for st, x, y in ((s0, xs[0], ys[0]), (s1, xs[1], ys[1])):
         ctx.set_stream(st.cuda_stream)
-        ctx.batch_matmul_noalloc(w.data_ptr(), 8, x.data_ptr(), F32, y.data_ptr(), N, K, 64, 0)
+        ctx.batch_matmul_noalloc(w.data_ptr(), 12, x.data_ptr(), F32, y.data_ptr(), N, K, 64, 0)
     ctx.set_stream(torch.cuda.current_stream().cuda_stream)
     torch.cuda.synchronize()
     for x, r in zip(xs, refs):
-        ctx.batch_matmul(w.data_ptr(), 8, x.data_ptr(), F32, r.data_ptr(), N, K, 64, 0)
+        ctx.batch_matmul(w.data_ptr(), 12, x.data_ptr(), F32, r.data_ptr(), N, K, 64, 0)
     torch.cuda.synchronize()
     ctx.close()
     for y, r in zip(ys, refs):
@@ -158,9 +162,9 @@ def test_captured_gemm_takes_no_workspace(dev):
     larger workspace between, gives the eager result to f32 summation order."""
     from conftest import rel_l2
     from llmr_amd import capi, ops
-    wtype, N, K, M = 12, 3840, 5120, 600  # 45 tiles cut into 3, 2 within the scratch
+    wtype, N, K, M = 8, 3840, 5120, 600  # 45 tiles, cut into fewer parts within the scratch
     w, x = _weights(dev, wtype, N, K, 41), _x(dev, M, K, BF16, 42)
-    ws, xs = _weights(dev, wtype, 512, 10240, 43), _x(dev, 64, 10240, F32, 44)  # split-K partials
+    ws, xs = _weights(dev, 12, 512, 10240, 43), _x(dev, 64, 10240, F32, 44)  # split-K partials
     g = ops.default_graph()
     g.bind_stream()
     y_ref = torch.empty((M, N), device=dev)
@@ -171,7 +175,7 @@ def test_captured_gemm_takes_no_workspace(dev):
     main = torch.cuda.current_stream().cuda_stream
 
     def scratch_call():
-        ctx.batch_matmul_noalloc(ws.data_ptr(), wtype, xs.data_ptr(), F32, ys.data_ptr(), 512, 10240, 64, 0)
+        ctx.batch_matmul_noalloc(ws.data_ptr(), 12, xs.data_ptr(), F32, ys.data_ptr(), 512, 10240, 64, 0)
 
     ctx.set_stream(main)
     scratch_call()
@@ -179,7 +183,7 @@ def test_captured_gemm_takes_no_workspace(dev):
     ctx.set_stream(side.cuda_stream)
     y, y_na = (torch.empty((M, N), device=dev) for _ in range(2))
     graph = torch.cuda.CUDAGraph()
-    print("capture of 600 x 3840 x 5120 Q4_K bf16", flush=True)
+    print("capture of 600 x 3840 x 5120 Q8_0 bf16", flush=True)
     with torch.cuda.graph(graph, stream=side):
         ctx.batch_matmul(w.data_ptr(), wtype, x.data_ptr(), BF16, y.data_ptr(), N, K, M, 0)
         ctx.batch_matmul_noalloc(w.data_ptr(), wtype, x.data_ptr(), BF16, y_na.data_ptr(), N, K, M, 0)
