@@ -157,6 +157,8 @@ int main() {
             {kQ8_0, kBF16, 2052, 5120, 513, none, kCut, true},    {kQ4K, kF16, 2052, 5120, 513, none, kCut, true},
             {kQ8_0, kBF16, 11520, 1088, 1536, none, kCut, true},  {kQ4K, kBF16, 9216, 3072, 2047, none, kCut, true},
             {kQ8_0, kF16, 2052, 2048, 2049, none, kCut, true},
+            {kQ4K, kF32, 256, 512, 100, none, kFew32, false},     {kQ4K, kF32, 512, 8448, 77, none, kSkinny, true},
+            {kQ4K, kF32, 520, 512, 600, none, kTiled, true},
             // test_zz_no_alloc.py
             {kQ8_0, kF32, 3072, 3072, 64, scratch, kFew32, false},
             {kQ4K, kF32, 3840, 10240, 64, scratch, kSkinny, true}, {kQ4K, kF32, 3840, 10240, 33, scratch, kSkinny, true},

@@ -622,8 +622,10 @@ def test_bf16_activations_beyond_fp16_range(orc, dev, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,path", [(2048, 4096, 256, "two-pass"), (1024, 8192, 256, "persistent"),
-                                        (256, 3072, 256, "few-token"), (100, 256, 512, "skinny"),
-                                        (300, 520, 512, "tiled"), (3, 1000, 512, "gemv")])
+                                        (256, 3072, 256, "few-token"), (100, 256, 512, "32-feature tiles"),
+                                        (77, 512, 8448, "skinny"), (600, 520, 512, "tiled"),
+                                        (1101, 3072, 3072, "cut tiles"), (3, 1000, 512, "gemv"),
+                                        (3, 100, 6400, "gemv, f32 rows")])
 def test_q4k_f32_activations_beyond_fp16_range(orc, dev, M, N, K, path):
     """f32 activations of magnitude ~1e5 against Q4_K weights stay finite and
     match the oracle on every kernel path: batch_matmul_q4k multiplies x in
