@@ -22,8 +22,8 @@ constexpr uint32_t kQ8_0 = LLMR_GGML_Q8_0, kQ4K = LLMR_GGML_Q4_K;
 
 constexpr uint32_t kStageK = 64;          // K per stage of every MFMA kernel
 constexpr uint32_t kImageBlock = 256u * 128u;  // bytes of one 256-row x 64-wide 16-bit image block
-// Q4_K weights times at most this many tokens run on the GEMV kernel (an
-// HBM-bound weight stream, gemv_q.hip).
+// Weights times at most this many tokens run on the GEMV kernels (an HBM-bound
+// weight stream, gemv_q.hip): Q4_K always, Q8_0 where gemv_q8_fits.
 constexpr uint32_t kGemvMaxTokens = 4;
 // From this many tokens the weight is dequantized once per call into a
 // 16-bit image (gemm_w16.hip) instead of once per 256-token tile.

@@ -1,7 +1,7 @@
 // Dequant-GEMM for few tokens (M <= 256): batch_matmul_q8 / batch_matmul_q4k
-// (llm.slang:1639-1767, :2277-2365) with f32 activations and rows past K = 8192,
-// where re-reading them per 32 features costs more than packing them once
-// (plan::few_features).
+// (llm.slang:1639-1767, :2277-2365) with long rows, where the few-token kernel's
+// waves walk too many K stages one after the other, or re-read f32 activations per
+// 32 features at more than it costs to pack them once (plan::few_features).
 //
 // Workgroup (n tile, split z) computes all M tokens x 64 features over the K
 // stages [z per, min(S, (z + 1) per)): the activations are read by N / 64

@@ -180,9 +180,12 @@ __global__ void __launch_bounds__(256) gemv_q4k_kernel(const uint8_t* __restrict
 // LDS holds three workgroups per CU. KS waves share 16 rows (each takes every
 // KS-th step), so that launches of few rows still put work on every CU.
 // Measured per call, before -> after (one token, FMA kernel; Q8_0, the few-token
-// GEMMs): 18432 x 3072 Q4_K 19.5 -> 9.7 us (3.3 TB/s), 38 of them grouped 328
+// GEMMs): 18432 x 3072 Q4_K 19.5 -> 8.9 us (3.6 TB/s), 38 of them grouped 328
 // -> 210 us (5.8 TB/s), 3072 x 15360 76 -> 12, two and four tokens of 18432 x
-// 3072 31 -> 15 and 56 -> 26 us; 11520 x 3840 Q8_0 54 -> 9.8 us (4.8 TB/s).
+// 3072 31 -> 14 and 56 -> 17 us; 11520 x 3840 Q8_0 54 -> 9.8 us (4.8 TB/s).
+// At three and four tokens over more rows than 64 a CU the Q8_0 few-token GEMM is
+// the faster one from K = 4096 on (18432 x 6144 27 against 31 us), with the
+// activations rounded to fp16: 2e-4 against 64 bits where this leaves 1e-7.
 // ---------------------------------------------------------------------------
 
 // Up to CAP projections of one shape [N, K] (each its own weight, input
@@ -721,9 +724,9 @@ hipError_t launch_gemv_k(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N,
 
 // Fewer than 128 workgroups of 64 rows leave half the CUs without one: the
 // four waves then share 16 rows (one token, 3072 x 15360 Q4_K: 24 -> 12 us; four
-// tokens, 3072 x 3072: 13.6 -> 9.4). From 128 on it costs more, as every
-// workgroup cuts the activations into digits (four tokens, 9216 x 3072: 13.7
-// against 25 us; one token, 18432 x 3072: 9.7 against 11.1).
+// tokens, 3072 x 3072: 13.6 -> 8.4). From 128 on it costs more, as every
+// workgroup cuts the activations into digits (four tokens, 9216 x 3072: 13.4
+// against 25 us; one token, 18432 x 3072: 9.7 against 11.1 before gemv_waves).
 template <uint32_t WT, uint32_t XT, int T, uint32_t CAP>
 hipError_t launch_gemv_t(const GemvJobs<CAP>& jobs, uint32_t n_jobs, uint32_t N, uint32_t K, uint32_t ldy,
                          int num_cus, hipStream_t st) {
