@@ -131,26 +131,28 @@ inline bool few_fits(uint32_t wtype, uint32_t N, uint32_t K, uint32_t M) {
 // 256 CUs, 96 -> 32 features: 77 x 9216 x 3072 Q4_K bf16 27.2 -> 19.2 us, 200 x 3840
 // x 3840 31.0 -> 22.7, 64 x 9216 x 3072 15.2 / 15.7, 200 x 3072 x 3072 15.2 / 15.4,
 // Q8_0 f32 15.7 / 21.0, 200 x 21504 x 15360 Q8_0 bf16 414 / 508, 150 x 21504 x 8192
-// 155 / 170.
+// 155 / 170; where both come close, within a quarter (113 x 9368 x 10240 72 / 93, 256
+// x 2048 x 8192 31 / 26, the 32-feature tiles both).
 // Below half the CUs' worth of 96-feature tiles the 32-feature tiles take 77 x 3072
 // x 4096 Q4_K bf16 in 12.8 us against the skinny kernel's 19.5 (packed activations,
 // K splits, partial sums: three launches), 32 x 3840 x 3840 8.7 against 19.6, 5 x
 // 9216 x 3072 10.5 against 43. The skinny kernel is the better one where a wave's K
 // stages, one after the other, are most of the time: f32 activations with long rows
-// (77 x 3072 x 12288 43 against 48 us; past 12288 with few features too, 150 x 64 x
-// 15360 28 against 34, tiled 23), 16-bit ones past 12288 where its splits still fill
-// the CUs with whole rounds (5 x 512 x 15360 19.6 against 23.6; bf16 x 256 and x
-// 1024 0.86-0.97 the other way, f16 33 x 1024 22.4 against 25.6), and long rows
-// where some CUs get a second tile (200 x 1536 x 8192 26 against 35, 150 x 2048 x
-// 15360 bf16 36 against 48).
+// (77 x 3072 x 12288 43 against 48 us; from 14336 with few features too, 150 x 64 x
+// 15360 28 against 34, tiled 23), 16-bit ones from 14336 with 257 to 1024 features
+// (few-token : skinny at 512 features 0.98 at K = 12288, 1.02-1.13 at 14336,
+// 1.03-1.20 at 15360; at 64 and 256 0.9-1.0 up to 16384, 1.0-1.1 past it), and long
+// rows where some CUs get a second tile (200 x 1536 x 8192 26 against 35, 150 x
+// 2048 x 15360 bf16 36 against 48).
 inline uint32_t few_features(uint32_t xtype, uint32_t N, uint32_t K, uint32_t M, int num_cus) {
     const uint64_t tm = (M + kFewTokens - 1) / kFewTokens, c = (uint64_t)num_cus;
     const uint64_t wide = tm * ((N + kFewFeatures - 1) / kFewFeatures), narrow = tm * ((N + kFewNarrow - 1) / kFewNarrow);
     const bool f32 = xtype == kF32;
     if (2 * wide < c) {
         const bool skinny = N % 4 == 0 && ((f32 && K > 8192 && N >= 512) || (narrow > c && K >= 8192 && N < 3072) ||
-                                           (K > 12288 && (xtype == kF16 ? N <= 1024 : N > 256 && N < 1024)));
-        return skinny || (f32 && K > 12288) ? 0u : kFewNarrow;
+                                           (!f32 && K >= 14336 && N > 256 && N <= 1024) ||
+                                           (!f32 && K > 16384 && N <= 1024));
+        return skinny || (f32 && K >= 14336 && N < 512) ? 0u : kFewNarrow;
     }
     const double f = f32 ? (K > 8192 ? 1.6 : 1.3) : K >= 8192 ? 1.14 : 1.03;
     return f * narrow + 0.7 * c < 3.0 * c * ((wide + c - 1) / c) ? kFewNarrow : kFewFeatures;

@@ -150,7 +150,7 @@ int main() {
         } const c[] = {
             // test_gpu_gemm.py: test_gemm_parity, test_few_token_tiles, test_split_tiles
             {kQ8_0, kF32, 516, 8256, 33, none, kSkinny, true},    {kQ4K, kF32, 512, 8448, 100, none, kSkinny, true},
-            {kQ8_0, kF16, 640, 12352, 17, none, kSkinny, true},   {kQ4K, kBF16, 1540, 8192, 200, none, kSkinny, true},
+            {kQ8_0, kF16, 640, 14400, 17, none, kSkinny, true},   {kQ4K, kBF16, 1540, 8192, 200, none, kSkinny, true},
             {kQ4K, kBF16, 3077, 1024, 77, none, kFew32, false},   {kQ4K, kF32, 1028, 768, 300, none, kFew32, false},
             {kQ8_0, kBF16, 1024, 1088, 512, none, kFew32, false}, {kQ8_0, kBF16, 3072, 640, 250, none, kFew96, false},
             {kQ8_0, kF32, 3840, 3840, 1101, none, kCut, true},    {kQ4K, kF32, 3072, 3072, 1101, none, kCut, true},
@@ -164,7 +164,7 @@ int main() {
             {kQ4K, kF32, 3840, 10240, 64, scratch, kSkinny, true}, {kQ4K, kF32, 3840, 10240, 33, scratch, kSkinny, true},
             {kQ4K, kF32, 4096, 1024, 2304, scratch, kPersist, true}, {kQ4K, kBF16, 12288, 3072, 2560, scratch, kPersist, false},
             {kQ4K, kBF16, 3072, 3072, 4608, scratch, kPersist, true}, {kQ4K, kBF16, 3072, 3072, 2048, scratch, kTiled, false},
-            {kQ8_0, kF16, 1000, 12352, 200, scratch, kSkinny, true}, {kQ8_0, kF16, 1000, 12352, 40, scratch, kSkinny, true},
+            {kQ8_0, kF16, 1000, 14400, 200, scratch, kSkinny, true}, {kQ8_0, kF16, 1000, 14400, 40, scratch, kSkinny, true},
             {kQ8_0, kBF16, 3840, 5120, 600, scratch, kCut, true},  {kQ8_0, kBF16, 3840, 5120, 513, scratch, kCut, true},
             {kQ4K, kF32, 512, 10240, 64, scratch, kSkinny, true},  {kQ4K, kF32, 4096, 4096, 4608, scratch, kTiled, false},
         };

@@ -68,7 +68,7 @@ CASES = [
     # workgroups)
     (8, 33, 516, 8256, 0, 4),        # f32 as fp16: 26 splits of 129 stages, four features past a tile
     (12, 100, 512, 8448, 0, 0),      # f32 as bf16
-    (8, 17, 640, 12352, 1, 0),       # f16, read in place
+    (8, 17, 640, 14400, 1, 0),       # f16, read in place
     (12, 200, 1540, 8192, 30, 8),    # bf16, row_offset, ragged M and N
 ]
 

@@ -55,7 +55,7 @@ CASES = [
     (12, F32, 4096, 1024, (4096, 2304), 8, (True, True), "f32 activations as bf16 + the weight image"),
     (12, BF16, 12288, 3072, (2560, 2304), 0, (True, True), "nothing: one-pass in place of a 75 MB weight image"),
     (12, BF16, 3072, 3072, (4608, 2048), 0, (True, False), "the weight image; then no partials"),
-    (8, F16, 1000, 12352, (200, 40), 4, (True, True), "split-K partials, ragged N"),
+    (8, F16, 1000, 14400, (200, 40), 4, (True, True), "split-K partials, ragged N"),
     (8, BF16, 3840, 5120, (600, 513), 0, (False, False), "partial tiles, in fewer parts"),
 ]
 
