@@ -327,7 +327,9 @@ static int release_workspace(llmr_context* ctx, size_t need) {
 static bool captures_whole(llmr_context* ctx, size_t need, size_t whole) {
     if (need == whole) return false;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(ctx->cur, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->cur, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // (the null stream beside a capture: the launch's own check is not to see it)
+    return true;
 }
 
 // Argument checks of llmr_batch_matmul and its no-allocation variant.
